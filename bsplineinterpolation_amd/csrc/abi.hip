@@ -374,8 +374,23 @@ int solve_axes(const GridData& g, bool refined, const double* values, void* x, v
     bool any_shift = false;
     for (int d = 0; d < g.dim; ++d) any_shift = any_shift || shift[d] != 0;
     const size_t elem = refined ? sizeof(float) : sizeof(double);
-    const bool fused =
-        values != nullptr && solve_tile_lines(g.setup[last].n, compute_bytes(axis_types(g, refined, last))) > 0;
+    // shape fields of axis a's line solve, and its tile
+    auto axis_params = [&](int a, SolveParams* sp) {
+        const DimSetup& s = g.setup[a];
+        const SolveTypes types = axis_types(g, refined, a);
+        sp->n = s.n;
+        sp->div_n = make_fast_div(static_cast<uint32_t>(s.n));
+        sp->inner = 1;
+        for (int d = a + 1; d < g.dim; ++d) sp->inner *= g.setup[d].n;
+        sp->nlines = g.total / s.n;
+        set_segment_params(types == SolveTypes::kF32 ? s.lu.seg32 : s.lu.seg64, sp);
+        const TilePlan plan = solve_tile_plan(*sp, s.lu.p, s.lu.cyclic, compute_bytes(types));
+        sp->lines_per_block = plan.lines;
+        sp->segs = plan.segs;
+        return plan;
+    };
+    SolveParams last_params{};
+    const bool fused = values != nullptr && axis_params(last, &last_params).lines > 0;
     if (values != nullptr && !fused) {
         if (any_shift || refined) {
             ShiftParams sh{};
@@ -399,24 +414,12 @@ int solve_axes(const GridData& g, bool refined, const double* values, void* x, v
         const bool f32 = types == SolveTypes::kF32;
         SolveParams sp{};
         sp.x = x;
-        sp.n = s.n;
-        int64_t inner = 1, outer = 1;
-        for (int d = a + 1; d < g.dim; ++d) inner *= g.setup[d].n;
-        for (int d = 0; d < a; ++d) outer *= g.setup[d].n;
-        sp.inner = inner;
-        sp.nlines = inner * outer;
+        const TilePlan plan = axis_params(a, &sp);
         sp.lower = f32 ? static_cast<const void*>(g.lower32[a]) : g.lower[a];
         sp.upper = f32 ? static_cast<const void*>(g.upper32[a]) : g.upper[a];
         sp.diag = f32 ? static_cast<const void*>(g.diag32[a]) : g.diag[a];
         sp.bottom = f32 ? static_cast<const void*>(g.bottom32[a]) : g.bottom[a];
         sp.right = f32 ? static_cast<const void*>(g.right32[a]) : g.right[a];
-        sp.lines_per_block = solve_tile_lines(s.n, compute_bytes(types));
-        // Strided axes with a wavefront or more of adjacent lines: lane l's
-        // line sits next to lane l+1's, so substituting in place reads and
-        // writes coalesced rows, and every wave of the workgroup substitutes
-        // (the LDS tile keeps one wave busy while the other three wait).
-        // The accumulating last pass keeps the tile, which adds on store.
-        if (inner >= 64 && !(a == last && fused) && !(a == 0 && accum != nullptr)) sp.lines_per_block = 0;
         if (a == last && fused) {
             sp.src = values;
             sp.outer_dims = last;
@@ -428,7 +431,7 @@ int solve_axes(const GridData& g, bool refined, const double* values, void* x, v
         }
         const bool add_after = a == 0 && accum != nullptr && sp.lines_per_block == 0;
         if (a == 0 && accum != nullptr && !add_after) sp.accum = accum;
-        hipError_t e = launch_solve(s.lu.p, s.lu.cyclic, types, sp, stream);
+        hipError_t e = launch_solve(s.lu.p, s.lu.cyclic, types, sp, plan.threads, stream);
         if (e == hipErrorNotSupported) return fail(INTP_E_UNSUPPORTED, "band width without a compiled solver");
         HIP_TRY(e, "solve launch");
         if (add_after) {

@@ -44,6 +44,11 @@ namespace {
 // Rows per substitution batch in the merged kernels (bounds registers:
 // two workgroups per CU).
 constexpr int kMergedRows = 4;
+// the segmented tile kernel holds a batch's factors next to its loop state
+template <int BW, bool CYC, int NT>
+constexpr int merged_rows() {
+    return NT == 256 && BW * (CYC ? 2 : 1) >= 4 ? 2 : kMergedRows;
+}
 // Small tiles (at most kSmallTileBytes of LDS) are solved by one-wave
 // workgroups, so that every resident wave substitutes a tile of its own
 // (a 256-thread workgroup has one substituting wave and three waiting at
@@ -73,6 +78,7 @@ __device__ __forceinline__ void batch_solve_item(const BatchSpline* specs, const
         SolveParams sp{};
         sp.x = ctrl + b.offset;
         sp.n = b.ep.dim[a].n;
+        sp.div_n = make_fast_div(static_cast<uint32_t>(sp.n));
         int64_t inner = 1;
         for (int d = a + 1; d < b.dim; ++d) inner *= b.ep.dim[d].n;
         sp.inner = inner;
@@ -83,6 +89,10 @@ __device__ __forceinline__ void batch_solve_item(const BatchSpline* specs, const
         sp.bottom = b.bottom[a];
         sp.right = b.right[a];
         sp.lines_per_block = b.lines_per_block[a];
+        if constexpr (NT == kTileThreads) {
+            sp.segs = b.segs[a];
+            set_segment_params(b.seg[a], &sp);
+        }
         if (first_pass) {
             sp.src = values + b.offset;
             sp.outer_dims = a;
@@ -94,7 +104,8 @@ __device__ __forceinline__ void batch_solve_item(const BatchSpline* specs, const
             }
             sp.shift_last = b.shift[a];
         }
-        solve_tile<BW, CYC, double, double, kMergedRows, NT>(sp, w.first_line, tile_bytes, dst_base, src_base);
+        solve_tile<BW, CYC, double, double, merged_rows<BW, CYC, NT>(), NT == kTileThreads, false>(sp, w.first_line, tile_bytes, dst_base, src_base,
+                                                       static_cast<int>(threadIdx.x), NT);
         return;
     }
     // kSolveLanes: one line per lane, in place
@@ -116,24 +127,34 @@ __device__ __forceinline__ void batch_solve_item(const BatchSpline* specs, const
 }
 
 // One-dimensional splines: one spline per 64-thread workgroup, longest
-// first (list1d).  The wave copies the values into the control-point array
-// with the periodic shift (coalesced), then its first lane substitutes the
-// line in place.  Runs on its own stream beside the passes of the
-// multi-dimensional splines: a 1D line is one long sequential chain, and
-// needs a wave, not a workgroup's LDS.
+// first (list1d), the line in LDS and cut into up to 64 segments
+// (solve_segments); lines too long for LDS are substituted in HBM by the
+// first lane.  Runs on its own stream beside the passes of the
+// multi-dimensional splines.
 template <int BW, bool CYC>
-__device__ __forceinline__ void batch_line(const BatchSpline& b, const double* values, double* ctrl) {
+__device__ __forceinline__ void batch_line(const BatchSpline& b, const double* values, double* ctrl,
+                                           unsigned char* tile_bytes, int64_t* dst_base, int64_t* src_base) {
     const int64_t n = b.ep.dim[0].n, shift = b.shift[0];
     double* x = ctrl + b.offset;
     const double* f = values + b.offset;
-    if constexpr (BW == 0) {
-        // a diagonal system: each row is one division, every lane takes rows
-        const double* __restrict__ diag = b.diag[0];
-        for (int64_t j = threadIdx.x; j < n; j += kLineThreads) {
-            int64_t js = j - shift;
-            if (js < 0) js += n;
-            x[j] = f[js] / diag[j];
-        }
+    SolveParams sp{};
+    sp.lower = b.lower[0];
+    sp.upper = b.upper[0];
+    sp.diag = b.diag[0];
+    sp.bottom = b.bottom[0];
+    sp.right = b.right[0];
+    if (b.lines_per_block[0] > 0) {
+        sp.x = x;
+        sp.src = f;
+        sp.n = n;
+        sp.inner = sp.nlines = 1;
+        sp.div_n = make_fast_div(static_cast<uint32_t>(n));
+        sp.shift_last = shift;
+        sp.lines_per_block = 1;
+        sp.segs = b.segs[0];
+        set_segment_params(b.seg[0], &sp);
+        solve_tile<BW, CYC, double, double, kMergedRows, true, false>(sp, 0, tile_bytes, dst_base, src_base,
+                                                         static_cast<int>(threadIdx.x), kLineThreads);
         return;
     }
     for (int64_t j = threadIdx.x; j < n; j += kLineThreads) {
@@ -143,12 +164,6 @@ __device__ __forceinline__ void batch_line(const BatchSpline& b, const double* v
     }
     __syncthreads();
     if (threadIdx.x != 0) return;
-    SolveParams sp{};
-    sp.lower = b.lower[0];
-    sp.upper = b.upper[0];
-    sp.diag = b.diag[0];
-    sp.bottom = b.bottom[0];
-    sp.right = b.right[0];
     substitute<BW, CYC, double, double, kMergedRows>(x, 1, n, sp);
 }
 
@@ -333,15 +348,18 @@ __device__ __forceinline__ void batch_line_split(const BatchSpline& b, const dou
 
 // skip_split: the lines with segment responses are solved by
 // batch_line_split_kernel instead.
-__global__ __launch_bounds__(kLineThreads, 4) void batch_line_kernel(const BatchSpline* specs, const int32_t* list1d,
+__global__ __launch_bounds__(kLineThreads, 2) void batch_line_kernel(const BatchSpline* specs, const int32_t* list1d,
                                                                   const double* values, double* ctrl,
                                                                   int32_t skip_split) {
+    extern __shared__ __align__(16) unsigned char tile_bytes[];
+    __shared__ int64_t dst_base[kMaxTileLines];
+    __shared__ int64_t src_base[kMaxTileLines];
     const BatchSpline& b = specs[list1d[blockIdx.x]];
     if (skip_split && b.nseg > 0) return;
     const int kind = 2 * b.band[0] + (b.ep.dim[0].periodic ? 1 : 0);
 #define INTP_LINE_CASE(BW, CYC) \
     case 2 * BW + CYC:          \
-        batch_line<BW, CYC>(b, values, ctrl); \
+        batch_line<BW, CYC>(b, values, ctrl, tile_bytes, dst_base, src_base); \
         break;
     switch (kind) {
         INTP_LINE_CASE(0, false)
@@ -390,7 +408,7 @@ __global__ __launch_bounds__(kLineThreads) void batch_line_split_kernel(const Ba
 // items are ordered longest line first, so the long sequential lines
 // start at once and the short tiles fill in around them).
 template <int NT>
-__global__ __launch_bounds__(NT, NT == kTileThreads ? 1 : 2) void batch_solve_kernel(const BatchSpline* specs,
+__global__ __launch_bounds__(NT, 2) void batch_solve_kernel(const BatchSpline* specs,
                                                                    const BatchSolveItem* items, int32_t nitems,
                                                                    const double* values, double* ctrl,
                                                                    int32_t first_pass) {
@@ -426,13 +444,22 @@ __global__ __launch_bounds__(NT, NT == kTileThreads ? 1 : 2) void batch_solve_ke
 constexpr int kEvalStreams = 4;
 
 // LDS budget of one solve workgroup (two per CU).
-constexpr int64_t kBatchTileBudget = 80 * 1024 - 2 * kMaxTileLines * 8;
+constexpr int64_t kBatchTileBudget = 80 * 1024 - 2 * kMaxTileLines * 8 - kEdgeMax * 8;
 
-int64_t tile_fit(int64_t n, int cap) {
-    const int64_t row = (n | 1) * 8;
+int64_t tile_fit(int64_t n, int64_t inner, int cap) {
     int lpb = kMaxTileLines;
-    while (lpb > 0 && (lpb > cap || lpb * row > kBatchTileBudget)) lpb /= 2;
+    while (lpb > 0 && (lpb > cap || tile_elements(n, lpb, inner) * 8 > kBatchTileBudget)) lpb /= 2;
+    // one line may take most of a CU's LDS
+    if (lpb == 0 && tile_elements(n, 1, inner) * 8 <= kBatchTileBudget + 80 * 1024) lpb = 1;
     return lpb;
+}
+
+// Elements of the staged edge factors of an axis (after the tile in LDS).
+int64_t edge_rows(const DimSetup& ds, int segs) {
+    SolveParams sp{};
+    set_segment_params(ds.lu.seg64, &sp);
+    sp.segs = segs;
+    return edge_elements(ds.n, ds.lu.p, sp);
 }
 
 struct SolveGroup {
@@ -449,7 +476,7 @@ struct EvalGroup {
 
 // Tunables (picked by the autotuner).
 struct Tuning {
-    int tile_cap = 64;           // lines per solve tile, at most
+    int tile_cap = kTileLines;   // lines per solve tile, at most
     int solve_blocks_per_cu = 4;  // persistent 256-thread solve workgroups per CU
     int eval_threads = 256;       // points per eval item (= workgroup size)
     int eval_blocks_per_cu = 8;   // persistent eval workgroups per CU
@@ -479,6 +506,7 @@ struct intp_batch_s {
     int64_t solve_cap = 0;
     std::vector<int32_t> list1d_host;  // the 1D splines, longest first
     int32_t* list1d = nullptr;
+    size_t line_lds = 0;               // LDS of batch_line_kernel
     double* split_tables = nullptr;    // segment responses of the split 1D lines
     std::vector<int32_t> split_host;   // the split lines, longest first
     int32_t* split_list = nullptr;
@@ -568,9 +596,23 @@ int make_solve_work(intp_batch b, hipStream_t stream) {
         BatchSpline& bs = b->host_specs[static_cast<size_t>(s)];
         const int D = b->dims[static_cast<size_t>(s)];
         for (int d = 0; d < D; ++d) {
-            const int64_t lpb = tile_fit(b->setups[static_cast<size_t>(s) * kBatchDim + d].n, b->tune.tile_cap);
             int64_t inner = 1;
             for (int e = d + 1; e < D; ++e) inner *= b->setups[static_cast<size_t>(s) * kBatchDim + e].n;
+            const DimSetup& ds = b->setups[static_cast<size_t>(s) * kBatchDim + d];
+            // a 1D spline is a tile of its own; an axis with 64 or more
+            // adjacent lines and no room for four of them is solved in HBM
+            int64_t lpb = tile_fit(ds.n, inner, D == 1 ? 1 : b->tune.tile_cap);
+            if (D > 1 && inner >= 64 && lpb < 4) lpb = 0;
+            // segments where they pay: one lane of the 256-thread tile
+            // workgroup (of the 64-thread line workgroup) per segment and line
+            bs.segs[d] = 0;
+            if (lpb > 0 && ds.n >= kMinSegmentRows && (ds.lu.seg64.warm > 0 || ds.lu.p == 0) &&
+                (!ds.lu.cyclic || ds.n >= 2 * ds.lu.seg64.warm)) {
+                int64_t segs = D == 1 ? kLineThreads : kTileThreads / lpb;
+                while (segs > 1 && segs * 8 > ds.n) segs /= 2;
+                if (segs < ds.lu.p || 4 * (ds.lu.seg64.warm + ds.n / segs) > 3 * ds.n) segs = D == 1 ? 1 : 0;
+                bs.segs[d] = static_cast<int32_t>(segs);
+            }
             if (lpb == 0 && inner < 64 && D > 1)
                 return fail(INTP_E_UNSUPPORTED, "spline " + std::to_string(s) + ": line too long for a batch");
             bs.lines_per_block[d] = static_cast<int32_t>(lpb);
@@ -607,15 +649,21 @@ int make_solve_work(intp_batch b, hipStream_t stream) {
             for (int d = a + 1; d < D; ++d) inner *= b->setups[static_cast<size_t>(s) * kBatchDim + d].n;
             const int64_t cost = ds.n * row_cost(ds);
             if (D == 1) {
-                continue;  // batch_line_kernel, beside the passes
-            } else if (inner >= 64) {
+                // batch_line_kernel, beside the passes
+                if (bs.lines_per_block[0] > 0)
+                    b->line_lds = std::max(b->line_lds, static_cast<size_t>((tile_elements(ds.n, 1, 1) +
+                                                                             edge_rows(ds, bs.segs[0])) * 8));
+                continue;
+            } else if (bs.lines_per_block[a] == 0) {
                 for (int64_t first = 0; first < nlines; first += kTileThreads)
                     large_items.push_back(
                         {cost, BatchSolveItem{s, static_cast<int16_t>(a), kind_of(ds, kSolveLanes), first}});
             } else {
                 const int64_t lpb = bs.lines_per_block[a];
-                const int64_t bytes = lpb * (ds.n | 1) * 8;
-                const bool small = bytes <= kSmallTileBytes, medium = !small && bytes <= kMediumTileBytes;
+                const int64_t bytes = (tile_elements(ds.n, lpb, inner) + edge_rows(ds, bs.segs[a])) * 8;
+                // lines cut into segments keep every wave busy; the others one
+                const bool small = bytes <= kSmallTileBytes && bs.segs[a] == 0;
+                const bool medium = !small && bytes <= kMediumTileBytes && bs.segs[a] == 0;
                 auto& to_items = small ? small_items : medium ? medium_items : large_items;
                 for (int64_t first = 0; first < nlines; first += lpb)
                     to_items.push_back({cost, BatchSolveItem{s, static_cast<int16_t>(a), kind_of(ds, kSolveTile), first}});
@@ -785,7 +833,7 @@ int launch_build(intp_batch b, const double* values, hipStream_t stream, bool sp
             HIP_TRY(hipEventRecord(b->join2, b->side2), "hipEventRecord");
         }
         hipLaunchKernelGGL(batch_line_kernel, dim3(static_cast<unsigned>(b->list1d_host.size())), dim3(kLineThreads),
-                           0, b->side, b->specs, b->list1d, values, b->ctrl, seg ? 1 : 0);
+                           b->line_lds, b->side, b->specs, b->list1d, values, b->ctrl, seg ? 1 : 0);
         HIP_TRY(hipGetLastError(), "batch line launch");
         HIP_TRY(hipEventRecord(b->join, b->side), "hipEventRecord");
     }
@@ -938,7 +986,7 @@ int autotune(intp_batch b, const double* values, const double* coords, const int
     // the solve knobs dominate and interact: they are visited twice
     int rc;
     for (int round = 0; round < 2; ++round) {
-        if ((rc = try_values("tile_cap", &Tuning::tile_cap, {8, 16, 32, 64})) != INTP_OK) return rc;
+        if ((rc = try_values("tile_cap", &Tuning::tile_cap, {8, 16, 32})) != INTP_OK) return rc;
         if ((rc = try_values("solve_blocks_per_cu", &Tuning::solve_blocks_per_cu, {1, 2, 4, 8})) != INTP_OK) return rc;
         if (round == 0) {
             if ((rc = try_values("eval_threads", &Tuning::eval_threads, {64, 128, 256})) != INTP_OK) return rc;
@@ -1088,6 +1136,7 @@ int intp_batch_create(intp_ctx ctx_, int32_t count, const intp_grid_desc* descs,
             bs.right[d] = dptr(w.right, ds.lu.right.size());
             bs.shift[d] = ds.periodic ? (K / 2) % ds.n : 0;
             bs.band[d] = ds.lu.p;
+            bs.seg[d] = ds.lu.seg64;
         }
         ep.ctrl = b->ctrl + bs.offset;
         ep.cs_dim = 1;

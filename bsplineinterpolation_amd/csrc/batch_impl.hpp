@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include "kernels.hpp"
+#include "setup.hpp"
 
 namespace intp_amd {
 
@@ -27,6 +28,8 @@ struct BatchSpline {
     int32_t dim, order;
     int32_t lines_per_block[kBatchDim];  // LDS tile of the solve along each axis
     int32_t band[kBatchDim];             // band width of each axis's LU
+    int32_t segs[kBatchDim];             // segments per line of the tile (0: plain substitution)
+    SegmentPlan seg[kBatchDim];
     // Split solve of a long 1D line (INTP_BATCH_SPLIT_LINES): nseg segments
     // of the first n - 2*band - 8 rows, and the responses of each segment's
     // rows to the band values entering it, forward (gf) and backward (gb),
@@ -39,10 +42,10 @@ struct BatchSpline {
 // Work of one solve workgroup.  kind & 15 = 2 * band width + cyclic
 // selects the substitution; kind >> 4 the mode:
 //   kSolveTile: lines first_line .. of `spline` along `axis`, staged
-//     through LDS (contiguous axes, and axes with fewer than 64 adjacent
-//     lines);
+//     through LDS;
 //   kSolveLanes: 256 adjacent lines first_line .. of `spline` along a
-//     strided `axis`, one per lane, substituted in place.
+//     strided `axis` too long for a tile, one per lane, substituted in
+//     place.
 enum : int16_t { kSolveTile = 0, kSolveLanes = 1 };
 
 struct BatchSolveItem {

@@ -36,4 +36,24 @@ inline DimParams make_dim_params(const DimSetup& s, int order, int64_t stride, c
     return p;
 }
 
+// The segment fields of a line solve.
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+inline void set_segment_params(const SegmentPlan& seg, SolveParams* sp) {
+    sp->warm = seg.warm;
+    sp->flo = seg.flo;
+    sp->fhi = seg.fhi;
+    sp->blo = seg.blo;
+    sp->bhi = seg.bhi;
+    sp->fast_divide = seg.fast_divide ? 1 : 0;
+    sp->zh = seg.zh;
+    sp->zl = seg.zl;
+    sp->strip_rest = seg.strip_rest;
+    for (int m = 0; m < kMaxOrder; ++m) {
+        sp->eq_lower[m] = seg.eq_lower[m];
+        sp->eq_upper[m] = seg.eq_upper[m];
+    }
+}
+
 }  // namespace intp_amd

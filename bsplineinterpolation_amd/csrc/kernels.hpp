@@ -149,6 +149,34 @@ hipError_t launch_first_outside(const BoundsParams& p, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t value, int64_t n, hipStream_t s);
 hipError_t launch_proxy_apply(int dim, int order, bool uniform, bool f32, const ProxyParams& p, hipStream_t s);
 
+// Division of 32-bit unsigned integers by an invariant d >= 1 with a
+// multiply-high (Granlund & Montgomery, "Division by invariant integers
+// using multiplication", PLDI 1994, Fig. 4.1): for s = ceil(log2 d) and
+// m = floor(2^32 (2^s - d) / d) + 1, q = (t + ((x - t) >> 1)) >> (s - 1)
+// with t = mulhi(x, m); d == 1 passes x through.
+struct FastDiv {
+    uint32_t d = 1, m = 0, s = 0;
+};
+
+__host__ __device__ inline FastDiv make_fast_div(uint32_t d) {
+    FastDiv f;
+    f.d = d;
+    if (d <= 1) return f;
+    uint32_t s = 0;
+    while ((uint64_t{1} << s) < d) ++s;
+    f.s = s;
+    f.m = static_cast<uint32_t>(((uint64_t{1} << 32) * ((uint64_t{1} << s) - d)) / d + 1);
+    return f;
+}
+
+#ifdef __HIPCC__
+__device__ __forceinline__ uint32_t fast_div(uint32_t x, const FastDiv& f) {
+    if (f.d == 1) return x;
+    const uint32_t t = __umulhi(x, f.m);
+    return (t + ((x - t) >> 1)) >> (f.s - 1);
+}
+#endif
+
 // Line solves along one axis of a C-order table viewed as
 // (outer, n, inner): line (o, i) holds elements o*n*inner + j*inner + i.
 // Element types of a line solve: storage (the table) and compute (the
@@ -166,6 +194,7 @@ struct SolveParams {
     // accum (storage type) instead of being stored to x.
     void* accum;
     int64_t n, inner, nlines;
+    FastDiv div_n;  // division by n
     // factors in the compute type
     const void* lower;   // n * bw
     const void* upper;   // n * bw
@@ -177,6 +206,23 @@ struct SolveParams {
     int64_t outer_shift[kMaxDim];  // their shifts
     int64_t shift_last;            // shift along the solved axis
     int32_t lines_per_block;       // LDS-tiled kernel: lines per workgroup (0: one lane per line from HBM)
+    int32_t segs;                  // LDS-tiled kernel: segments per line (0: plain substitution)
+    int32_t warm;                  // rows a segment starts early (SegmentPlan)
+    int32_t flo, fhi, blo, bhi;    // rows of equal factors, forward and backward (SegmentPlan)
+    int32_t fast_divide;           // zh, zl divide by the pivot of rows [blo, bhi) (SegmentPlan)
+    double zh, zl;
+    double strip_rest;             // the largest bottom strip entry from row `warm` on (cyclic)
+    double eq_lower[kMaxOrder], eq_upper[kMaxOrder];  // the factors of those rows
+};
+
+// Lines shorter than this are not cut into segments.
+constexpr int64_t kMinSegmentRows = 128;
+
+// Shape of the LDS-tiled kernel for one axis: lines per workgroup (0: the
+// tile does not fit, solve in HBM), segments per line (0: plain
+// substitution), threads.
+struct TilePlan {
+    int lines = 0, segs = 0, threads = 256;
 };
 
 struct ShiftParams {
@@ -222,11 +268,10 @@ hipError_t eval_dispatch_f64_d6(int order, bool grad, bool uniform, const EvalPa
 hipError_t eval_dispatch_f32_d4(int order, bool grad, bool uniform, const EvalParams& p, hipStream_t s);
 hipError_t eval_dispatch_f32_d5(int order, bool grad, bool uniform, const EvalParams& p, hipStream_t s);
 hipError_t eval_dispatch_f32_d6(int order, bool grad, bool uniform, const EvalParams& p, hipStream_t s);
-hipError_t launch_solve(int bw, bool cyclic, SolveTypes types, const SolveParams& p, hipStream_t s);
-// Lines of length n that one LDS-tiled solve workgroup holds on the
-// current device (a power of two up to 64) for compute elements of
-// `compute_bytes`, 0 if a line does not fit.
-int solve_tile_lines(int64_t n, int compute_bytes);
+hipError_t launch_solve(int bw, bool cyclic, SolveTypes types, const SolveParams& p, int threads, hipStream_t s);
+// The tile for the lines of p (n, nlines, inner and the segment fields set)
+// on the current device, for compute elements of `compute_bytes`.
+TilePlan solve_tile_plan(const SolveParams& p, int bw, bool cyclic, int compute_bytes);
 
 // One-pass grouping (group.hip): per-block LDS histograms of the brick
 // keys over fixed ranges of points, one exclusive scan of the bin-major
@@ -276,34 +321,6 @@ hipError_t launch_shift_copy(const ShiftParams& p, bool dst_f32, hipStream_t s);
 // y = M x along one axis of a table viewed as (outer, n, inner), M the
 // axis' collocation matrix as rows colloc[j*(2w+1) + (m+w)] = M(j, j+m)
 // (columns mod n if periodic); with src set, y = (shifted src) - M x.
-// Division of 32-bit unsigned integers by an invariant d >= 1 with a
-// multiply-high (Granlund & Montgomery, "Division by invariant integers
-// using multiplication", PLDI 1994, Fig. 4.1): for s = ceil(log2 d) and
-// m = floor(2^32 (2^s - d) / d) + 1, q = (t + ((x - t) >> 1)) >> (s - 1)
-// with t = mulhi(x, m); d == 1 passes x through.
-struct FastDiv {
-    uint32_t d = 1, m = 0, s = 0;
-};
-
-inline FastDiv make_fast_div(uint32_t d) {
-    FastDiv f;
-    f.d = d;
-    if (d <= 1) return f;
-    uint32_t s = 0;
-    while ((uint64_t{1} << s) < d) ++s;
-    f.s = s;
-    f.m = static_cast<uint32_t>(((uint64_t{1} << 32) * ((uint64_t{1} << s) - d)) / d + 1);
-    return f;
-}
-
-#ifdef __HIPCC__
-__device__ __forceinline__ uint32_t fast_div(uint32_t x, const FastDiv& f) {
-    if (f.d == 1) return x;
-    const uint32_t t = __umulhi(x, f.m);
-    return (t + ((x - t) >> 1)) >> (f.s - 1);
-}
-#endif
-
 struct MatvecParams {
     const void* x;  // float or double
     void* y;        // float or double

@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 
 namespace intp_amd {
 
@@ -94,6 +95,141 @@ class PatternMatrix {
     bool cyclic_;
     std::vector<double> band_, right_, bottom_;
 };
+
+// Rows until the recurrence of either sweep, started from a unit state with
+// zero right-hand sides, falls below 2^-24 and below 2^-53 (the largest over
+// the unit states and a few starting rows: the middle row on a uniform grid,
+// whose interior rows are alike, eight rows otherwise); kMaxForget if it
+// does not.
+constexpr int kMaxForget = 128;
+
+void forget_rows(const LineFactors& f, bool uniform, int* rows24, int* rows53) {
+    const int bw = f.p;
+    const int64_t starts = uniform ? 1 : std::min<int64_t>(8, f.n);
+    *rows24 = *rows53 = 0;
+    for (int64_t s = 0; s < 2 * starts; ++s)
+        for (int unit = 0; unit < bw; ++unit) {
+            const bool forward = s < starts;
+            double h[16] = {};
+            h[unit] = 1.0;
+            const int64_t j0 = uniform ? f.n / 2 : (s % starts) * f.n / starts;
+            int rows = 0, r24 = kMaxForget, r53 = kMaxForget;
+            for (int64_t j = forward ? j0 : f.n - 1 - j0; j >= 0 && j < f.n; j += forward ? 1 : -1) {
+                double v = 0.0, big = 0.0;
+                const double* c = forward ? &f.lower[static_cast<size_t>(j * bw)] : &f.upper[static_cast<size_t>(j * bw)];
+                for (int m = 0; m < bw; ++m) v -= c[m] * h[m];
+                if (!forward) v /= f.diag[static_cast<size_t>(j)];
+                for (int m = bw - 1; m > 0; --m) h[m] = h[m - 1];
+                h[0] = v;
+                for (int m = 0; m < bw; ++m) big = std::max(big, std::fabs(h[m]));
+                ++rows;
+                if (big <= 0x1p-24) r24 = std::min(r24, rows);
+                if (big <= 0x1p-53) r53 = rows;
+                if (r53 < kMaxForget || rows >= kMaxForget) break;
+            }
+            // a start that runs out of rows says nothing
+            if (r53 == kMaxForget && rows < kMaxForget) continue;
+            *rows24 = std::max(*rows24, r24);
+            *rows53 = std::max(*rows53, r53);
+        }
+    if (*rows53 == 0) *rows24 = *rows53 = kMaxForget;  // short lines: no start had the rows
+}
+
+// Division by a divisor known in advance: with zh = 1/d rounded down and zl
+// = 1/d - zh rounded, RN(x zh + RN(x zl)) differs from x/d before the last
+// rounding by less than 2^(2-2p) of it (p mantissa bits: 2^-2p from the
+// rounding of zl, twice that from x zl).  It is the correctly rounded
+// quotient unless x/d lies that close to the middle M of two neighbouring
+// numbers.  With X and Y the p-bit integer mantissas of x and d, M = N /
+// 2^K (N odd, p+1 bits; K = p for X >= Y, else p + 1) and R = 2^K X - N Y
+// such an x has |R| < 16, so N = -R / Y modulo 2^K: every candidate is
+// listed and tried.  (Brisebarre, Muller and Raina, IEEE Transactions on
+// Computers 53(8), 2004.)
+template <typename C>
+bool known_divisor_impl(C d, int p, C* zh, C* zl) {
+    if (!(d > static_cast<C>(0x1p-40) && d < static_cast<C>(0x1p40))) return false;
+    C h = static_cast<C>(1) / d;
+    C e = std::fma(-d, h, static_cast<C>(1));
+    if (e < 0) {
+        h = std::nextafter(h, static_cast<C>(0));
+        e = std::fma(-d, h, static_cast<C>(1));
+    }
+    *zh = h;
+    *zl = e / d;
+    int exponent = 0;
+    const uint64_t Y = static_cast<uint64_t>(std::ldexp(std::frexp(d, &exponent), p));
+    int s = 0;
+    while (((Y >> s) & 1) == 0) ++s;
+    const uint64_t odd = Y >> s;
+    uint64_t inv = odd;  // inverse modulo 2^64 by Newton's iteration
+    for (int i = 0; i < 6; ++i) inv *= 2 - odd * inv;
+    for (int K = p; K <= p + 1; ++K)
+        for (int64_t R = -16; R <= 16; ++R) {
+            if (R == 0 || (R & ((int64_t{1} << std::min(s, 40)) - 1)) != 0) continue;
+            const uint64_t mod = uint64_t{1} << (K - s);
+            const uint64_t first = (static_cast<uint64_t>(-(R >> s)) * inv) & (mod - 1);
+            for (uint64_t N = first; N < (uint64_t{1} << (p + 1)); N += mod) {
+                if (N < (uint64_t{1} << p) || (N & 1) == 0) continue;
+                const __int128 num = static_cast<__int128>(N) * Y + R;
+                const uint64_t X = static_cast<uint64_t>(num >> K);
+                if (X < (uint64_t{1} << (p - 1)) || X >= (uint64_t{1} << p)) continue;
+                const C x = static_cast<C>(X);
+                const C low = x * *zl;
+                if (std::fma(x, *zh, low) != x / d) return false;
+            }
+        }
+    return true;
+}
+
+// Segment plan of one compute type from its factors.  The warm-up covers
+// the decay of the starting state to a rounding (`base` rows) and
+// then the rows two almost equal states take to round to the same bits,
+// 4 decades of probability in about 10 r^2 + 2 rows, r = rows per factor e
+// of decay (fitted to measured merges, orders 2 to 7); 2.2 times that
+// leaves about one failed comparison in 10^10.
+template <typename C>
+SegmentPlan segment_plan(const LineFactors& f, const std::vector<C>& lower, const std::vector<C>& upper,
+                         const std::vector<C>& diag, int base, int rows53) {
+    SegmentPlan s;
+    const int bw = f.p;
+    const int64_t n = f.n;
+    if (n >= (int64_t{1} << 30)) return s;
+    auto same = [&](const std::vector<C>& v, int w, int64_t a, int64_t b) {
+        return w == 0 || std::memcmp(&v[static_cast<size_t>(a * w)], &v[static_cast<size_t>(b * w)],
+                                     static_cast<size_t>(w) * sizeof(C)) == 0;
+    };
+    const int64_t mid = n / 2;
+    int64_t a = mid, e = mid + 1;
+    while (a > 0 && same(lower, bw, a - 1, mid)) --a;
+    while (e < n && same(lower, bw, e, mid)) ++e;
+    s.flo = static_cast<int>(a);
+    s.fhi = static_cast<int>(e);
+    a = mid;
+    e = mid + 1;
+    while (a > 0 && same(upper, bw, a - 1, mid) && same(diag, 1, a - 1, mid)) --a;
+    while (e < n && same(upper, bw, e, mid) && same(diag, 1, e, mid)) ++e;
+    s.blo = static_cast<int>(a);
+    s.bhi = static_cast<int>(e);
+    for (int m = 0; m < bw; ++m) {
+        s.eq_lower[m] = static_cast<double>(lower[static_cast<size_t>(s.flo * bw + m)]);
+        s.eq_upper[m] = static_cast<double>(upper[static_cast<size_t>(s.blo * bw + m)]);
+    }
+    if (bw > 0) {
+        if (base >= kMaxForget) return s;
+        const double r = rows53 / 36.74;
+        s.warm = (static_cast<int>(base + 2.2 * (10.0 * r * r + 2.0)) + 7) / 8 * 8;
+        C zh = 0, zl = 0;
+        s.fast_divide = known_divisor(diag[static_cast<size_t>(s.blo)], &zh, &zl);
+        s.zh = static_cast<double>(zh);
+        s.zl = static_cast<double>(zl);
+        for (int q = 0; f.cyclic && q < bw; ++q)
+            for (int64_t j = s.warm; j < n; ++j)
+                s.strip_rest = std::max(s.strip_rest, std::fabs(f.bottom[static_cast<size_t>(q * n + j)]));
+        // as a C, not below any rounded strip entry
+        s.strip_rest = static_cast<double>(std::nextafter(static_cast<C>(s.strip_rest), static_cast<C>(1)));
+    }
+    return s;
+}
 
 // Span containing x among t[order .. last]: the unique mu with
 // t[mu] <= x < t[mu+1], clamped to [order, last] (BSpline.hpp:146-156).
@@ -194,6 +330,9 @@ void set_range(int order, DimSetup& s) {
 }
 
 }  // namespace
+
+bool known_divisor(double d, double* zh, double* zl) { return known_divisor_impl(d, 53, zh, zl); }
+bool known_divisor(float d, float* zh, float* zl) { return known_divisor_impl(d, 24, zh, zl); }
 
 int64_t knot_count(int order, bool periodic, int64_t n) {
     const int64_t np = n + (periodic ? 1 : 0);
@@ -333,6 +472,10 @@ std::string setup_dimension(int order, bool periodic, int64_t n, double xmin, do
     for (int64_t i = 0; i < n; ++i)
         if (!(std::fabs(s.lu.diag[static_cast<size_t>(i)]) > 0.0) || !std::isfinite(s.lu.diag[static_cast<size_t>(i)]))
             return "singular collocation matrix";
+    int rows24 = 0, rows53 = 0;
+    if (s.lu.p > 0) forget_rows(s.lu, s.uniform, &rows24, &rows53);
+    s.lu.seg64 = segment_plan(s.lu, s.lu.lower, s.lu.upper, s.lu.diag, rows53, rows53);
+    s.lu.seg32 = segment_plan(s.lu, s.lower32, s.upper32, s.diag32, rows24, rows53);
     fill_recip(k, s);
     return "";
 }

@@ -18,11 +18,28 @@ namespace intp_amd {
 //   diag[i]          = U(i, i)
 //   bottom[r*n + j]  = L(n-q+r, j), j < n-q+r-p   (periodic only)
 //   right[c*n + i]   = U(i, n-p+c), i < n-p+c-q   (periodic only)
+// Segmented substitution of a line (solve_impl.hpp), per compute type:
+// rows a segment starts early (0: lines are not cut; a multiple of 8), and
+// the rows whose factors equal those of row flo (lower) or blo (upper and
+// diagonal) bit for bit: [flo, fhi) and [blo, bhi).  fast_divide: v zh +
+// (v zl), the product in brackets and the sum rounded once each, is the
+// correctly rounded v / diag[blo] for every v whose v zl does not
+// underflow.  strip_rest: the largest |bottom[q][j]| with j >= warm.
+struct SegmentPlan {
+    int warm = 0;
+    int flo = 0, fhi = 0, blo = 0, bhi = 0;
+    bool fast_divide = false;
+    double zh = 0, zl = 0;
+    double strip_rest = 0;
+    double eq_lower[7] = {}, eq_upper[7] = {};  // the factors of rows flo and blo
+};
+
 struct LineFactors {
     int64_t n = 0;
     int p = 0, q = 0;
     bool cyclic = false;
     std::vector<double> lower, upper, diag, bottom, right;
+    SegmentPlan seg64, seg32;  // for the FP64 factors and for their FP32 rounding
 };
 
 struct DimSetup {
@@ -63,6 +80,10 @@ struct DimSetup {
 // Returns an empty string on success, else the reason.
 std::string setup_dimension(int order, bool periodic, int64_t n, double xmin, double xmax,
                             const double* nodes, DimSetup& out);
+// Whether the two-operation division above is exact for divisor d, and its
+// zh and zl (also for tests).
+bool known_divisor(double d, double* zh, double* zl);
+bool known_divisor(float d, float* zh, float* zl);
 // For explicit knot vectors (no collocation matrix).
 std::string setup_from_knots(int order, bool periodic, int64_t n, const double* knots,
                              int64_t nknots, DimSetup& out);

@@ -1,24 +1,32 @@
 // solve_impl.hpp -- control-point solve on gfx950 (device code shared by
 // solve.hip and the batched kernels of batch.hip): every grid line of one axis
 // is an independent band (or cyclic band) system sharing one LU
-// factorization (InterpolationTemplate.hpp:448-580).  One lane solves one
-// line.
+// factorization (InterpolationTemplate.hpp:448-580).
 //
-// Contiguous axis (solve_tile_kernel): a workgroup copies the lines of up
-// to 64 neighbouring lanes into LDS with coalesced bulk loads (runs of one
-// line), each lane substitutes its line in LDS, and the workgroup writes
-// the tile back the same way.  The first pass reads the caller's values
-// with the periodic index shift applied (InterpolationTemplate.hpp:452-462),
-// so no separate copy precedes it.  Strided axes with 64 or more adjacent
-// lines, and lines too long for LDS, use solve_kernel, which substitutes
-// in place in HBM (coalesced across lanes on a strided axis).
+// solve_tile: a workgroup copies up to 32 lines into LDS with coalesced
+// loads, substitutes them there, each line cut into segments of one lane
+// each (solve_segments), and writes the tile back.  The first pass reads
+// the caller's values with the periodic index shift applied
+// (InterpolationTemplate.hpp:452-462), so no separate copy precedes it.
+// Lines too long for LDS use solve_kernel (one lane per line, in HBM).
+//
+// What bounds it.  Substituting a line is a chain of dependent rows: 16
+// cycles forward (order 3), and backward 16 and an IEEE division of 70.
+// With one lane per line a CU held at most 64 chains (its LDS full of
+// lines), and one 1D line kept one lane of the chip busy.  Segments put 8
+// lanes or more on a line; the division by a pivot that repeats takes two
+// operations (KnownDivisor); rows whose factors repeat take them from
+// scalar registers.  Whole solves, before -> after:
+//   1D 8192 cubic 643 -> 49 us (clamped), order 6 periodic FP32 storage,
+//   two solves, 3314 -> 199 us; 2D 1021 x 769 order 5 364 -> 74 us, 2000^2
+//   cubic 655 -> 80 us; 3D 128^3 cubic 100 -> 70 us, 256^3 cubic 300 -> 273
+//   us (one axis 76 to 100 us, of which copying the tile in and out is 44,
+//   6.1 TB/s).
 //
 // The substitution is the reference's (BandLU.hpp:121-143, 216-259)
 // reordered by rows: each entry receives the same updates in the same
-// order, the last `bw` values ride in registers, and the cyclic strips are
-// register accumulators (forward) and register-held corner values
-// (backward).  Built without FMA contraction and with a true division by
-// the pivot, the result is bit-identical to the reference's.
+// order.  Built without FMA contraction and with correctly rounded
+// divisions, the result is bit-identical to the reference's.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -39,6 +47,8 @@ constexpr int kMaxTileLines = 64;
 // coefficients) are issued together, then substituted in order, then
 // stored.
 constexpr int kBatch = 8;
+// Loads of a tile copy in flight per thread.
+constexpr int kCopyBatch = 8;
 
 template <int BW, bool CYC, typename C>
 struct LineState {
@@ -313,28 +323,513 @@ __device__ __forceinline__ void warm_factors(const SolveParams& sp, int64_t n) {
     asm volatile("" ::"v"(acc));  // the loads' results are used
 }
 
-// Fallback: one lane per line, substituting in HBM (storage T, compute C;
-// with T narrower than C the forward results are rounded to T between
-// the two sweeps).
+// ---- segmented substitution ---------------------------------------------
+//
+// A line's substitution is one dependent chain of rows, but the chain
+// forgets: an interpolating spline's LU recurrences contract (0.27 per row
+// at order 3, 0.54 at order 7), so started `warm` rows early from a zero
+// state they arrive at the very bits of the full recurrence (measured over
+// all orders, 2 to 7, clamped, periodic and graded, on noise and on smooth
+// data: 27 to 38 rows at the worst for orders 2 and 3 in FP64, 97 at order
+// 7; the median is 22, 30 and 66).  So the line is cut into segments, one
+// lane each.  Every lane warms up on the rows before its segment without
+// storing, then substitutes its own rows.  Afterwards each lane compares
+// the state it started from with the rows its neighbour stored, bit for
+// bit.  Equal states mean equal rows, so a line that passes holds exactly
+// the sequential result.  If any comparison of a workgroup fails, the tile
+// is loaded again and solved with one segment per line.  That happens on
+// exactly constant lines (two starts can settle on neighbouring fixed
+// points: 0.7 to 16 % of the boundaries for orders 3 and 4, up to 40 % at
+// order 5), on long runs of zeros after data (a true state there is a tail
+// of the data) and on infinities and NaN.
+//
+// The strips of a cyclic matrix are the other chain: x[n-BW+q] minus
+// bottom[q][j] * y[j] over all j.  The strip decays like the recurrence, so
+// after a prefix of `warm` rows, summed in order, the remaining terms are
+// below the rounding of the sum A.  That is checked too: with t the
+// largest remaining strip entry (strip_rest) times the largest |y|,
+// A - t == A and A + t == A make every later subtraction a no-op
+// (rounding is monotonic).
+//
+// Rows whose factors repeat bit for bit (the interior of a uniform grid,
+// all but the first ~8 * order rows and the last few) take them from
+// registers instead of memory: [flo, fhi) for the forward sweep and [blo,
+// bhi) for the backward one.
+constexpr int kSegRows = 8;  // segments and warm-ups are multiples of this
 
-// Odd LDS row stride (in elements), so that lanes reading the same column
-// of their rows hit distinct banks.
-__host__ __device__ __forceinline__ int64_t tile_stride(int64_t n) { return n | 1; }
+__device__ __forceinline__ bool same_bits(double a, double b) {
+    return __double_as_longlong(a) == __double_as_longlong(b);
+}
+__device__ __forceinline__ bool same_bits(float a, float b) { return __float_as_int(a) == __float_as_int(b); }
 
-// One workgroup: lines [blockIdx.x * lpb, + lpb) staged through LDS in
-// the compute type C; the table holds T.  With sp.accum set, the solved
-// lines are added into accum instead of being stored to x.
-// WARM: warm_factors before the substitution (single-spline launches).
-template <int BW, bool CYC, typename T, typename C, int B = batch_rows<BW, CYC>(), int NT = kTileThreads,
-          bool WARM = false>
+// Factors of the rows outside [flo, fhi) and [blo, bhi), with one row of
+// each range for the rest, staged in LDS after the tile: a few rows on a
+// uniform grid.  On grids where that is more than kEdgeMax elements (the
+// non-uniform ones) nothing is staged and every row reads global memory.
+constexpr int kEdgeMax = 1024;
+
+__host__ __device__ __forceinline__ int edge_elements(int64_t n, int bw, const SolveParams& sp) {
+    const int64_t e = (sp.flo + 1 + n - sp.fhi) * bw + (sp.blo + 1 + n - sp.bhi) * (bw + 1);
+    return sp.segs > 0 && e <= kEdgeMax ? static_cast<int>(e) : 0;
+}
+
+// Row of the staged table that stands for row r, and its inverse.
+__device__ __forceinline__ int edge_row(int r, int lo, int hi) { return r < hi ? min(r, lo) : r - hi + lo + 1; }
+__device__ __forceinline__ int edge_source(int i, int lo, int hi) { return i <= lo ? i : i - lo - 1 + hi; }
+
+template <typename C>
+struct EdgeTable {
+    const C* lower = nullptr;  // LDS, or null
+    const C* upper = nullptr;
+    const C* diag = nullptr;
+};
+
+template <int BW, typename C>
+__device__ __forceinline__ EdgeTable<C> stage_edges(const SolveParams& sp, C* lds, int tid, int NT) {
+    const int n = static_cast<int>(sp.n);
+    EdgeTable<C> t;
+    if (edge_elements(n, BW, sp) == 0) return t;
+    const int ef = sp.flo + 1 + n - sp.fhi, eb = sp.blo + 1 + n - sp.bhi;
+    const GlobalPtr<C> lower = (GlobalPtr<C>)(sp.lower);
+    const GlobalPtr<C> upper = (GlobalPtr<C>)(sp.upper);
+    const GlobalPtr<C> diag = (GlobalPtr<C>)(sp.diag);
+    C* el = lds;
+    C* eu = el + ef * BW;
+    C* ed = eu + eb * BW;
+    for (int i = tid; i < ef; i += NT) {
+        const int r = edge_source(i, sp.flo, sp.fhi);
+#pragma unroll
+        for (int m = 0; m < BW; ++m) el[i * BW + m] = r < n ? lower[r * BW + m] : C(0);
+    }
+    for (int i = tid; i < eb; i += NT) {
+        const int r = edge_source(i, sp.blo, sp.bhi);
+#pragma unroll
+        for (int m = 0; m < BW; ++m) eu[i * BW + m] = r < n ? upper[r * BW + m] : C(0);
+        ed[i] = r < n ? diag[r] : C(1);
+    }
+    t.lower = el;
+    t.upper = eu;
+    t.diag = ed;
+    return t;
+}
+
+// The batches t (multiples of B) of a sweep in which every lane of the
+// wave is on rows of equal factors, as one scalar range.  The lane of
+// segment s covers rows len * s - before + t .. + B - 1 (sweep order), of
+// which [lo, hi) have equal factors and rows from `end` on do not count;
+// the wave holds the segments first .. last.  The first segment of a wave
+// reaches `lo` last and its last segment leaves `hi` first.
+struct BatchRange {
+    int lo, hi;
+};
+
+__device__ __forceinline__ BatchRange equal_batches(int first, int last, int len, int before, int count, int lo,
+                                                    int hi, int end, int B) {
+    const int a = lo - (first * len - before), b = hi - (last * len - before);
+    BatchRange r;
+    r.lo = a > 0 ? (a + B - 1) / B * B : 0;
+    r.hi = hi >= end ? count : b < 0 ? 0 : min(b / B * B, count);
+    if (first > last) r = {0, 0};
+    return r;
+}
+
+// One batch of forward rows (row u at x + u * step) from right-hand sides
+// xb; lc(u, m) gives the factors.
+template <int BW, bool CYC, bool STORE, typename C, int B, typename L>
+__device__ __forceinline__ void seg_forward_rows(const C (&xb)[B], C* x, int step, C (&hist)[BW + 1], C& vmax, L lc) {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+        C v = xb[u];
+#pragma unroll
+        for (int m = BW; m >= 1; --m) v = v - lc(u, m - 1) * hist[m - 1];
+#pragma unroll
+        for (int m = BW; m >= 2; --m) hist[m - 1] = hist[m - 2];
+        if (BW > 0) hist[0] = v;
+        if constexpr (STORE) {
+            x[u * step] = v;
+            if constexpr (CYC) vmax = fmax(vmax, fabs(v));
+        }
+    }
+}
+
+// Rows j0 .. j0+count-1 (both multiples of B; batches below row 0 or from
+// `end` on are skipped) of one lane.  The batches of equal factors run in a
+// loop of their own, the next batch's right-hand sides in flight while one
+// is substituted; the few others before and after it in a second.  A batch
+// that crosses `end` also stores up to B - 1 rows after it.
+template <int BW, bool CYC, bool STORE, typename C, int B>
+__device__ __forceinline__ void seg_forward(C* line, int step, int j0, int count, int end, bool mine, BatchRange eq,
+                                            const SolveParams& sp, const EdgeTable<C>& edge, C (&hist)[BW + 1],
+                                            C& vmax) {
+    const GlobalPtr<C> __restrict__ lower = (GlobalPtr<C>)(sp.lower);
+    C kl[BW + 1];
+#pragma unroll
+    for (int m = 0; m < BW; ++m) kl[m] = static_cast<C>(sp.eq_lower[m]);
+    const int stride = B * step, low = -B * step, high = end * step;
+    int t = 0;
+#pragma unroll 1
+    for (int part = 0; part < 2; ++part) {
+        const int stop = part == 0 ? min(eq.lo, count) : count;
+#pragma unroll 1
+        for (; t < stop; t += B) {
+            const int j = j0 + t;
+            if (!(mine && j >= 0 && j < end)) continue;
+            C xb[B], lb[B][BW + 1];
+            C* x = line + j * step;
+#pragma unroll
+            for (int u = 0; u < B; ++u) xb[u] = x[u * step];
+            if (edge.lower) {
+#pragma unroll
+                for (int u = 0; u < B; ++u) {
+                    const int r = edge_row(min(j + u, end - 1), sp.flo, sp.fhi);
+#pragma unroll
+                    for (int m = 0; m < BW; ++m) lb[u][m] = edge.lower[r * BW + m];
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < B; ++u)
+#pragma unroll
+                    for (int m = 0; m < BW; ++m) lb[u][m] = lower[min(j + u, end - 1) * BW + m];
+            }
+            seg_forward_rows<BW, CYC, STORE, C, B>(xb, x, step, hist, vmax, [&](int u, int m) { return lb[u][m]; });
+        }
+        if (part == 1 || t >= eq.hi) continue;
+        // batches outside [0, end) read the rows next to it, which are there
+        // (the tile is padded by B rows on both sides)
+        int at = (j0 + t) * step;
+        C xa[B], xb[B];
+        auto load = [&](C (&xv)[B], int i) {
+            i = min(max(i, low), high);
+#pragma unroll
+            for (int u = 0; u < B; ++u) xv[u] = line[i + u * step];
+        };
+        auto run = [&](const C (&xv)[B]) {
+            const int j = j0 + t;
+            if (mine && j >= 0 && j < end)
+                seg_forward_rows<BW, CYC, STORE, C, B>(xv, line + at, step, hist, vmax,
+                                                       [&](int, int m) { return kl[m]; });
+            t += B;
+            at += stride;
+            asm volatile("" : "+v"(at));  // one running index, not one per row
+        };
+        load(xa, at);
+#pragma unroll 1
+        while (true) {
+            load(xb, at + stride);
+            run(xa);
+            if (t >= eq.hi) break;
+            load(xa, at + stride);
+            run(xb);
+            if (t >= eq.hi) break;
+        }
+    }
+}
+
+// v / d for the pivot d of the rows [blo, bhi) in two operations, RN(v zh
+// + RN(v zl)) with zh + zl the reciprocal of d (Brisebarre, Muller and
+// Raina, "Accelerating correctly rounded floating-point division when the
+// divisor is known in advance", IEEE Transactions on Computers 53(8),
+// 2004).  The host has checked every numerator whose quotient lies near
+// enough to a rounding boundary, so the result is the correctly rounded
+// quotient (zl >= 0 keeps the sign of a zero) unless v zl underflows,
+// which the caller's check of the smallest exponent finds, or v is
+// infinite, which its finite check finds.
+template <typename C>
+struct KnownDivisor {
+    C zh, zl;
+    // the smallest exponent of a numerator so far (a zero, an infinity and
+    // a NaN count as 0)
+    __device__ __forceinline__ C divide(C v, int& least) const {
+#pragma clang fp contract(off)
+        if constexpr (sizeof(C) == 8) {
+            least = min(least, __builtin_amdgcn_frexp_exp(v));
+            return __builtin_fma(v, zh, v * zl);
+        } else {
+            least = min(least, __builtin_amdgcn_frexp_expf(v));
+            return __builtin_fmaf(v, zh, v * zl);
+        }
+    }
+    __device__ __forceinline__ static bool underflows(int least) { return least < (sizeof(C) == 8 ? -900 : -90); }
+};
+
+// One batch of backward rows (row u at x - u * step, u downward from row j).
+template <int BW, bool CYC, bool STORE, typename C, int B, typename U, typename D, typename R>
+__device__ __forceinline__ void seg_backward_rows(const C (&xb)[B], C* x, int step, int n, int j,
+                                                  const C (&corner)[BW + 1], C (&nxt)[BW + 1], U uc, D divide, R rc) {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+        C v = xb[u];
+        if constexpr (CYC) {
+#pragma unroll
+            for (int c = BW - 1; c >= 0; --c)
+                if (j - u < n - BW + c - BW) v = v - rc(u, c) * corner[c];
+        }
+#pragma unroll
+        for (int m = BW; m >= 1; --m) v = v - uc(u, m - 1) * nxt[m - 1];
+        v = divide(u, v);
+#pragma unroll
+        for (int m = BW; m >= 2; --m) nxt[m - 1] = nxt[m - 2];
+        if (BW > 0) nxt[0] = v;
+        if constexpr (STORE) x[-u * step] = v;
+    }
+}
+
+// Rows j0, j0-1, .., j0-count+1 of one lane (batches below row 0 or from
+// `end` on are skipped; j0 + 1 - end and count are multiples of B), in two
+// loops like seg_forward.  A batch that crosses row 0 also stores up to
+// B - 1 rows before it.
+template <int BW, bool CYC, bool STORE, typename C, int B>
+__device__ __forceinline__ void seg_backward(C* line, int step, int n, int j0, int count, int end, bool mine,
+                                             BatchRange eq, const SolveParams& sp, const EdgeTable<C>& edge,
+                                             const KnownDivisor<C>& kz, const C (&corner)[BW + 1], C (&nxt)[BW + 1],
+                                             int& least) {
+    const GlobalPtr<C> __restrict__ upper = (GlobalPtr<C>)(sp.upper);
+    const GlobalPtr<C> __restrict__ diag = (GlobalPtr<C>)(sp.diag);
+    const GlobalPtr<C> __restrict__ right = (GlobalPtr<C>)(sp.right);
+    C ku[BW + 1];
+#pragma unroll
+    for (int m = 0; m < BW; ++m) ku[m] = static_cast<C>(sp.eq_upper[m]);
+    if (!sp.fast_divide) eq.hi = eq.lo = 0;
+    const int stride = B * step, low = -step, high = (end + B - 1) * step;
+    auto load_strips = [&](C (&rb)[B][BW + 1], int j) {
+        if constexpr (CYC) {
+#pragma unroll
+            for (int u = 0; u < B; ++u)
+#pragma unroll
+                for (int c = 0; c < BW; ++c) rb[u][c] = right[c * n + min(max(j - u, 0), n - 1)];
+        }
+    };
+    int t = 0;
+#pragma unroll 1
+    for (int part = 0; part < 2; ++part) {
+        const int stop = part == 0 ? min(eq.lo, count) : count;
+#pragma unroll 1
+        for (; t < stop; t += B) {
+            const int j = j0 - t;
+            if (!(mine && j >= 0 && j < end)) continue;
+            C xb[B], rb[B][BW + 1], ub[B][BW + 1], db[B];
+            C* x = line + j * step;
+#pragma unroll
+            for (int u = 0; u < B; ++u) xb[u] = x[-u * step];
+            load_strips(rb, j);
+            if (edge.lower) {
+#pragma unroll
+                for (int u = 0; u < B; ++u) {
+                    const int r = edge_row(max(j - u, 0), sp.blo, sp.bhi);
+#pragma unroll
+                    for (int m = 0; m < BW; ++m) ub[u][m] = edge.upper[r * BW + m];
+                    db[u] = edge.diag[r];
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < B; ++u) {
+#pragma unroll
+                    for (int m = 0; m < BW; ++m) ub[u][m] = upper[max(j - u, 0) * BW + m];
+                    db[u] = diag[max(j - u, 0)];
+                }
+            }
+            seg_backward_rows<BW, CYC, STORE, C, B>(xb, x, step, n, j, corner, nxt,
+                                                    [&](int u, int m) { return ub[u][m]; },
+                                                    [&](int u, C v) { return v / db[u]; },
+                                                    [&](int u, int c) { return rb[u][c]; });
+        }
+        if (part == 1 || t >= eq.hi) continue;
+        int at = (j0 - t) * step;
+        C xa[B], xb[B], ra[B][BW + 1], rb[B][BW + 1];
+        auto load = [&](C (&xv)[B], C (&rv)[B][BW + 1], int i, int j) {
+            i = min(max(i, low), high);
+#pragma unroll
+            for (int u = 0; u < B; ++u) xv[u] = line[i - u * step];
+            load_strips(rv, j);
+        };
+        auto run = [&](const C (&xv)[B], const C (&rv)[B][BW + 1]) {
+            const int j = j0 - t;
+            if (mine && j >= 0 && j < end)
+                seg_backward_rows<BW, CYC, STORE, C, B>(xv, line + at, step, n, j, corner, nxt,
+                                                        [&](int, int m) { return ku[m]; },
+                                                        [&](int, C v) { return kz.divide(v, least); },
+                                                        [&](int u, int c) { return rv[u][c]; });
+            t += B;
+            at -= stride;
+            asm volatile("" : "+v"(at));  // one running index, not one per row
+        };
+        load(xa, ra, at, j0 - t);
+#pragma unroll 1
+        while (true) {
+            load(xb, rb, at - stride, j0 - t - B);
+            run(xa, ra);
+            if (t >= eq.hi) break;
+            load(xa, ra, at - stride, j0 - t - B);
+            run(xb, rb);
+            if (t >= eq.hi) break;
+        }
+    }
+}
+
+// Substitutes the lines of one tile (rows of `step` elements, line l at
+// tile + l) in `segs` segments each, thread tid taking segment tid / lpb of
+// line tid % lpb.  False: a comparison failed and the tile's contents are
+// undefined.  Every thread of the workgroup takes part.
+template <int BW, bool CYC, typename C, int B>
+__device__ __forceinline__ bool solve_segments(const SolveParams& sp, C* tile, int step, int nl, int lpb, int segs,
+                                               const EdgeTable<C>& edge, int tid, int* failed) {
+    const int n = static_cast<int>(sp.n);
+    const int shift = __builtin_ctz(static_cast<unsigned>(lpb));
+    const int line = tid & (lpb - 1), seg = tid >> shift;
+    const int H = CYC ? n - BW : n;  // the last BW rows of a cyclic matrix follow the strips
+    const int len = ((H + segs - 1) / segs + kSegRows - 1) / kSegRows * kSegRows;
+    const int warm = sp.warm;
+    const bool mine = line < nl && seg < segs && seg * len < H;
+    // the wave's segments (a wave is 64 threads in a row of tid)
+    const int wave = __builtin_amdgcn_readfirstlane(tid) & ~63;
+    const int seg0 = wave >> shift, seg1 = min((wave + 63) >> shift, (H + len - 1) / len - 1);
+    C* x = tile + line;
+    C hist[BW + 1], start[BW + 1], corner[BW + 1];
+    C vmax = C(0);
+#pragma unroll
+    for (int m = 0; m <= BW; ++m) hist[m] = start[m] = corner[m] = C(0);
+    // whether any thread's `bad` is set (LDS flag, cleared below between
+    // barriers)
+    auto any_bad = [&](bool bad) {
+        if (__any(bad) && (threadIdx.x & 63) == 0) *failed = 1;
+        __syncthreads();
+        return *failed != 0;
+    };
+    if (tid == 0) *failed = 0;
+    // forward
+    const int a = seg * len;
+    C strip_row = C(0);  // x[n-BW+q] of the thread that sums strip q (the forward sweep stores past row H)
+    if constexpr (CYC && BW > 0) {
+        if (line < nl && seg < BW) strip_row = x[(H + seg) * step];
+    }
+    if (segs > 1) {
+        seg_forward<BW, CYC, false, C, B>(x, step, a - warm, warm, H, mine && seg > 0,
+                                          equal_batches(max(seg0, 1), seg1, len, warm, warm, sp.flo, sp.fhi, H, B),
+                                          sp, edge, hist, vmax);
+#pragma unroll
+        for (int m = 0; m < BW; ++m) start[m] = hist[m];
+    }
+    __syncthreads();
+    seg_forward<BW, CYC, true, C, B>(x, step, a, len, H, mine,
+                                     equal_batches(seg0, seg1, len, 0, len, sp.flo, sp.fhi, H, B), sp, edge, hist,
+                                     vmax);
+    __syncthreads();
+    bool bad = false;
+    if (mine && seg > 0) {
+#pragma unroll
+        for (int m = 0; m < BW; ++m) bad = bad || !same_bits(start[m], x[(a - 1 - m) * step]);
+    }
+    if constexpr (CYC && BW > 0) {
+        if (mine) bad = bad || !(hist[0] - hist[0] == C(0));  // infinities and NaN
+        if (line < nl) {
+#pragma clang fp contract(off)
+            const GlobalPtr<C> __restrict__ bottom = (GlobalPtr<C>)(sp.bottom);
+            if (seg < BW) {
+                C acc = strip_row;
+                const int last = min(warm, n - 2 * BW + seg);
+#pragma unroll 8
+                for (int j = 0; j < last; ++j) acc = acc - bottom[seg * n + j] * x[j * step];
+                x[(H + seg) * step] = acc;
+            }
+        }
+        __syncthreads();
+        if (mine) {
+#pragma unroll
+            for (int q = 0; q < BW; ++q) {
+                const C A = x[(H + q) * step];
+                const C t = static_cast<C>(sp.strip_rest) * vmax;
+                bad = bad || !(A - t == A && A + t == A) || same_bits(A, C(-0.0));
+            }
+        }
+        if (any_bad(bad)) return false;
+        if (line < nl && seg == 0) {
+            // the last rows, then the backward rows that fix the corners
+            LineState<BW, CYC, C> st;
+#pragma unroll
+            for (int m = 0; m <= BW; ++m) st.hist[m] = st.nxt[m] = st.corner[m] = st.acc[m] = C(0);
+#pragma unroll
+            for (int m = 0; m < BW; ++m) {
+                st.hist[m] = x[(H - 1 - m) * step];
+                st.acc[m] = x[(H + m) * step];
+            }
+            const int32_t z = lane_zero();
+            forward_range<BW, CYC, C, C, 1>(x, step, n, H, n, sp, st, z);
+            backward_range<BW, CYC, C, C, 1>(x, step, n, H, n, sp, st, z);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < BW; ++c) corner[c] = x[(H + c) * step];
+    } else {
+        if (segs > 1 && any_bad(bad)) return false;
+    }
+    // backward: segment `seg` from the end; in sweep order row r is H - 1 - r
+    const int top = H - seg * len;
+    const int blo = H - min(sp.bhi, H), bhi = H - sp.blo;
+    const KnownDivisor<C> kz{static_cast<C>(sp.zh), static_cast<C>(sp.zl)};
+    int least = 0;
+    C nxt[BW + 1];
+    nxt[BW] = C(0);
+#pragma unroll
+    for (int m = 0; m < BW; ++m) nxt[m] = CYC && top + warm >= H ? corner[m] : C(0);
+    if (segs > 1) {
+        seg_backward<BW, CYC, false, C, B>(x, step, n, top + warm - 1, warm, H, mine && seg > 0,
+                                           equal_batches(max(seg0, 1), seg1, len, warm, warm, blo, bhi, H, B), sp,
+                                           edge, kz, corner, nxt, least);
+#pragma unroll
+        for (int m = 0; m < BW; ++m) start[m] = nxt[m];
+        __syncthreads();
+    }
+    seg_backward<BW, CYC, true, C, B>(x, step, n, top - 1, len, H, mine,
+                                      equal_batches(seg0, seg1, len, 0, len, blo, bhi, H, B), sp, edge, kz, corner,
+                                      nxt, least);
+    __syncthreads();
+    bad = kz.underflows(least);
+    if (mine) {
+        if (BW > 0) bad = bad || !(nxt[0] - nxt[0] == C(0));  // infinities and NaN
+        if (seg > 0) {
+#pragma unroll
+            for (int m = 0; m < BW; ++m) bad = bad || !same_bits(start[m], x[(top + m) * step]);
+        }
+    }
+    return !any_bad(bad);
+}
+
+// Row stride of a tile in elements: odd on the contiguous axis, so that
+// the coalesced runs along a line spread over the LDS banks, and for
+// kTileLines lines on any axis.
+constexpr int kTileLines = 32;
+constexpr int kTileStep = kTileLines + 1;
+__host__ __device__ __forceinline__ int64_t tile_step(int64_t lpb, int64_t inner) {
+    return inner == 1 || lpb == kTileLines ? lpb | 1 : lpb;
+}
+// Rows before and after the tile, zeroed: a segment's first or last batch
+// can read and write past the line's ends.
+constexpr int64_t kTilePad = kSegRows;
+__host__ __device__ __forceinline__ int64_t tile_elements(int64_t n, int64_t lpb, int64_t inner) {
+    return (n + 2 * kTilePad) * tile_step(lpb, inner);
+}
+
+// One workgroup: lines [first, first + lpb) staged through LDS in the
+// compute type C; the table holds T.  Row j of line l sits at
+// tile[j * step + l].  With sp.accum set, the solved lines are added into
+// accum instead of being stored to x.  segs == 0: plain substitution.
+// tid: the thread's place in the workgroup of NT threads, whole waves of it
+// in any order (the callers rotate the waves: where one wave substitutes,
+// neighbouring workgroups on a CU then use different SIMDs).
+// SEG false: kernels whose lines are never cut.  FIXED: with a copy of the
+// segment code for the row stride kTileStep.
+template <int BW, bool CYC, typename T, typename C, int B = batch_rows<BW, CYC>(), bool SEG = true,
+          bool FIXED = true>
 __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first, unsigned char* tile_bytes,
-                                           int64_t* dst_base, int64_t* src_base) {
-    C* tile = reinterpret_cast<C*>(tile_bytes);
-    T* __restrict__ X = static_cast<T*>(sp.x);
+                                           int64_t* dst_base, int64_t* src_base, int tid, int NT) {
     const int lpb = sp.lines_per_block;
-    const int64_t n = sp.n, inner = sp.inner, stride = tile_stride(n);
+    const int64_t n = sp.n, inner = sp.inner;
+    const int step = static_cast<int>(tile_step(lpb, inner));
+    C* tile = reinterpret_cast<C*>(tile_bytes) + kTilePad * step;
+    T* __restrict__ X = static_cast<T*>(sp.x);
     const int nl = static_cast<int>(min(static_cast<int64_t>(lpb), sp.nlines - first));
-    const int tid = threadIdx.x;
     if (tid < nl) {
         const int64_t line = first + tid;
         const int64_t o = line / inner, ii = line - o * inner;
@@ -360,101 +855,166 @@ __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first,
     }
     __syncthreads();
 
-    // ---- load ----
-    // Contiguous lines: tile element e is (line e / n, element e % n).
-    // Strided lines: (line e % lpb, element e / lpb); as NT % lpb == 0 a
-    // thread keeps one line.
+    // Contiguous lines: tile element e is (line e / n, row e % n).
+    // Strided lines: (line e % lpb, row e / lpb); as NT % lpb == 0 a
+    // thread keeps one line.  Pairs (FP64) or quads (FP32) of strided lines
+    // that are adjacent and aligned in memory move as 16-byte vectors.  A
+    // batch of kCopyBatch loads is in flight at once: a tile is a round
+    // trip or two, not one per few elements.
+    typedef T VecT __attribute__((ext_vector_type(16 / sizeof(T))));
+    constexpr int V = 16 / sizeof(T);
     const uint32_t un = static_cast<uint32_t>(n);
     const int lshift = __builtin_ctz(static_cast<unsigned>(lpb));
     const uint32_t count = static_cast<uint32_t>(inner == 1 ? nl * n : lpb * n);
     const uint32_t my_l = static_cast<uint32_t>(tid) & static_cast<uint32_t>(lpb - 1);
-    if (sp.src) {
-        for (uint32_t e0 = tid; e0 < count; e0 += NT * kBatch) {
-            int64_t from[kBatch];
-            uint32_t at[kBatch];
+    const bool vec = inner > 1 && lpb >= V && inner % V == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0 &&
+                     (reinterpret_cast<uintptr_t>(sp.accum) & 15) == 0;
+    const int vshift = lshift - __builtin_ctz(static_cast<unsigned>(V));
+    const uint32_t my_v = (static_cast<uint32_t>(tid) & ((1u << max(vshift, 0)) - 1u)) * V;
+    auto load = [&]() {
+        if (sp.src) {
+            for (uint32_t e0 = tid; e0 < count; e0 += NT * kCopyBatch) {
+                // the values are read once: non-temporal loads keep them from
+                // evicting the factors and the lines being written
+                C v[kCopyBatch];
+                uint32_t at[kCopyBatch];
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                const uint32_t e = min(e0 + u * NT, count - 1);
-                const uint32_t l = e / un, jj = e - l * un;
-                int64_t js = static_cast<int64_t>(jj) - sp.shift_last;
-                if (js < 0) js += n;
-                from[u] = src_base[l] + js;
-                at[u] = l * static_cast<uint32_t>(stride) + jj;
+                for (int u = 0; u < kCopyBatch; ++u) {
+                    const uint32_t e = min(e0 + u * NT, count - 1);
+                    const uint32_t l = fast_div(e, sp.div_n), jj = e - l * un;
+                    int64_t js = static_cast<int64_t>(jj) - sp.shift_last;
+                    if (js < 0) js += n;
+                    v[u] = static_cast<C>(__builtin_nontemporal_load(&sp.src[src_base[l] + js]));
+                    at[u] = jj * static_cast<uint32_t>(step) + l;
+                }
+#pragma unroll
+                for (int u = 0; u < kCopyBatch; ++u)
+                    if (e0 + u * NT < count) tile[at[u]] = v[u];
             }
-            // the values are read once: non-temporal loads keep them from
-            // evicting the factors and the lines being written
-            C v[kBatch];
+        } else if (inner == 1) {
+            const T* __restrict__ base = X + first * n;
+            for (uint32_t e0 = tid; e0 < count; e0 += NT * kCopyBatch) {
+                C v[kCopyBatch];
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u) v[u] = static_cast<C>(__builtin_nontemporal_load(&sp.src[from[u]]));
+                for (int u = 0; u < kCopyBatch; ++u) v[u] = static_cast<C>(base[min(e0 + u * NT, count - 1)]);
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u)
-                if (e0 + u * NT < count) tile[at[u]] = v[u];
-        }
-    } else if (inner == 1) {
-        const T* __restrict__ base = X + first * n;
-        for (uint32_t e0 = tid; e0 < count; e0 += NT * kBatch) {
-            C v[kBatch];
+                for (int u = 0; u < kCopyBatch; ++u) {
+                    const uint32_t e = e0 + u * NT;
+                    if (e < count) {
+                        const uint32_t l = fast_div(e, sp.div_n), jj = e - l * un;
+                        tile[jj * static_cast<uint32_t>(step) + l] = v[u];
+                    }
+                }
+            }
+        } else if (vec) {
+            if (static_cast<int>(my_v) < nl) {
+                const T* __restrict__ line = X + dst_base[my_v];
+                const uint32_t rows = NT >> vshift;
+                for (uint32_t j0 = static_cast<uint32_t>(tid) >> vshift; j0 < un; j0 += rows * kCopyBatch) {
+                    VecT v[kCopyBatch];
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u) v[u] = static_cast<C>(base[min(e0 + u * NT, count - 1)]);
+                    for (int u = 0; u < kCopyBatch; ++u)
+                        v[u] = *reinterpret_cast<const VecT*>(
+                            line + static_cast<int64_t>(min(j0 + u * rows, un - 1)) * inner);
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                const uint32_t e = e0 + u * NT;
-                if (e < count) {
-                    const uint32_t l = e / un, jj = e - l * un;
-                    tile[l * static_cast<uint32_t>(stride) + jj] = v[u];
+                    for (int u = 0; u < kCopyBatch; ++u)
+                        if (j0 + u * rows < un) {
+#pragma unroll
+                            for (int i = 0; i < V; ++i)
+                                tile[(j0 + u * rows) * static_cast<uint32_t>(step) + my_v + i] = static_cast<C>(v[u][i]);
+                        }
+                }
+            }
+        } else if (static_cast<int>(my_l) < nl) {
+            const T* __restrict__ line = X + dst_base[my_l];
+            for (uint32_t e0 = tid; e0 < count; e0 += NT * kCopyBatch) {
+                C v[kCopyBatch];
+#pragma unroll
+                for (int u = 0; u < kCopyBatch; ++u) {
+                    const uint32_t jj = min(e0 + u * NT, count - 1) >> lshift;
+                    v[u] = static_cast<C>(line[static_cast<int64_t>(jj) * inner]);
+                }
+#pragma unroll
+                for (int u = 0; u < kCopyBatch; ++u) {
+                    const uint32_t e = e0 + u * NT;
+                    if (e < count) tile[(e >> lshift) * static_cast<uint32_t>(step) + my_l] = v[u];
                 }
             }
         }
-    } else if (static_cast<int>(my_l) < nl) {
-        const T* __restrict__ line = X + dst_base[my_l];
-        C* __restrict__ row = tile + my_l * stride;
-        for (uint32_t e0 = tid; e0 < count; e0 += NT * kBatch) {
-            C v[kBatch];
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                const uint32_t jj = min(e0 + u * NT, count - 1) >> lshift;
-                v[u] = static_cast<C>(line[static_cast<int64_t>(jj) * inner]);
-            }
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                const uint32_t e = e0 + u * NT;
-                if (e < count) row[e >> lshift] = v[u];
-            }
+        __syncthreads();
+    };
+    bool done = false;
+    if constexpr (SEG) {
+        __shared__ int failed;
+        EdgeTable<C> edge;
+        if (sp.segs > 0) {
+            const int pad = static_cast<int>(kTilePad) * step;
+            for (int i = tid; i < pad; i += NT) tile[i - pad] = tile[static_cast<int>(n) * step + i] = C(0);
+            edge = stage_edges<BW, C>(sp, reinterpret_cast<C*>(tile_bytes) + tile_elements(n, lpb, inner), tid, NT);
         }
+        load();
+        // segmented; then, if a comparison failed, one segment per line;
+        // then, if the strips or a pivot's division need it, the plain
+        // substitution
+#pragma unroll 1
+        for (int segs = sp.segs; segs > 0 && !done; segs = segs > 1 ? 1 : 0) {
+            // the usual row stride of many lines as a constant: row offsets
+            // become immediates of the LDS instructions
+            if (FIXED && step == kTileStep)
+                done = solve_segments<BW, CYC, C, B>(sp, tile, kTileStep, nl, lpb, segs, edge, tid, &failed);
+            else
+                done = solve_segments<BW, CYC, C, B>(sp, tile, step, nl, lpb, segs, edge, tid, &failed);
+            if (!done) load();
+        }
+    } else {
+        load();
     }
-    if constexpr (WARM) warm_factors<BW, CYC, C, NT>(sp, n);
-    __syncthreads();
-
-    if (tid < nl) substitute<BW, CYC, C, C, B>(tile + tid * stride, 1, n, sp);
-    __syncthreads();
+    if (!done) {
+        if (tid < nl) substitute<BW, CYC, C, C, B>(tile + tid, step, n, sp);
+        __syncthreads();
+    }
 
     // ---- store ----
     T* __restrict__ Y = sp.accum ? static_cast<T*>(sp.accum) : X;
     const bool add = sp.accum != nullptr;
     if (inner == 1) {
         T* __restrict__ base = Y + first * n;
-        for (uint32_t e0 = tid; e0 < count; e0 += NT * kBatch) {
-            C v[kBatch];
+        for (uint32_t e0 = tid; e0 < count; e0 += NT * kCopyBatch) {
+            C v[kCopyBatch];
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
+            for (int u = 0; u < kCopyBatch; ++u) {
                 const uint32_t e = min(e0 + u * NT, count - 1);
-                const uint32_t l = e / un, jj = e - l * un;
-                v[u] = tile[l * static_cast<uint32_t>(stride) + jj];
+                const uint32_t l = fast_div(e, sp.div_n), jj = e - l * un;
+                v[u] = tile[jj * static_cast<uint32_t>(step) + l];
             }
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u)
+            for (int u = 0; u < kCopyBatch; ++u)
                 if (e0 + u * NT < count) {
                     T* at = base + e0 + u * NT;
                     *at = add ? static_cast<T>(*at + static_cast<T>(v[u])) : static_cast<T>(v[u]);
                 }
         }
+    } else if (vec) {
+        if (static_cast<int>(my_v) < nl) {
+            T* __restrict__ line = Y + dst_base[my_v];
+            const uint32_t rows = NT >> vshift;
+#pragma unroll 4
+            for (uint32_t j = static_cast<uint32_t>(tid) >> vshift; j < un; j += rows) {
+                VecT* at = reinterpret_cast<VecT*>(line + static_cast<int64_t>(j) * inner);
+                VecT v;
+#pragma unroll
+                for (int i = 0; i < V; ++i) v[i] = static_cast<T>(tile[j * static_cast<uint32_t>(step) + my_v + i]);
+                if (add) v = *at + v;
+                *at = v;
+            }
+        }
     } else if (static_cast<int>(my_l) < nl) {
         T* __restrict__ line = Y + dst_base[my_l];
-        const C* __restrict__ row = tile + my_l * stride;
         for (uint32_t e0 = tid; e0 < count; e0 += NT * kBatch) {
             C v[kBatch];
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u) v[u] = row[min(e0 + u * NT, count - 1) >> lshift];
+            for (int u = 0; u < kBatch; ++u)
+                v[u] = tile[(min(e0 + u * NT, count - 1) >> lshift) * static_cast<uint32_t>(step) + my_l];
 #pragma unroll
             for (int u = 0; u < kBatch; ++u) {
                 const uint32_t e = e0 + u * NT;
