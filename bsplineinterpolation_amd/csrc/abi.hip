@@ -389,8 +389,16 @@ int solve_axes(const GridData& g, bool refined, const double* values, void* x, v
         sp->segs = plan.segs;
         return plan;
     };
+    // lines too long for a tile are solved in chunks, through scratch
+    auto long_scratch = [&](int a, const SolveParams& sp) -> size_t {
+        const DimSetup& s = g.setup[a];
+        return sp.lines_per_block > 0
+                   ? 0
+                   : solve_long_scratch(sp, s.lu.p, s.lu.cyclic, compute_bytes(axis_types(g, refined, a)));
+    };
     SolveParams last_params{};
-    const bool fused = values != nullptr && axis_params(last, &last_params).lines > 0;
+    const bool fused =
+        values != nullptr && (axis_params(last, &last_params).lines > 0 || long_scratch(last, last_params) > 0);
     if (values != nullptr && !fused) {
         if (any_shift || refined) {
             ShiftParams sh{};
@@ -431,7 +439,15 @@ int solve_axes(const GridData& g, bool refined, const double* values, void* x, v
         }
         const bool add_after = a == 0 && accum != nullptr && sp.lines_per_block == 0;
         if (a == 0 && accum != nullptr && !add_after) sp.accum = accum;
-        hipError_t e = launch_solve(s.lu.p, s.lu.cyclic, types, sp, plan.threads, stream);
+        hipError_t e;
+        if (const size_t bytes = long_scratch(a, sp)) {
+            void* scratch = nullptr;
+            HIP_TRY(device_alloc(&scratch, bytes, stream), "device allocation (long lines)");
+            e = launch_solve_long(s.lu.p, s.lu.cyclic, types, sp, scratch, stream);
+            (void)hipFreeAsync(scratch, stream);
+        } else {
+            e = launch_solve(s.lu.p, s.lu.cyclic, types, sp, plan.threads, stream);
+        }
         if (e == hipErrorNotSupported) return fail(INTP_E_UNSUPPORTED, "band width without a compiled solver");
         HIP_TRY(e, "solve launch");
         if (add_after) {

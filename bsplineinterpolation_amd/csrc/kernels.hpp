@@ -269,6 +269,12 @@ hipError_t eval_dispatch_f32_d4(int order, bool grad, bool uniform, const EvalPa
 hipError_t eval_dispatch_f32_d5(int order, bool grad, bool uniform, const EvalParams& p, hipStream_t s);
 hipError_t eval_dispatch_f32_d6(int order, bool grad, bool uniform, const EvalParams& p, hipStream_t s);
 hipError_t launch_solve(int bw, bool cyclic, SolveTypes types, const SolveParams& p, int threads, hipStream_t s);
+// Lines too long for a tile (solve_long.hip): scratch bytes of the solve of
+// p's lines in chunks, or 0 where they cannot be cut, and the solve (p as
+// for launch_solve, without accum).
+size_t solve_long_scratch(const SolveParams& p, int bw, bool cyclic, int compute_bytes);
+hipError_t launch_solve_long(int bw, bool cyclic, SolveTypes types, const SolveParams& p, void* scratch,
+                             hipStream_t s);
 // The tile for the lines of p (n, nlines, inner and the segment fields set)
 // on the current device, for compute elements of `compute_bytes`.
 TilePlan solve_tile_plan(const SolveParams& p, int bw, bool cyclic, int compute_bytes);

@@ -8,7 +8,7 @@
 // each (solve_segments), and writes the tile back.  The first pass reads
 // the caller's values with the periodic index shift applied
 // (InterpolationTemplate.hpp:452-462), so no separate copy precedes it.
-// Lines too long for LDS use solve_kernel (one lane per line, in HBM).
+// Lines too long for LDS are cut into chunks first (solve_long.hip).
 //
 // What bounds it.  Substituting a line is a chain of dependent rows: 16
 // cycles forward (order 3), and backward 16 and an IEEE division of 70.
@@ -454,19 +454,20 @@ __device__ __forceinline__ void seg_forward_rows(const C (&xb)[B], C* x, int ste
 }
 
 // Rows j0 .. j0+count-1 (both multiples of B; batches below row 0 or from
-// `end` on are skipped) of one lane.  The batches of equal factors run in a
+// `end` on are skipped) of one lane; row j sits at line[(j - origin) * step],
+// with rows origin - B .. limit + B - 1 there to read.  The batches of equal factors run in a
 // loop of their own, the next batch's right-hand sides in flight while one
 // is substituted; the few others before and after it in a second.  A batch
 // that crosses `end` also stores up to B - 1 rows after it.
 template <int BW, bool CYC, bool STORE, typename C, int B>
-__device__ __forceinline__ void seg_forward(C* line, int step, int j0, int count, int end, bool mine, BatchRange eq,
-                                            const SolveParams& sp, const EdgeTable<C>& edge, C (&hist)[BW + 1],
-                                            C& vmax) {
+__device__ __forceinline__ void seg_forward(C* line, int step, int origin, int limit, int j0, int count, int end,
+                                            bool mine, BatchRange eq, const SolveParams& sp,
+                                            const EdgeTable<C>& edge, C (&hist)[BW + 1], C& vmax) {
     const GlobalPtr<C> __restrict__ lower = (GlobalPtr<C>)(sp.lower);
     C kl[BW + 1];
 #pragma unroll
     for (int m = 0; m < BW; ++m) kl[m] = static_cast<C>(sp.eq_lower[m]);
-    const int stride = B * step, low = -B * step, high = end * step;
+    const int stride = B * step, low = -B * step, high = (limit - origin) * step;
     int t = 0;
 #pragma unroll 1
     for (int part = 0; part < 2; ++part) {
@@ -476,7 +477,7 @@ __device__ __forceinline__ void seg_forward(C* line, int step, int j0, int count
             const int j = j0 + t;
             if (!(mine && j >= 0 && j < end)) continue;
             C xb[B], lb[B][BW + 1];
-            C* x = line + j * step;
+            C* x = line + (j - origin) * step;
 #pragma unroll
             for (int u = 0; u < B; ++u) xb[u] = x[u * step];
             if (edge.lower) {
@@ -495,9 +496,8 @@ __device__ __forceinline__ void seg_forward(C* line, int step, int j0, int count
             seg_forward_rows<BW, CYC, STORE, C, B>(xb, x, step, hist, vmax, [&](int u, int m) { return lb[u][m]; });
         }
         if (part == 1 || t >= eq.hi) continue;
-        // batches outside [0, end) read the rows next to it, which are there
-        // (the tile is padded by B rows on both sides)
-        int at = (j0 + t) * step;
+        // batches outside the held rows read the ones next to them
+        int at = (j0 + t - origin) * step;
         C xa[B], xb[B];
         auto load = [&](C (&xv)[B], int i) {
             i = min(max(i, low), high);
@@ -581,8 +581,8 @@ __device__ __forceinline__ void seg_backward_rows(const C (&xb)[B], C* x, int st
 // loops like seg_forward.  A batch that crosses row 0 also stores up to
 // B - 1 rows before it.
 template <int BW, bool CYC, bool STORE, typename C, int B>
-__device__ __forceinline__ void seg_backward(C* line, int step, int n, int j0, int count, int end, bool mine,
-                                             BatchRange eq, const SolveParams& sp, const EdgeTable<C>& edge,
+__device__ __forceinline__ void seg_backward(C* line, int step, int origin, int n, int j0, int count, int end,
+                                             bool mine, BatchRange eq, const SolveParams& sp, const EdgeTable<C>& edge,
                                              const KnownDivisor<C>& kz, const C (&corner)[BW + 1], C (&nxt)[BW + 1],
                                              int& least) {
     const GlobalPtr<C> __restrict__ upper = (GlobalPtr<C>)(sp.upper);
@@ -592,7 +592,7 @@ __device__ __forceinline__ void seg_backward(C* line, int step, int n, int j0, i
 #pragma unroll
     for (int m = 0; m < BW; ++m) ku[m] = static_cast<C>(sp.eq_upper[m]);
     if (!sp.fast_divide) eq.hi = eq.lo = 0;
-    const int stride = B * step, low = -step, high = (end + B - 1) * step;
+    const int stride = B * step, low = -step, high = (end + B - 1 - origin) * step;
     auto load_strips = [&](C (&rb)[B][BW + 1], int j) {
         if constexpr (CYC) {
 #pragma unroll
@@ -610,7 +610,7 @@ __device__ __forceinline__ void seg_backward(C* line, int step, int n, int j0, i
             const int j = j0 - t;
             if (!(mine && j >= 0 && j < end)) continue;
             C xb[B], rb[B][BW + 1], ub[B][BW + 1], db[B];
-            C* x = line + j * step;
+            C* x = line + (j - origin) * step;
 #pragma unroll
             for (int u = 0; u < B; ++u) xb[u] = x[-u * step];
             load_strips(rb, j);
@@ -636,7 +636,7 @@ __device__ __forceinline__ void seg_backward(C* line, int step, int n, int j0, i
                                                     [&](int u, int c) { return rb[u][c]; });
         }
         if (part == 1 || t >= eq.hi) continue;
-        int at = (j0 - t) * step;
+        int at = (j0 - t - origin) * step;
         C xa[B], xb[B], ra[B][BW + 1], rb[B][BW + 1];
         auto load = [&](C (&xv)[B], C (&rv)[B][BW + 1], int i, int j) {
             i = min(max(i, low), high);
@@ -705,14 +705,14 @@ __device__ __forceinline__ bool solve_segments(const SolveParams& sp, C* tile, i
         if (line < nl && seg < BW) strip_row = x[(H + seg) * step];
     }
     if (segs > 1) {
-        seg_forward<BW, CYC, false, C, B>(x, step, a - warm, warm, H, mine && seg > 0,
+        seg_forward<BW, CYC, false, C, B>(x, step, 0, H, a - warm, warm, H, mine && seg > 0,
                                           equal_batches(max(seg0, 1), seg1, len, warm, warm, sp.flo, sp.fhi, H, B),
                                           sp, edge, hist, vmax);
 #pragma unroll
         for (int m = 0; m < BW; ++m) start[m] = hist[m];
     }
     __syncthreads();
-    seg_forward<BW, CYC, true, C, B>(x, step, a, len, H, mine,
+    seg_forward<BW, CYC, true, C, B>(x, step, 0, H, a, len, H, mine,
                                      equal_batches(seg0, seg1, len, 0, len, sp.flo, sp.fhi, H, B), sp, edge, hist,
                                      vmax);
     __syncthreads();
@@ -774,14 +774,14 @@ __device__ __forceinline__ bool solve_segments(const SolveParams& sp, C* tile, i
 #pragma unroll
     for (int m = 0; m < BW; ++m) nxt[m] = CYC && top + warm >= H ? corner[m] : C(0);
     if (segs > 1) {
-        seg_backward<BW, CYC, false, C, B>(x, step, n, top + warm - 1, warm, H, mine && seg > 0,
+        seg_backward<BW, CYC, false, C, B>(x, step, 0, n, top + warm - 1, warm, H, mine && seg > 0,
                                            equal_batches(max(seg0, 1), seg1, len, warm, warm, blo, bhi, H, B), sp,
                                            edge, kz, corner, nxt, least);
 #pragma unroll
         for (int m = 0; m < BW; ++m) start[m] = nxt[m];
         __syncthreads();
     }
-    seg_backward<BW, CYC, true, C, B>(x, step, n, top - 1, len, H, mine,
+    seg_backward<BW, CYC, true, C, B>(x, step, 0, n, top - 1, len, H, mine,
                                       equal_batches(seg0, seg1, len, 0, len, blo, bhi, H, B), sp, edge, kz, corner,
                                       nxt, least);
     __syncthreads();
