@@ -225,10 +225,21 @@ int check_dims(int dim, int order) {
     return INTP_OK;
 }
 
+// Whether the uniform fast path of the evaluation serves the grid: every
+// dimension uniform (knots in closed form, basis polynomials) and 32-bit
+// table offsets.
+bool uniform_grid(const GridData& g) {
+    if (g.total >= (int64_t{1} << 32)) return false;
+    for (int d = 0; d < g.dim; ++d)
+        if (!g.setup[d].uniform || g.setup[d].poly.empty()) return false;
+    return true;
+}
+
 // Knots, factored collocation matrices and basis tables of `desc`,
 // uploaded on `stream` (on the device's setup stream, waited for, when
 // `stream` is null: a template outlives any one stream).
-int make_grid(intp_ctx ctx, const intp_grid_desc* desc, hipStream_t stream, bool own_stream,
+// `refined`: with the tables of refined builds.
+int make_grid(intp_ctx ctx, const intp_grid_desc* desc, hipStream_t stream, bool own_stream, bool refined,
               std::shared_ptr<GridData>& out) {
     if (!ctx || !desc) return fail(INTP_E_INVALID, "null argument");
     int rc = check_dims(desc->dim, desc->order);
@@ -240,10 +251,12 @@ int make_grid(intp_ctx ctx, const intp_grid_desc* desc, hipStream_t stream, bool
     g->has_factors = true;
     for (int d = 0; d < desc->dim; ++d) {
         const std::string err = setup_dimension(desc->order, desc->periodic[d] != 0, desc->n[d], desc->xmin[d],
-                                                desc->xmax[d], desc->coords[d], g->setup[d]);
+                                                desc->xmax[d], desc->coords[d], g->setup[d], refined);
         if (!err.empty()) return fail(INTP_E_INVALID, err + " (dimension " + std::to_string(d) + ")");
         g->total *= desc->n[d];
     }
+    if (!uniform_grid(*g))
+        for (int d = 0; d < desc->dim; ++d) fill_reciprocals(desc->order, g->setup[d]);
     DeviceScope scope(ctx->device);
     if (!scope.ok()) return fail(INTP_E_HIP, "cannot select device");
     DeviceRuntime* rt = device_runtime(ctx->device);
@@ -269,11 +282,12 @@ constexpr size_t kGridCacheBytes = size_t{8} << 20;
 
 struct GridKey {
     int device = 0, dim = 0, order = 0;
+    bool refined = false;  // with the tables of refined builds
     int64_t n[kMaxDim] = {};
     int32_t periodic[kMaxDim] = {};
     double xmin[kMaxDim] = {}, xmax[kMaxDim] = {};
     bool operator==(const GridKey& o) const {
-        if (device != o.device || dim != o.dim || order != o.order) return false;
+        if (device != o.device || dim != o.dim || order != o.order || refined != o.refined) return false;
         for (int d = 0; d < dim; ++d)
             if (n[d] != o.n[d] || periodic[d] != o.periodic[d] || std::memcmp(&xmin[d], &o.xmin[d], 8) != 0 ||
                 std::memcmp(&xmax[d], &o.xmax[d], 8) != 0)
@@ -332,14 +346,16 @@ void remember_grid(const GridKey& key, const std::shared_ptr<GridData>& g) {
 }
 
 // make_grid for a build: a cached grid when the descriptor has one.
-int build_grid(intp_ctx ctx, const intp_grid_desc* desc, hipStream_t stream, std::shared_ptr<GridData>& out) {
+int build_grid(intp_ctx ctx, const intp_grid_desc* desc, bool refined, hipStream_t stream,
+               std::shared_ptr<GridData>& out) {
     GridKey key;
+    key.refined = refined;
     const bool cacheable = ctx && desc && desc->dim >= 1 && desc->dim <= kMaxDim && grid_key(ctx->device, *desc, &key);
     if (cacheable) {
         DeviceScope scope(ctx->device);
         if (scope.ok() && (out = cached_grid(key, stream))) return INTP_OK;
     }
-    const int rc = make_grid(ctx, desc, stream, false, out);
+    const int rc = make_grid(ctx, desc, stream, false, refined, out);
     if (rc == INTP_OK && cacheable) remember_grid(key, out);
     return rc;
 }
@@ -637,15 +653,6 @@ int64_t two_pass_scratch(int64_t npts) {
            256;
 }
 
-// The uniform fast path needs every dimension uniform (knots in closed
-// form, basis polynomial classes uploaded) and 32-bit table offsets.
-bool uniform_path(const GridData& g) {
-    if (g.total >= (int64_t{1} << 32)) return false;
-    for (int d = 0; d < g.dim; ++d)
-        if (!g.setup[d].uniform || g.poly[d] == nullptr) return false;
-    return true;
-}
-
 }  // namespace
 
 // ---- the fixed scratch buffer of intp_eval_static ------------------------
@@ -720,7 +727,7 @@ int intp_ctx_destroy(intp_ctx ctx) {
 int intp_template_create(intp_ctx ctx, const intp_grid_desc* desc, intp_template* out) {
     if (!out) return fail(INTP_E_INVALID, "null output handle");
     std::shared_ptr<GridData> g;
-    const int rc = make_grid(ctx, desc, nullptr, true, g);
+    const int rc = make_grid(ctx, desc, nullptr, true, true, g);
     if (rc != INTP_OK) return rc;
     *out = new intp_template_s{std::move(g)};
     return INTP_OK;
@@ -816,7 +823,7 @@ int intp_build_refined(intp_ctx ctx, const intp_grid_desc* desc, const double* v
                        int32_t sweeps, intp_spline* out, void* stream) {
     if (!out) return fail(INTP_E_INVALID, "null output handle");
     intp_template_s t;
-    const int rc = build_grid(ctx, desc, static_cast<hipStream_t>(stream), t.grid);
+    const int rc = build_grid(ctx, desc, true, static_cast<hipStream_t>(stream), t.grid);
     if (rc != INTP_OK) return rc;
     return intp_interpolate_refined(&t, values, values_mem, sweeps, out, stream);
 }
@@ -825,7 +832,7 @@ int intp_build(intp_ctx ctx, const intp_grid_desc* desc, const double* values, i
                void* stream) {
     if (!out) return fail(INTP_E_INVALID, "null output handle");
     intp_template_s t;
-    const int rc = build_grid(ctx, desc, static_cast<hipStream_t>(stream), t.grid);
+    const int rc = build_grid(ctx, desc, false, static_cast<hipStream_t>(stream), t.grid);
     if (rc != INTP_OK) return rc;
     return intp_interpolate(&t, values, values_mem, out, stream);
 }
@@ -1191,7 +1198,7 @@ int eval_call(intp_spline s, int64_t npts, const double* coords, int64_t cs_dim,
         p.out_packed = packed ? 1 : 0;
     }
     hipError_t e = hipSuccess;
-    const bool fast = uniform_path(g);
+    const bool fast = uniform_grid(g);
     TimedCall timed{g.device, {nullptr, nullptr, nullptr}};
     const bool timing = (flags & INTP_EVAL_TIMED) != 0;
     if (timing) {
@@ -1513,7 +1520,7 @@ int intp_proxy_create(intp_template t, intp_spline s, int64_t npts, const double
     HIP_TRY(device_alloc(reinterpret_cast<void**>(&p->dev), bytes, stream), "device allocation (proxy)");
     p->first_d = reinterpret_cast<int32_t*>(p->dev);
     p->weights_d = reinterpret_cast<double*>(p->dev + first_bytes);
-    p->uniform = uniform_path(g);
+    p->uniform = uniform_grid(g);
     ProxyParams pp{};
     for (int d = 0; d < D; ++d) pp.dim[d] = dim_params(g, d);
     pp.npts = npts;

@@ -1031,12 +1031,17 @@ int intp_batch_create(intp_ctx ctx_, int32_t count, const intp_grid_desc* descs,
             for (int d = 0; d < g.dim; ++d) {
                 const std::string err =
                     setup_dimension(g.order, g.periodic[d] != 0, g.n[d], g.xmin[d], g.xmax[d], g.coords[d],
-                                    b->setups[static_cast<size_t>(s) * kBatchDim + d]);
+                                    b->setups[static_cast<size_t>(s) * kBatchDim + d], false);
                 if (!err.empty()) {
                     errors[static_cast<size_t>(s)] = err + " (dimension " + std::to_string(d) + ")";
                     break;
                 }
             }
+            if (!errors[static_cast<size_t>(s)].empty()) continue;
+            // evaluation takes the uniform path where every dimension is
+            DimSetup* ds = &b->setups[static_cast<size_t>(s) * kBatchDim];
+            const bool uniform = std::all_of(ds, ds + g.dim, [](const DimSetup& x) { return x.uniform; });
+            for (int d = 0; d < g.dim && !uniform; ++d) fill_reciprocals(g.order, ds[d]);
         }
     };
     const int nthreads = static_cast<int>(std::max(1u, std::min(16u, std::thread::hardware_concurrency())));

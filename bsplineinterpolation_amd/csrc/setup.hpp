@@ -77,9 +77,13 @@ struct DimSetup {
     std::vector<double> poly;
 };
 
-// Returns an empty string on success, else the reason.
+// Returns an empty string on success, else the reason.  refined: with the
+// tables of refined builds (colloc, the FP32 factors and their plan).
 std::string setup_dimension(int order, bool periodic, int64_t n, double xmin, double xmax,
-                            const double* nodes, DimSetup& out);
+                            const double* nodes, DimSetup& out, bool refined = true);
+// Fills `recip`, which evaluation reads on grids outside the uniform path
+// (a non-uniform dimension, or 2^32 control points and more).
+void fill_reciprocals(int order, DimSetup& s);
 // Whether the two-operation division above is exact for divisor d, and its
 // zh and zl (also for tests).
 bool known_divisor(double d, double* zh, double* zl);
