@@ -333,7 +333,17 @@ __device__ __forceinline__ int uniform_weights(const DimParams& dp, double x, in
 // One stencil row along the last dimension.  LASTC: the last dimension is
 // not periodic, so the row is K+1 consecutive elements from one address
 // (one address computation, immediate offsets).
-template <int K, bool LASTC, typename T, typename Off, typename W>
+// FAR: the table is read through the caches, not from LDS, and the loads of
+// one row stay together in the instruction stream.  A wave's load of one
+// 16-byte piece of its rows touches 64 lines, a quarter of the 32 KB L1, so
+// a row whose pieces are issued apart fetches its lines from L2 again for
+// each of them.  Together, every row costs its lines once: 1M random points
+// on 100^3, order 5, value: 1.00e8 -> 4.97e7 L2 reads (36 rows of 48 bytes
+// touch 1.37 lines each: 4.9e7), 576 -> 405 us; gradient cells 1.46e8 ->
+// 5.9e7, 1024 -> 731 us; order 4, FP64, all partials 377 -> 284 us; 2D
+// 1021 x 769, order 5, 3M points, all partials 236 -> 196 us.  The rest is
+// L2 misses: half the lines of an 8 MB table (4 MB of L2 per XCD).
+template <int K, bool LASTC, bool FAR, typename T, typename Off, typename W>
 __device__ __forceinline__ void load_row(const T* __restrict__ c, Off rowoff, const DimW<K, Off, W>& dl,
                                          T (&cv)[K + 1]) {
     if constexpr (LASTC) {
@@ -345,6 +355,7 @@ __device__ __forceinline__ void load_row(const T* __restrict__ c, Off rowoff, co
 #pragma unroll
         for (int e = 0; e <= K; ++e) cv[e] = r[dl.off[e]];
     }
+    if constexpr (FAR) __builtin_amdgcn_sched_barrier(0);
 }
 
 // Shifts the weights/offsets of the first dimension down by one, so a
@@ -366,7 +377,7 @@ __device__ __forceinline__ void shift_down(DimW<K, Off, W>& d) {
 // dimension.  The weights are indexed at run time, so these kernels keep
 // them in scratch memory.  GRAD: res = value and the D first partials
 // (dw along one dimension, w along the others); otherwise res[0] only.
-template <int D, int K, bool GRAD, bool LASTC, typename T, typename Off>
+template <int D, int K, bool GRAD, bool LASTC, bool FAR, typename T, typename Off>
 __device__ void contract_nd(const T* __restrict__ c, DimW<K, Off, T> (&dd)[D], T (&res)[D + 1]) {
     int a[D - 1];
 #pragma unroll
@@ -382,7 +393,7 @@ __device__ void contract_nd(const T* __restrict__ c, DimW<K, Off, T> (&dd)[D], T
             wv *= dd[d].w[a[d]];
         }
         T cv[K + 1];
-        load_row<K, LASTC, T>(c, rowoff, dd[D - 1], cv);
+        load_row<K, LASTC, FAR, T>(c, rowoff, dd[D - 1], cv);
         T sB = T(0), sD = T(0);
 #pragma unroll
         for (int e = 0; e <= K; ++e) {
@@ -409,11 +420,11 @@ __device__ void contract_nd(const T* __restrict__ c, DimW<K, Off, T> (&dd)[D], T
     }
 }
 
-template <int D, int K, bool LASTC, typename T, typename Off>
+template <int D, int K, bool LASTC, bool FAR, typename T, typename Off>
 __device__ __forceinline__ void contract_grad(const T* __restrict__ c, DimW<K, Off, T> (&dd)[D], T (&res)[D + 1]) {
     if constexpr (D == 1) {
         T cv[K + 1];
-        load_row<K, LASTC, T>(c, Off(0), dd[0], cv);
+        load_row<K, LASTC, FAR, T>(c, Off(0), dd[0], cv);
         T v = T(0), g = T(0);
 #pragma unroll
         for (int a = 0; a <= K; ++a) {
@@ -427,7 +438,7 @@ __device__ __forceinline__ void contract_grad(const T* __restrict__ c, DimW<K, O
 #pragma unroll
         for (int a = 0; a <= K; ++a) {
             T cv[K + 1];
-            load_row<K, LASTC, T>(c, dd[0].off[a], dd[1], cv);
+            load_row<K, LASTC, FAR, T>(c, dd[0].off[a], dd[1], cv);
             T sB = T(0), sD = T(0);
 #pragma unroll
             for (int b = 0; b <= K; ++b) {
@@ -442,7 +453,7 @@ __device__ __forceinline__ void contract_grad(const T* __restrict__ c, DimW<K, O
         res[1] = g0;
         res[2] = g1;
     } else if constexpr (D >= 4) {
-        contract_nd<D, K, true, LASTC>(c, dd, res);
+        contract_nd<D, K, true, LASTC, FAR>(c, dd, res);
     } else {
         T v = T(0), g0 = T(0), g1 = T(0), g2 = T(0);
         constexpr int kOuterUnroll = K <= INTP_OUTER_UNROLL_MAX_K ? K + 1 : 1;
@@ -452,7 +463,7 @@ __device__ __forceinline__ void contract_grad(const T* __restrict__ c, DimW<K, O
 #pragma unroll
             for (int b = 0; b <= K; ++b) {
                 T cv[K + 1];
-                load_row<K, LASTC, T>(c, dd[0].off[0] + dd[1].off[b], dd[2], cv);
+                load_row<K, LASTC, FAR, T>(c, dd[0].off[0] + dd[1].off[b], dd[2], cv);
                 T sB = T(0), sD = T(0);
 #pragma unroll
                 for (int e = 0; e <= K; ++e) {
@@ -476,19 +487,19 @@ __device__ __forceinline__ void contract_grad(const T* __restrict__ c, DimW<K, O
     }
 }
 
-template <int D, int K, bool LASTC, typename T, typename Off>
+template <int D, int K, bool LASTC, bool FAR, typename T, typename Off>
 __device__ __forceinline__ T contract_single(const T* __restrict__ c, DimW<K, Off, T> (&dd)[D]) {
     T v = T(0);
     if constexpr (D == 1) {
         T cv[K + 1];
-        load_row<K, LASTC, T>(c, Off(0), dd[0], cv);
+        load_row<K, LASTC, FAR, T>(c, Off(0), dd[0], cv);
 #pragma unroll
         for (int a = 0; a <= K; ++a) v += dd[0].w[a] * cv[a];
     } else if constexpr (D == 2) {
 #pragma unroll
         for (int a = 0; a <= K; ++a) {
             T cv[K + 1];
-            load_row<K, LASTC, T>(c, dd[0].off[a], dd[1], cv);
+            load_row<K, LASTC, FAR, T>(c, dd[0].off[a], dd[1], cv);
             T sum = T(0);
 #pragma unroll
             for (int b = 0; b <= K; ++b) sum += dd[1].w[b] * cv[b];
@@ -496,7 +507,7 @@ __device__ __forceinline__ T contract_single(const T* __restrict__ c, DimW<K, Of
         }
     } else if constexpr (D >= 4) {
         T res[D + 1];
-        contract_nd<D, K, false, LASTC>(c, dd, res);
+        contract_nd<D, K, false, LASTC, FAR>(c, dd, res);
         v = res[0];
     } else {
         constexpr int kOuterUnroll = K <= INTP_OUTER_UNROLL_MAX_K ? K + 1 : 1;
@@ -506,7 +517,7 @@ __device__ __forceinline__ T contract_single(const T* __restrict__ c, DimW<K, Of
 #pragma unroll
             for (int b = 0; b <= K; ++b) {
                 T cv[K + 1];
-                load_row<K, LASTC, T>(c, dd[0].off[0] + dd[1].off[b], dd[2], cv);
+                load_row<K, LASTC, FAR, T>(c, dd[0].off[0] + dd[1].off[b], dd[2], cv);
                 T sum = T(0);
 #pragma unroll
                 for (int e = 0; e <= K; ++e) sum += dd[2].w[e] * cv[e];
@@ -523,12 +534,12 @@ __device__ __forceinline__ T contract_single(const T* __restrict__ c, DimW<K, Of
 // the value contracts c with the value weights w, partial d contracts e_d
 // with the difference weights (dw) along d and w along the others.  Same
 // axis order as contract_grad.
-template <int D, int K, bool LASTC, typename T, typename Off>
+template <int D, int K, bool LASTC, bool FAR, typename T, typename Off>
 __device__ __forceinline__ void contract_cells(const T* __restrict__ c, DimW<K, Off, float> (&dd)[D],
                                                float (&res)[D + 1]) {
     if constexpr (D == 1) {
         T cv[K + 1];
-        load_row<K, LASTC, T>(c, Off(0), dd[0], cv);
+        load_row<K, LASTC, FAR, T>(c, Off(0), dd[0], cv);
         float v = 0.f, g = 0.f;
 #pragma unroll
         for (int a = 0; a <= K; ++a) {
@@ -542,7 +553,7 @@ __device__ __forceinline__ void contract_cells(const T* __restrict__ c, DimW<K, 
 #pragma unroll
         for (int a = 0; a <= K; ++a) {
             T cv[K + 1];
-            load_row<K, LASTC, T>(c, dd[0].off[a], dd[1], cv);
+            load_row<K, LASTC, FAR, T>(c, dd[0].off[a], dd[1], cv);
             float sC = 0.f, s0 = 0.f, s1 = 0.f;
 #pragma unroll
             for (int b = 0; b <= K; ++b) {
@@ -566,7 +577,7 @@ __device__ __forceinline__ void contract_cells(const T* __restrict__ c, DimW<K, 
 #pragma unroll
             for (int b = 0; b <= K; ++b) {
                 T cv[K + 1];
-                load_row<K, LASTC, T>(c, dd[0].off[0] + dd[1].off[b], dd[2], cv);
+                load_row<K, LASTC, FAR, T>(c, dd[0].off[0] + dd[1].off[b], dd[2], cv);
                 float sC = 0.f, s0 = 0.f, s1 = 0.f, s2 = 0.f;
 #pragma unroll
                 for (int e = 0; e <= K; ++e) {
@@ -594,13 +605,13 @@ __device__ __forceinline__ void contract_cells(const T* __restrict__ c, DimW<K, 
 }
 
 // The gradient kernels' contraction for a table of element type T.
-template <int D, int K, bool LASTC, typename T, typename Off>
+template <int D, int K, bool LASTC, bool FAR, typename T, typename Off>
 __device__ __forceinline__ void contract_outputs(const T* __restrict__ c, DimW<K, Off, weight_t<T>> (&dd)[D],
                                                  weight_t<T> (&res)[D + 1]) {
     if constexpr (is_cells<T>())
-        contract_cells<D, K, LASTC, T, Off>(c, dd, res);
+        contract_cells<D, K, LASTC, FAR, T, Off>(c, dd, res);
     else
-        contract_grad<D, K, LASTC, T, Off>(c, dd, res);
+        contract_grad<D, K, LASTC, FAR, T, Off>(c, dd, res);
 }
 
 // Stores the value and first partials of one point.
@@ -651,12 +662,12 @@ __device__ __forceinline__ void general_point(const EvalParams& p, int64_t pt) {
     }
     if constexpr (GRAD) {
         W res[D + 1];
-        contract_outputs<D, K, LASTC>(ctrl, dd, res);
+        contract_outputs<D, K, LASTC, true>(ctrl, dd, res);
 #pragma unroll
         for (int s = 0; s <= D; ++s)
             if (p.slot[s] >= 0) store_out(p, p.slot[s] * p.os_out + opt * p.os_pt, res[s]);
     } else {
-        const T v = contract_single<D, K, LASTC>(ctrl, dd);
+        const T v = contract_single<D, K, LASTC, true>(ctrl, dd);
         store_out(p, p.out_index * p.os_out + opt * p.os_pt, zero ? 0.0 : static_cast<double>(v));
     }
 }
@@ -683,10 +694,10 @@ __device__ __forceinline__ void uniform_point(const EvalParams& p, int64_t pt) {
     }
     if constexpr (GRAD) {
         W res[D + 1];
-        contract_outputs<D, K, LASTC>(ctrl, dd, res);
+        contract_outputs<D, K, LASTC, true>(ctrl, dd, res);
         store_grad<D>(p, opt, res);
     } else {
-        const T v = contract_single<D, K, LASTC>(ctrl, dd);
+        const T v = contract_single<D, K, LASTC, true>(ctrl, dd);
         store_out(p, p.out_index * p.os_out + opt * p.os_pt, zero ? 0.0 : static_cast<double>(v));
     }
 }
@@ -750,14 +761,14 @@ __device__ __forceinline__ void patch_point(const EvalParams& p, const T* s_patc
 #pragma unroll
             for (int m = 0; m <= K; ++m) dd[d].off[m] = static_cast<uint32_t>(local[d] + m) * lstride[d];
         if constexpr (GRAD)
-            contract_outputs<D, K, true>(s_patch, dd, res);
+            contract_outputs<D, K, true, false>(s_patch, dd, res);
         else
-            res[0] = contract_single<D, K, true>(s_patch, dd);
+            res[0] = contract_single<D, K, true, false>(s_patch, dd);
     } else {
         if constexpr (GRAD)
-            contract_outputs<D, K, LASTC>(ctrl, dd, res);
+            contract_outputs<D, K, LASTC, true>(ctrl, dd, res);
         else
-            res[0] = contract_single<D, K, LASTC>(ctrl, dd);
+            res[0] = contract_single<D, K, LASTC, true>(ctrl, dd);
     }
     if constexpr (GRAD) {
         store_grad<D>(p, opt, res);

@@ -73,7 +73,7 @@ __global__ __launch_bounds__(kProxyBlock) void proxy_apply_kernel(ProxyParams p)
             dd[d].dw[m] = T(0);
         }
     }
-    const T v = contract_single<D, K, LASTC>(static_cast<const T*>(p.ctrl), dd);
+    const T v = contract_single<D, K, LASTC, true>(static_cast<const T*>(p.ctrl), dd);
     if (p.out32)
         p.out32[pt * p.os_pt] = static_cast<float>(v);
     else
