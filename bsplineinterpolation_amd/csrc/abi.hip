@@ -552,25 +552,46 @@ DimParams dim_params(const GridData& g, int d) {
     return make_dim_params(g.setup[d], g.order, stride, g.knots[d], g.recip[d], g.poly[d]);
 }
 
-// Batches at least this large are grouped by brick before evaluation when
-// the table is large enough for grouping to pay (group_pays).
-constexpr int64_t kGroupMinPoints = int64_t{1} << 20;
-
-// Whether grouping pays for a batch (measured on MI355X, value + first
-// partials, cubic): 3D tables of 17 MB and more gain from 2^20 points on
-// (2^24 points: 1.4x at 128^3, 1.9x at 256^3); 2D tables up to 34 MB do
-// not (their (k+1)-row stencils stay cache-friendly: 2.5x faster
-// ungrouped at 1024^2 and 2^24 points), nor do 3D tables below 16 MB.
-// 2D tables beyond the 256 MB Infinity Cache are grouped.
-bool group_pays(int dim, int64_t table_bytes, int64_t npts) {
-    if (npts < kGroupMinPoints) return false;
-    if (dim == 3) return table_bytes >= (int64_t{16} << 20);
-    return table_bytes >= (int64_t{256} << 20);
+// Whether grouping by brick before evaluation pays.  In caller order a point
+// costs the cache lines of its stencil rows: 4.2 ps a line from L2 and 12.5
+// ps more for the share of the table beyond it.  Grouped, a call costs
+// about 85 us and 30 ps a point, each result 16 ps and each stencil element
+// of a launch 0.0125 ps a byte; 30 ps more where the patches come from
+// beyond L2, 100 us and 200 ps more where they do not fit LDS (`staged`
+// false), and the caller-order cost of the points that leave their chunk's
+// brick, about 5 a brick.  Measured on both sides of the line (us, caller order / grouped,
+// 3D, value and first partials unless said):
+//   cubic,   100^3:        400,000 points 84/110, 1M 187/155, 10M 1717/1252
+//   cubic,   48^3:         3M points 248/269, 10M 807/1037
+//   order 4, 48^3, value:  400,000 points 66/83, 1M 143/112, 10M 1269/684
+//   order 5, 100^3:        131,072 points 63/98, 400,000 185/134, 10M 3984/1429
+//   order 5, 160x140x150:  131,072 points 101/105, 400,000 300/154
+//   order 5, 100^3, refined: 131,072 points 107/112, 400,000 319/149
+//   order 5, 256^3, refined: 131,072 points 157/190, 400,000 463/334
+//   order 2, 160x140x150:  1M points 172/156, 10M 1565/1261
+//   order 1, 256^3:        1M points 100/176, 10M 915/1352
+// 2D stencils have k + 1 rows only: 2D tables gain beyond the 256 MB
+// Infinity Cache, from 2^20 points on (2^24 points on 1024^2, cubic: 0.87
+// ms in caller order, 2.15 ms grouped).
+bool group_pays(int dim, int order, int elem_bytes, int64_t elements, int64_t npts, int launches, int results,
+                bool staged, int64_t bricks) {
+    const double table = static_cast<double>(elements) * elem_bytes;
+    if (dim != 3) return npts >= (int64_t{1} << 20) && table >= 0x1p28;
+    const int row = order + 1;
+    const double lines = static_cast<double>(row) * row * (1.0 + order * elem_bytes / 128.0);
+    const double missed = table > 0x1.4p22 ? 1.0 - 0x1.4p22 / table : 0.0;  // 5 MB
+    const double n = static_cast<double>(npts);
+    const double caller_order = n * launches * lines * (4.2 + 12.5 * missed);
+    const double grouped = 85e6 + n * (30.0 + 16.0 * results + launches * 0.0125 * elem_bytes * row * row * row +
+                                       30.0 * missed) +
+                           (staged ? 0.0 : 100e6 + 200.0 * n) +
+                           caller_order * std::min(1.0, 5.0 * static_cast<double>(bricks) / n);
+    return caller_order > grouped;
 }
 
 // Bricks of B^D stencil starts, B a power of two: the largest B whose
 // (B + order)^D patch of table elements (elem_bytes each) stays within
-// kPatchBytes (the LDS patch of the grouped
+// patch_bytes() (the LDS patch of the grouped
 // evaluation kernel), coarsened until the brick key fits 16 bits (then
 // the patch no longer fits and the grouped kernel reads HBM only).
 BinParams bin_params(const GridData& g, int elem_bytes, int64_t* patch_volume) {
@@ -583,7 +604,7 @@ BinParams bin_params(const GridData& g, int elem_bytes, int64_t* patch_volume) {
         for (int d = 0; d < g.dim; ++d) v *= b + g.order;
         return v;
     };
-    while (patch(2 * B) * elem_bytes <= kPatchBytes) B *= 2;
+    while (patch(2 * B) * elem_bytes <= patch_bytes(elem_bytes, g.order)) B *= 2;
     for (;;) {
         int64_t nbin = 1;
         for (int d = 0; d < g.dim; ++d) nbin *= (g.setup[d].n + B - 1) / B;
@@ -597,7 +618,7 @@ BinParams bin_params(const GridData& g, int elem_bytes, int64_t* patch_volume) {
         bp.bricks.brick_shift[d] = shift;
         bp.bricks.nbrick[d] = static_cast<int32_t>((g.setup[d].n + B - 1) / B);
     }
-    *patch_volume = (patch(B) * elem_bytes <= kPatchBytes && B + g.order <= 64) ? patch(B) : 0;
+    *patch_volume = (patch(B) * elem_bytes <= patch_bytes(elem_bytes, g.order) && B + g.order <= 64) ? patch(B) : 0;
     return bp;
 }
 
@@ -1223,19 +1244,38 @@ int eval_call(intp_spline s, int64_t npts, const double* coords, int64_t cs_dim,
     // whose elements size the grouping's brick patches
     const bool cells = any_grad && s->cells != nullptr;
     const int elem_bytes = cells ? cell_bytes(D) : s->ctrl_bytes;
-    const bool group = (flags & INTP_EVAL_GROUPED) ? npts > 0
-                       : !(flags & INTP_EVAL_UNGROUPED) && group_pays(D, g.total * s->ctrl_bytes, npts);
+    const bool forced = (flags & INTP_EVAL_GROUPED) != 0;
+    const bool two_ok = fast && D >= 2 && D <= kGroupDim && npts <= 0xFFFFFFFFll && bin_scan_tiles(npts) <= 4096;
+    int64_t patch_volume = 0;
+    BinParams bp{};
+    if (two_ok && !(flags & INTP_EVAL_UNGROUPED)) bp = bin_params(g, elem_bytes, &patch_volume);
+    int64_t bricks = 1;
+    for (int d = 0; d < bp.dim_count; ++d) bricks *= bp.bricks.nbrick[d];
+    bool group = forced ? npts > 0
+                        : !(flags & INTP_EVAL_UNGROUPED) &&
+                              group_pays(D, g.order, elem_bytes, g.total, npts,
+                                         static_cast<int>(single.size()) + (any_grad ? 1 : 0), nout, patch_volume > 0, bricks);
+    if (group && !forced && (npts < (int64_t{1} << 20) || g.total * s->ctrl_bytes < (int64_t{16} << 20))) {
+        // a call that is being captured allocates only for large batches
+        // on large tables
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) (void)hipGetLastError();
+        group = capturing == hipStreamCaptureStatusNone;
+    }
     BrickGrid ib{};
     int64_t item_patch = 0;
     int32_t item_bins = 0;
-    // Two radix passes by default (measured faster at 256^3); one pass on
-    // request, and for a fixed scratch buffer, where it needs half the
-    // memory.
     const bool groupable = fast && D >= 2 && D <= kGroupDim && group && npts <= 0xFFFFFFFFll;
     const bool bricks_ok = groupable && item_bricks(g, elem_bytes, &ib, &item_patch, &item_bins);
-    const bool two_ok = groupable && bin_scan_tiles(npts) <= 4096;
-    bool one_pass = bricks_ok && ((flags & INTP_EVAL_GROUP_ONE_PASS) || sc.fixed() || !two_ok);
-    bool two_pass = !one_pass && two_ok;
+    // Two radix passes by default (measured faster at 256^3); one pass on
+    // request, for a fixed scratch buffer, where it needs half the memory,
+    // and where the radix bricks' patches exceed LDS and the bricks of the
+    // one pass hold enough points for its counters (order 7, value, us in
+    // two passes/one: 200x220x210, 1M points 429/568, 3M 1101/1059; 256^3,
+    // 3M 1198/1459, 10M 3614/3334).
+    bool one_pass = bricks_ok && ((flags & INTP_EVAL_GROUP_ONE_PASS) || sc.fixed() || !two_ok ||
+                                  (!forced && patch_volume == 0 && npts >= 384 * static_cast<int64_t>(item_bins)));
+    bool two_pass = !one_pass && groupable && two_ok;
     if (sc.fixed() && (one_pass || two_pass)) {
         // the grouping's scratch must fit the fixed buffer; otherwise the
         // points are evaluated in caller order (same results), unless the
@@ -1253,6 +1293,27 @@ int eval_call(intp_spline s, int64_t npts, const double* coords, int64_t cs_dim,
             }
             one_pass = two_pass = false;
         }
+    }
+    // histograms, their scan, scan tiles, then the 16-bit keys from a
+    // 16-byte boundary (the pass-1 histogram reads them 8 at a time)
+    const int64_t bin_entries = bin_hist_entries(npts), bin_tiles = (bin_scan_tiles(npts) + 3) / 4 * 4;
+    if (one_pass) {
+        e = sc.get(static_cast<size_t>(one_pass_scratch(npts, item_bins)), reinterpret_cast<void**>(&rec_a));
+    } else if (two_pass) {
+        e = sc.get(static_cast<size_t>(npts) * sizeof(BinRecord), reinterpret_cast<void**>(&rec_a));
+        if (e == hipSuccess) e = sc.get(static_cast<size_t>(npts) * sizeof(BinRecord), reinterpret_cast<void**>(&rec_b));
+        if (e == hipSuccess)
+            e = sc.get(static_cast<size_t>(2 * bin_entries + bin_tiles + (npts + 1) / 2) * 4,
+                       reinterpret_cast<void**>(&bin_scratch));
+    }
+    if (e == hipErrorOutOfMemory && !forced) {
+        // no room for the library's own choice: caller order (same results)
+        (void)hipGetLastError();
+        free_bins();
+        rec_a = rec_b = nullptr;
+        bin_scratch = nullptr;
+        one_pass = two_pass = false;
+        e = hipSuccess;
     }
     if (one_pass) {
         GroupParams gp{};
@@ -1273,7 +1334,6 @@ int eval_call(intp_spline s, int64_t npts, const double* coords, int64_t cs_dim,
         const int64_t b_rec = up(npts * static_cast<int64_t>(sizeof(BinRecord)));
         const int64_t b_hist = up(nh * 4), b_tiles = up(nt * 4);
         const int64_t b_items = up(gp.max_items * static_cast<int64_t>(sizeof(BrickItem)));
-        e = sc.get(static_cast<size_t>(one_pass_scratch(npts, item_bins)), reinterpret_cast<void**>(&rec_a));
         if (e == hipSuccess) {
             unsigned char* base = reinterpret_cast<unsigned char*>(rec_a);
             gp.rec = rec_a;
@@ -1300,22 +1360,13 @@ int eval_call(intp_spline s, int64_t npts, const double* coords, int64_t cs_dim,
         p.item_count = gp.item_count;
         p.max_items = gp.max_items;
     } else if (two_pass) {
-        int64_t patch_volume = 0;
-        BinParams bp = bin_params(g, elem_bytes, &patch_volume);
         bp.coords = p.coords;
         bp.cs_dim = p.cs_dim;
         bp.cs_pt = p.cs_pt;
         bp.npts = npts;
-        // histograms, their scan, scan tiles, then the 16-bit keys from a
-        // 16-byte boundary (the pass-1 histogram reads them 8 at a time)
-        const int64_t nh = bin_hist_entries(npts), nt = (bin_scan_tiles(npts) + 3) / 4 * 4;
-        e = sc.get(static_cast<size_t>(npts) * sizeof(BinRecord), reinterpret_cast<void**>(&rec_a));
-        if (e == hipSuccess) e = sc.get(static_cast<size_t>(npts) * sizeof(BinRecord), reinterpret_cast<void**>(&rec_b));
         if (e == hipSuccess)
-            e = sc.get(static_cast<size_t>(2 * nh + nt + (npts + 1) / 2) * 4, reinterpret_cast<void**>(&bin_scratch));
-        if (e == hipSuccess)
-            e = launch_binning(bp, bin_scratch, bin_scratch + nh, bin_scratch + 2 * nh, bin_scratch + 2 * nh + nt,
-                               rec_a, rec_b, stream);
+            e = launch_binning(bp, bin_scratch, bin_scratch + bin_entries, bin_scratch + 2 * bin_entries,
+                               bin_scratch + 2 * bin_entries + bin_tiles, rec_a, rec_b, stream);
         if (e != hipSuccess) {
             free_bins();
             cleanup();

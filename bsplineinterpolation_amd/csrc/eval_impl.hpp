@@ -724,9 +724,9 @@ __device__ __forceinline__ BinRecord load_record(const BinRecord* src) {
     return u.r;
 }
 
-template <typename T>
+template <int K, typename T>
 constexpr int patch_max() {
-    return kPatchBytes / static_cast<int>(sizeof(T));
+    return patch_bytes(sizeof(T), K) / static_cast<int>(sizeof(T));
 }
 
 // One point of a grouped chunk: if its stencil lies in the staged patch
@@ -766,9 +766,9 @@ __device__ __forceinline__ void patch_point(const EvalParams& p, const T* s_patc
             res[0] = contract_single<D, K, true, false>(s_patch, dd);
     } else {
         if constexpr (GRAD)
-            contract_outputs<D, K, LASTC, true>(ctrl, dd, res);
+            contract_outputs<D, K, LASTC, false>(ctrl, dd, res);
         else
-            res[0] = contract_single<D, K, LASTC, true>(ctrl, dd);
+            res[0] = contract_single<D, K, LASTC, false>(ctrl, dd);
     }
     if constexpr (GRAD) {
         store_grad<D>(p, opt, res);
@@ -782,7 +782,7 @@ __device__ __forceinline__ void patch_point(const EvalParams& p, const T* s_patc
 // past the end of clamped ones, where no stencil reaches), then evaluates.
 template <int D, int K, bool GRAD, bool LASTC, typename T>
 __global__ __launch_bounds__(kEvalBlock) void eval_patch_kernel(EvalParams p) {
-    constexpr int kPatchMax = patch_max<T>();
+    constexpr int kPatchMax = patch_max<K, T>();
     const T* __restrict__ ctrl = static_cast<const T*>(p.ctrl);
     __shared__ T s_patch[kPatchMax];
     const int64_t first = block_index() * kEvalBlock;
@@ -1017,7 +1017,7 @@ hipError_t launch_variant(bool grad, bool uniform, const EvalParams& p, hipStrea
     if (uniform && p.patch_volume > 0) {
         // the patch kernels read the grouping passes' records
         if constexpr (D >= 2 && D <= kGroupDim) {
-            if (p.patch_volume > patch_max<T>() || !p.perm || !p.key || p.cs_dim != 1 ||
+            if (p.patch_volume > patch_max<K, T>() || !p.perm || !p.key || p.cs_dim != 1 ||
                 p.cs_pt != static_cast<int64_t>(sizeof(BinRecord) / sizeof(double)))
                 return hipErrorInvalidValue;
             if (grad) return launch_chunks<eval_patch_kernel<D, K, true, LASTC, T>>(p, s);

@@ -37,8 +37,16 @@ struct DimParams {
 // of a point is its brick index in C order.  Brick b's stencils read only
 // control points [b*B, b*B + B - 1 + order] (B = 1 << brick_shift), wrapped
 // on periodic dimensions.
-// LDS bytes of one brick patch in the grouped evaluation kernels.
-constexpr int kPatchBytes = 24576;
+// LDS bytes of one brick patch in the grouped evaluation kernels: six
+// workgroups a CU by LDS, more than their registers allow.  Gradient cells
+// of order 4 and 5 take 36 KB (four workgroups, as many as their registers
+// allow): their 8^3 bricks need 28 and 35 KB, and 4^3 bricks are too many
+// for a 16-bit key on tables from 4.2M cells on and hold few points (value
+// and partials, order 5: 1M points on 100^3 315 -> 213 us, 10M on 256^3 3.48
+// -> 1.89 ms).
+constexpr int patch_bytes(int elem_bytes, int order) {
+    return elem_bytes == 16 && (order == 4 || order == 5) ? 36864 : 24576;
+}
 
 struct BrickGrid {
     int32_t brick_shift[kGroupDim];
