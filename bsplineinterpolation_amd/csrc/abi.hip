@@ -504,11 +504,30 @@ int refine_into(const GridData& g, const double* values, float* ctrl, void* cell
     t[1] = t[0] + ((g.total + 31) / 32) * 32;
     int64_t shift[kMaxDim];
     solve_shifts(g, shift);
+    // 2D and 3D in one pass
+    bool fused = (g.dim == 2 || g.dim == 3) && g.order >= 1;
+    for (int d = 0; d < g.dim; ++d) fused = fused && g.setup[d].n < (1 << 30);
     for (int sweep = 0; sweep < sweeps; ++sweep) {
+        if (fused) {
+            ResidualParams rp{};
+            rp.c = ctrl;
+            rp.out = delta;
+            rp.src = values;
+            rp.n[0] = 1;
+            for (int d = 0; d < g.dim; ++d) {
+                const int at = 3 - g.dim + d;
+                rp.colloc[at] = g.colloc[d];
+                rp.n[at] = static_cast<int32_t>(g.setup[d].n);
+                rp.w[at] = g.setup[d].colloc_w;
+                rp.periodic[at] = g.setup[d].periodic ? 1 : 0;
+                rp.shift[at] = static_cast<int32_t>(shift[d]);
+            }
+            HIP_TRY(launch_residual(g.dim, g.order, rp, stream), "residual launch");
+        }
         // residual, axes last to first: c -> t -> ... -> delta
         const void* in = ctrl;
         bool in_f32 = true;
-        for (int a = g.dim - 1; a >= 0; --a) {
+        for (int a = g.dim - 1; a >= 0 && !fused; --a) {
             MatvecParams mp{};
             const DimSetup& s = g.setup[a];
             mp.x = in;

@@ -376,6 +376,22 @@ inline int cell_bytes(int dim) { return dim == 1 ? static_cast<int>(sizeof(Cell1
 // gradient-table bytes per control point of a refined build (0: none)
 inline int gradient_table_bytes(int dim) { return dim <= kCellMaxDim ? cell_bytes(dim) : 0; }
 
+// The whole residual of a 2D or 3D table in one pass (residual_kernel):
+// out = (shifted src) - (M_0 x M_1 x M_2) c, rounded to FP32.  2D tables
+// are given as dimensions 1 and 2 with n[0] = 1.  Orders 1 to 7; tables below
+// 2^32 elements; not in place.
+struct ResidualParams {
+    const float* c;
+    float* out;
+    const double* src;
+    const double* colloc[3];
+    int32_t n[3], w[3], periodic[3], shift[3];
+    // set by launch_residual
+    int32_t chunk;  // planes of dimension 0 per workgroup
+    int32_t tiles1, tiles2;
+};
+hipError_t launch_residual(int dim, int order, const ResidualParams& p, hipStream_t s);
+
 struct CellParams {
     const float* c0;     // FP32 control points
     const float* delta;  // FP32 correction (c = c0 + delta in FP64), or null

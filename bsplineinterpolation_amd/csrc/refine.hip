@@ -11,6 +11,9 @@
 // for the correction in FP32 with the LU factors, and adds it to c.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "kernels.hpp"
 
 namespace intp_amd {
@@ -144,6 +147,198 @@ __global__ __launch_bounds__(kBlock) void band_matvec_rows_kernel(MatvecParams p
     }
 }
 
+// The residual of a 2D or 3D table in one pass.  A workgroup owns a tile of
+// kResRows x 64 positions of dimensions 1 and 2 and walks a chunk of
+// dimension 0 plane by plane: the plane's tile of c, with its halo, goes to
+// LDS; the products along dimension 2 (a thread's column is fixed, its matrix
+// row stays in registers) go to LDS again; those along dimension 1 run down a
+// thread's kResR rows (the matrix rows are the same for a wave: scalar
+// loads); and along dimension 0 every plane adds its term to the 2W + 1
+// results still open, held in registers.  The sums take the products in the
+// order of the kernels above, so the results are the same bits.
+// Plane p is loaded, p - 1 multiplied along dimension 2 and p - 2 along 1 and
+// 0 between two barriers, each from its own half of the buffers.
+// Against three passes over FP64 tables (0.67 GB at 256^3) this one moves
+// c, the values and the result, 0.27 GB.  256^3, order 5: 281 -> 113 us, of
+// which the FP64 products at full rate take 35 and the traffic 55; one
+// workgroup a CU (156 VGPRs) leaves the barriers and LDS waits between.
+constexpr int kResWaves = 8;
+constexpr int kResR = 4;
+constexpr int kResRows = kResWaves * kResR;
+constexpr int kResThreads = kResWaves * 64;
+
+template <int K, int D>
+__global__ __launch_bounds__(kResThreads) void residual_kernel(ResidualParams p) {
+    constexpr int W = K > 1 ? K - 1 : 0, WP = K / 2;  // clamped, periodic half-widths
+    constexpr int ROWS = kResRows + 2 * W, COLS = 64 + 2 * W, TILE = ROWS * COLS;
+    constexpr int PER = (TILE + kResThreads - 1) / kResThreads;
+    constexpr int WROWS = (ROWS + kResWaves - 1) / kResWaves;
+    typedef const __attribute__((address_space(4))) double* Uniform;
+    __shared__ float xs[2][TILE];
+    __shared__ double ys[2][ROWS * 64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = p.n[0], n1 = p.n[1], n2 = p.n[2];
+    uint32_t b = static_cast<uint32_t>(xcd_chunk_index());
+    const int t2 = static_cast<int>(b % static_cast<uint32_t>(p.tiles2));
+    b /= static_cast<uint32_t>(p.tiles2);
+    const int t1 = static_cast<int>(b % static_cast<uint32_t>(p.tiles1));
+    const int j0 = static_cast<int>(b / static_cast<uint32_t>(p.tiles1)) * p.chunk;
+    const int j1 = min(n0, j0 + p.chunk);
+    const int first1 = t1 * kResRows, first2 = t2 * 64;
+    const int row0 = first1 + wave * kResR, col = first2 + lane;
+
+    // wrapped index of a periodic dimension, or -1 outside
+    auto element = [](int i, int n, int periodic) {
+        if (periodic) i = i < 0 ? i + n : i >= n ? i - n : i;
+        return i >= 0 && i < n ? i : -1;
+    };
+    // the thread's elements of a plane's tile
+    int64_t off[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int e = threadIdx.x + q * kResThreads;
+        const int r = element(first1 - W + e / COLS, n1, p.periodic[1]);
+        const int c = element(first2 - W + e % COLS, n2, p.periodic[2]);
+        off[q] = e < TILE && r >= 0 && c >= 0 ? static_cast<int64_t>(r) * n2 + c : -1;
+    }
+    // the matrix row of the thread's column, in the middle of 2W + 1 entries
+    double m2[2 * W + 1];
+#pragma unroll
+    for (int m = -W; m <= W; ++m) {
+        const int w = p.w[2];
+        const int64_t at = static_cast<int64_t>(min(col, n2 - 1)) * (2 * w + 1) + m + w;
+        m2[m + W] = m >= -w && m <= w ? p.colloc[2][at] : 0.0;
+    }
+    // sources of the thread's results, less their plane
+    int64_t from[kResR];
+#pragma unroll
+    for (int r = 0; r < kResR; ++r) {
+        int s1 = row0 + r - p.shift[1], s2 = col - p.shift[2];
+        s1 += s1 < 0 ? n1 : 0;
+        s2 += s2 < 0 ? n2 : 0;
+        from[r] = static_cast<int64_t>(s1) * n2 + s2;
+    }
+    const int64_t plane = static_cast<int64_t>(n1) * n2;
+    const int w0 = p.w[0], w1 = p.w[1], w2 = p.w[2];
+    const int begin = j0 - w0, end = j1 + w0;  // planes (outside [0, n0): wrapped, or zeros)
+
+    float next[PER];
+    auto load = [&](int pl) {
+        const int g = pl < end ? element(pl, n0, p.periodic[0]) : -1;
+        const float* __restrict__ x = p.c + static_cast<int64_t>(max(g, 0)) * plane;
+#pragma unroll
+        for (int q = 0; q < PER; ++q) next[q] = g >= 0 && off[q] >= 0 ? x[off[q]] : 0.f;
+    };
+    auto store = [&](int pl) {
+        float* x = xs[pl & 1];
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const int e = threadIdx.x + q * kResThreads;
+            if (e < TILE) x[e] = next[q];
+        }
+    };
+    // along dimension 2, half-width w of W
+    auto along2 = [&](int pl, auto width) {
+        constexpr int w = decltype(width)::value;
+        const float* x = xs[pl & 1] + lane + (W - w);
+        double* y = ys[pl & 1] + lane;
+#pragma unroll
+        for (int q = 0; q < WROWS; ++q) {
+            const int r = q * kResWaves + wave;
+            if (r >= ROWS) break;
+            double acc = 0.0;
+#pragma unroll
+            for (int m = 0; m <= 2 * w; ++m) acc += m2[W - w + m] * static_cast<double>(x[r * COLS + m]);
+            y[r * 64] = acc;
+        }
+    };
+    double y1[kResR];
+    auto along1 = [&](int pl, auto width) {
+        constexpr int w = decltype(width)::value;
+        const double* y = ys[pl & 1] + (wave * kResR + W - w) * 64 + lane;
+        double v[kResR + 2 * w];
+#pragma unroll
+        for (int q = 0; q < kResR + 2 * w; ++q) v[q] = y[q * 64];
+#pragma unroll
+        for (int r = 0; r < kResR; ++r) {
+            const Uniform row = (Uniform)p.colloc[1] + static_cast<int64_t>(min(row0 + r, n1 - 1)) * (2 * w + 1);
+            double acc = 0.0;
+#pragma unroll
+            for (int m = 0; m <= 2 * w; ++m) acc += row[m] * v[r + m];
+            y1[r] = acc;
+        }
+    };
+    // open results along dimension 0: sum[i] belongs to plane pl - w + i
+    double sum[D == 3 ? 2 * W + 1 : 1][kResR];
+#pragma unroll
+    for (auto& s : sum)
+#pragma unroll
+        for (int r = 0; r < kResR; ++r) s[r] = 0.0;
+    auto along0 = [&](int pl, auto width) {
+        constexpr int w = decltype(width)::value;
+#pragma unroll
+        for (int i = 0; i <= 2 * w; ++i) {
+            const int j = min(max(pl - w + i, 0), n0 - 1);
+            const double m = ((Uniform)p.colloc[0])[static_cast<int64_t>(j) * (2 * w + 1) + 2 * w - i];
+#pragma unroll
+            for (int r = 0; r < kResR; ++r) sum[i][r] += m * y1[r];
+        }
+    };
+    auto emit = [&](int j, const double (&src)[kResR], const double (&v)[kResR]) {
+#pragma unroll
+        for (int r = 0; r < kResR; ++r)
+            if (row0 + r < n1 && col < n2)
+                p.out[j * plane + static_cast<int64_t>(row0 + r) * n2 + col] = static_cast<float>(src[r] - v[r]);
+    };
+
+    load(begin);
+    store(begin);
+    load(begin + 1);
+    __syncthreads();
+    for (int pl = begin; pl <= end; ++pl) {
+        // plane pl + 1 to LDS, pl along dimension 2, pl - 1 along 1 and 0
+        store(pl + 1);
+        load(pl + 2);
+        const int done = pl - 1 - w0;  // the result that plane pl - 1 completes
+        double src[kResR];
+        if (done >= j0) {
+            int s0 = done - p.shift[0];
+            s0 += s0 < 0 ? n0 : 0;
+#pragma unroll
+            for (int r = 0; r < kResR; ++r)
+                src[r] = row0 + r < n1 && col < n2 ? p.src[s0 * plane + from[r]] : 0.0;
+        }
+        if (pl < end) {
+            if (w2 == W)
+                along2(pl, std::integral_constant<int, W>{});
+            else
+                along2(pl, std::integral_constant<int, WP>{});
+        }
+        if (pl > begin) {
+            if (w1 == W)
+                along1(pl - 1, std::integral_constant<int, W>{});
+            else
+                along1(pl - 1, std::integral_constant<int, WP>{});
+            if constexpr (D == 3) {
+                if (w0 == W)
+                    along0(pl - 1, std::integral_constant<int, W>{});
+                else
+                    along0(pl - 1, std::integral_constant<int, WP>{});
+                if (done >= j0) emit(done, src, sum[0]);
+#pragma unroll
+                for (int i = 0; i < 2 * W; ++i)
+#pragma unroll
+                    for (int r = 0; r < kResR; ++r) sum[i][r] = sum[i + 1][r];
+#pragma unroll
+                for (int r = 0; r < kResR; ++r) sum[w0 == W ? 2 * W : 2 * WP][r] = 0.0;
+            } else {
+                emit(0, src, y1);
+            }
+        }
+        __syncthreads();
+    }
+}
+
 __global__ __launch_bounds__(kBlock) void add_f32_kernel(float* __restrict__ c, const float* __restrict__ d,
                                                          int64_t total) {
     const int64_t e = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
@@ -258,6 +453,45 @@ hipError_t launch_band_matvec(const MatvecParams& p_in, bool in_f32, bool out_f3
         case 6: return launch_matvec_width<6>(p, in_f32, out_f32, blocks, s);
         default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_residual(int dim, int order, const ResidualParams& p_in, hipStream_t s) {
+    ResidualParams p = p_in;
+    if (dim < 2 || dim > 3 || order < 1 || order > 7 || (dim == 2 && p.n[0] != 1)) return hipErrorInvalidValue;
+    const int w = order > 1 ? order - 1 : 0;
+    for (int d = 3 - dim; d < 3; ++d)
+        if (p.n[d] < 1 || p.w[d] != (p.periodic[d] ? order / 2 : w) || (p.periodic[d] && p.n[d] < 2 * p.w[d] + 1))
+            return hipErrorInvalidValue;
+    p.tiles1 = (p.n[1] + kResRows - 1) / kResRows;
+    p.tiles2 = (p.n[2] + 63) / 64;
+    // chunks along dimension 0: as many workgroups as the 256 CUs hold (two
+    // each up to order 4, by registers), if that leaves the chunks longer
+    // than the 2 w planes each multiplies again
+    const int64_t tiles = static_cast<int64_t>(p.tiles1) * p.tiles2;
+    const int64_t fill = (order <= 4 ? 512 : 256) / tiles;
+    const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(fill, p.n[0] / std::max(8, 2 * p.w[0])));
+    p.chunk = static_cast<int32_t>((p.n[0] + chunks - 1) / chunks);
+    const int64_t blocks = tiles * ((p.n[0] + p.chunk - 1) / p.chunk);
+    if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
+    const dim3 grid(static_cast<unsigned>(blocks)), block(kResThreads);
+#define RESIDUAL_CASE(K)                                                          \
+    case K:                                                                       \
+        if (dim == 2)                                                             \
+            hipLaunchKernelGGL((residual_kernel<K, 2>), grid, block, 0, s, p);    \
+        else                                                                      \
+            hipLaunchKernelGGL((residual_kernel<K, 3>), grid, block, 0, s, p);    \
+        return hipGetLastError();
+    switch (order) {
+        RESIDUAL_CASE(1)
+        RESIDUAL_CASE(2)
+        RESIDUAL_CASE(3)
+        RESIDUAL_CASE(4)
+        RESIDUAL_CASE(5)
+        RESIDUAL_CASE(6)
+        RESIDUAL_CASE(7)
+        default: return hipErrorInvalidValue;
+    }
+#undef RESIDUAL_CASE
 }
 
 hipError_t launch_refined_cells(const CellParams& p_in, hipStream_t s) {
