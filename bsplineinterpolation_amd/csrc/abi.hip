@@ -483,15 +483,38 @@ int solve_into(const GridData& g, const double* values, double* ctrl, hipStream_
 // Refined-FP32 control points of `values` into `ctrl` (FP32): an FP32
 // solve, then `sweeps` rounds of an FP64 residual r = S f - (M_0 (x) ...) c
 // and an FP32 correction solve added to c; and the gradient table `cells`.
-// The last round's correction d is kept apart: the cells take their
-// differences from c + d in FP64 before c becomes c + d rounded.
-// `scratch` holds N floats and 2 N doubles (N doubles for 1D).
+// The last round's correction d is kept apart: with a gradient table the
+// rounds run on c in the scratch, and the cells' launch takes their
+// differences from c + d in FP64 and rounds c + d into `ctrl`.
+// Scratch: the correction (N floats), then c (N floats, gradient tables), then
+// two tables for the residual's passes where it does not take one
+// (refine_scratch).
+bool fused_residual(const GridData& g) {
+    bool fused = (g.dim == 2 || g.dim == 3) && g.order >= 1;
+    for (int d = 0; d < g.dim; ++d) fused = fused && g.setup[d].n < (1 << 30);
+    return fused;
+}
+
+struct RefineScratch {
+    size_t c = 0, tables = 0, bytes = 0;  // offsets, total
+};
+RefineScratch refine_scratch(const GridData& g, bool cells) {
+    RefineScratch r;
+    const size_t floats = (static_cast<size_t>(g.total) * 4 + 255) / 256 * 256;
+    r.c = floats;
+    r.tables = r.c + (cells ? floats : 0);
+    r.bytes = r.tables + (g.dim == 1 || fused_residual(g) ? 0 : 4 * floats);
+    return r;
+}
+
 int refine_into(const GridData& g, const double* values, float* ctrl, void* cells, int sweeps,
                 unsigned char* scratch, hipStream_t stream) {
-    int rc = solve_axes(g, true, values, ctrl, nullptr, stream);
+    const RefineScratch at = refine_scratch(g, cells != nullptr);
+    float* const c = cells && sweeps > 0 ? reinterpret_cast<float*>(scratch + at.c) : ctrl;
+    int rc = solve_axes(g, true, values, c, nullptr, stream);
     if (rc != INTP_OK) return rc;
     CellParams cp{};
-    cp.c0 = ctrl;
+    cp.c0 = c;
     cp.cells = cells;
     cp.dim = g.dim;
     cp.total = g.total;
@@ -500,17 +523,15 @@ int refine_into(const GridData& g, const double* values, float* ctrl, void* cell
         cp.periodic[d] = g.setup[d].periodic ? 1 : 0;
     }
     float* delta = reinterpret_cast<float*>(scratch);
-    double* t[2] = {reinterpret_cast<double*>(scratch + ((g.total * 4 + 255) / 256) * 256), nullptr};
-    t[1] = t[0] + ((g.total + 31) / 32) * 32;
+    double* t[2] = {reinterpret_cast<double*>(scratch + at.tables), nullptr};
+    t[1] = t[0] + ((g.total + 63) / 64) * 64;
     int64_t shift[kMaxDim];
     solve_shifts(g, shift);
-    // 2D and 3D in one pass
-    bool fused = (g.dim == 2 || g.dim == 3) && g.order >= 1;
-    for (int d = 0; d < g.dim; ++d) fused = fused && g.setup[d].n < (1 << 30);
+    const bool fused = fused_residual(g);
     for (int sweep = 0; sweep < sweeps; ++sweep) {
         if (fused) {
             ResidualParams rp{};
-            rp.c = ctrl;
+            rp.c = c;
             rp.out = delta;
             rp.src = values;
             rp.n[0] = 1;
@@ -525,7 +546,7 @@ int refine_into(const GridData& g, const double* values, float* ctrl, void* cell
             HIP_TRY(launch_residual(g.dim, g.order, rp, stream), "residual launch");
         }
         // residual, axes last to first: c -> t -> ... -> delta
-        const void* in = ctrl;
+        const void* in = c;
         bool in_f32 = true;
         for (int a = g.dim - 1; a >= 0 && !fused; --a) {
             MatvecParams mp{};
@@ -555,11 +576,14 @@ int refine_into(const GridData& g, const double* values, float* ctrl, void* cell
             in = mp.y;
             in_f32 = false;
         }
-        // correction: solve on delta (already shifted), added into ctrl
+        // correction: solve on delta (already shifted), added into c
         // (the last one by the cells' launch)
         const bool keep = sweep + 1 == sweeps && cells != nullptr;
-        if ((rc = solve_axes(g, true, nullptr, delta, keep ? nullptr : ctrl, stream)) != INTP_OK) return rc;
-        if (keep) cp.delta = delta;
+        if ((rc = solve_axes(g, true, nullptr, delta, keep ? nullptr : c, stream)) != INTP_OK) return rc;
+        if (keep) {
+            cp.delta = delta;
+            cp.c = ctrl;
+        }
     }
     if (cells) HIP_TRY(launch_refined_cells(cp, stream), "gradient table launch");
     return INTP_OK;
@@ -822,8 +846,7 @@ int interpolate_impl(intp_template t, const double* values, int values_mem, bool
         src = staged;
     }
     if (rc == INTP_OK && refined && sweeps > 0) {
-        const size_t bytes = ((static_cast<size_t>(g.total) * 4 + 255) / 256) * 256 +
-                             2 * ((static_cast<size_t>(g.total) + 31) / 32) * 32 * sizeof(double);
+        const size_t bytes = refine_scratch(g, s->cells != nullptr).bytes;
         e = device_alloc(reinterpret_cast<void**>(&scratch), bytes, stream);
         if (e != hipSuccess) rc = hip_fail(e, "device allocation (refinement scratch)");
     }

@@ -395,6 +395,7 @@ hipError_t launch_residual(int dim, int order, const ResidualParams& p, hipStrea
 struct CellParams {
     const float* c0;     // FP32 control points
     const float* delta;  // FP32 correction (c = c0 + delta in FP64), or null
+    float* c;            // the sums rounded once, or null (not c0: neighbours read it)
     void* cells;         // Cell1 (1D) or Cell3 (2D, 3D)
     int32_t dim;
     int64_t n[kMaxDim];
@@ -402,8 +403,7 @@ struct CellParams {
     int64_t total;
     FastDiv div_n[kMaxDim];  // set by launch_refined_cells
 };
-// cells from (c0, delta); then c0 += delta rounded once from FP64.
-// Tables below 2^32 elements.
+// Cells and c from (c0, delta).  Tables below 2^32 elements.
 hipError_t launch_refined_cells(const CellParams& p, hipStream_t s);
 // gradient kernels on a gradient table (eval_cells_d*.hip)
 hipError_t eval_cells_d1(int order, bool uniform, const EvalParams& p, hipStream_t s);

@@ -347,10 +347,14 @@ __global__ __launch_bounds__(kBlock) void add_f32_kernel(float* __restrict__ c, 
 
 // Gradient-table cells of element e: c = c0 + delta in FP64 (exact: the
 // correction is far below c0's last bit), the backward differences of
-// those sums along each dimension, each rounded once to FP32.
+// those sums along each dimension, each rounded once to FP32; and c itself.
+// Neighbouring blocks share their rows and planes, so each XCD takes a
+// contiguous range of blocks, and the cells are streamed past L2.  256^3 (0.47
+// GB moved): 147 us, and 35 for c in a pass of its own -> 108 us; 156 us
+// without the streaming stores.
 template <int D, typename C>
 __global__ __launch_bounds__(kBlock) void refined_cells_kernel(CellParams p) {
-    const uint64_t e64 = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    const uint64_t e64 = static_cast<uint64_t>(xcd_chunk_index()) * kBlock + threadIdx.x;
     if (e64 >= static_cast<uint64_t>(p.total)) return;
     const uint32_t e = static_cast<uint32_t>(e64);
     const float* __restrict__ c0 = p.c0;
@@ -382,14 +386,15 @@ __global__ __launch_bounds__(kBlock) void refined_cells_kernel(CellParams p) {
         out.e1 = diff[1];
         out.e2 = diff[2];
     }
-    static_cast<C*>(p.cells)[e] = out;
-}
-
-// c0 = c0 + delta, summed in FP64 and rounded once (the cells' c).
-__global__ __launch_bounds__(kBlock) void add_rounded_kernel(float* __restrict__ c, const float* __restrict__ d,
-                                                             int64_t total) {
-    const int64_t e = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    if (e < total) c[e] = static_cast<float>(static_cast<double>(c[e]) + static_cast<double>(d[e]));
+    if constexpr (D >= 2) {
+        // streamed past the rows and planes that the next blocks read again
+        typedef float f32x4 __attribute__((ext_vector_type(4)));
+        static_assert(sizeof(C) == sizeof(f32x4), "a cell is one 16-byte store");
+        __builtin_nontemporal_store(f32x4{out.c, out.e0, out.e1, out.e2}, static_cast<f32x4*>(p.cells) + e);
+    } else {
+        static_cast<C*>(p.cells)[e] = out;
+    }
+    if (p.c) p.c[e] = out.c;
 }
 
 constexpr int kRunRows = 8;
@@ -495,7 +500,7 @@ hipError_t launch_residual(int dim, int order, const ResidualParams& p_in, hipSt
 }
 
 hipError_t launch_refined_cells(const CellParams& p_in, hipStream_t s) {
-    if (p_in.total >= (int64_t{1} << 32) || p_in.dim < 1 || p_in.dim > kCellMaxDim) return hipErrorInvalidValue;
+    if (p_in.total >= (int64_t{1} << 32) || p_in.dim < 1 || p_in.dim > kCellMaxDim || p_in.c == p_in.c0) return hipErrorInvalidValue;
     CellParams p = p_in;
     int64_t total = 1;
     for (int d = 0; d < p.dim; ++d) {
@@ -511,10 +516,6 @@ hipError_t launch_refined_cells(const CellParams& p_in, hipStream_t s) {
         case 2: hipLaunchKernelGGL((refined_cells_kernel<2, Cell3>), grid, block, 0, s, p); break;
         default: hipLaunchKernelGGL((refined_cells_kernel<3, Cell3>), grid, block, 0, s, p); break;
     }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || !p.delta) return e;
-    // the cells read c0 around each element: update it only afterwards
-    hipLaunchKernelGGL(add_rounded_kernel, grid, block, 0, s, const_cast<float*>(p.c0), p.delta, p.total);
     return hipGetLastError();
 }
 
