@@ -632,6 +632,15 @@ bool group_pays(int dim, int order, int elem_bytes, int64_t elements, int64_t np
     return caller_order > grouped;
 }
 
+// Grouped results go to their callers' positions in random order.  Three or
+// four outputs in separate rows are that many partial lines a point; from
+// this many points on they are stored as one 32-byte record each, and
+// unpacked by a second kernel (value and partials, us, rows/records: cubic
+// 128^3, 1M points 160/162, 2M 253/246, 8M 938/834, 33M 6482/3287; 256^3, 2M
+// 465/337; order 5, 100^3, 2M 314/320, 4M 656/582).  Two outputs gain nothing
+// (cubic 128^3: 2M 214/227, 33M 3370/3176).
+constexpr int64_t kRecordMinPoints = int64_t{1} << 21;
+
 // Bricks of B^D stencil starts, B a power of two: the largest B whose
 // (B + order)^D patch of table elements (elem_bytes each) stays within
 // patch_bytes() (the LDS patch of the grouped
@@ -1428,12 +1437,34 @@ int eval_call(intp_spline s, int64_t npts, const double* coords, int64_t cs_dim,
     if (timing && e == hipSuccess) e = hipEventRecord(timed.ev[1], stream);
     const bool f32 = s->ctrl_bytes == 4;
     if (any_grad && e == hipSuccess) {
+        EvalParams pg = p;
+        int wanted = 0;
+        for (int i = 0; i <= D; ++i) wanted += p.slot[i] >= 0 ? 1 : 0;
+        const bool records = two_pass && !p.out_packed && wanted >= 3 && npts >= kRecordMinPoints;
+        if (records) {
+            // the first radix pass's records are done with
+            pg.out = reinterpret_cast<double*>(rec_a);
+            pg.out32 = nullptr;
+            pg.os_out = 1;
+            pg.os_pt = 4;
+            pg.out_packed = 1;
+        }
         if (cells) {
-            EvalParams pc = p;
-            pc.ctrl = s->cells;
-            e = launch_eval_cells(D, g.order, fast, pc, stream);
+            pg.ctrl = s->cells;
+            e = launch_eval_cells(D, g.order, fast, pg, stream);
         } else {
-            e = launch_eval_grad(D, g.order, fast, f32, p, stream);
+            e = launch_eval_grad(D, g.order, fast, f32, pg, stream);
+        }
+        if (records && e == hipSuccess) {
+            UnpackParams up{};
+            up.rec = pg.out;
+            up.out = p.out;
+            up.out32 = p.out32;
+            up.npts = npts;
+            up.os_out = p.os_out;
+            up.os_pt = p.os_pt;
+            for (int i = 0; i < 4; ++i) up.slot[i] = i <= D ? p.slot[i] : -1;
+            e = launch_unpack(up, stream);
         }
     }
     for (size_t i = 0; e == hipSuccess && i < single.size(); ++i) {

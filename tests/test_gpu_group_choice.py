@@ -71,3 +71,22 @@ def test_gpu_captured_call_keeps_to_caller_order(amd):
         torch.cuda.synchronize()
         assert torch.equal(out, want), i
         g.eval(q, GRAD[:1])
+
+
+@pytest.mark.parametrize("precision,order", [("f64", 3), ("f32_refined", 2)])
+def test_gpu_record_results_equal_caller_order(amd, precision, order):
+    """Large grouped batches store result records and unpack them: rows,
+    strided rows, a permuted choice of outputs, FP64 and FP32."""
+    import torch
+    shape, npts = (70, 61, 83), (1 << 21) + 5
+    g = _spline(amd, shape, order, [False, True, False], precision)
+    q = _points(shape, npts, 11)
+    some = [GRAD[3], GRAD[0], [1, 1, 0], GRAD[2]]
+    for orders in (GRAD, some):
+        want = g.eval(q, orders, group=False)
+        assert torch.equal(g.eval(q, orders, group=True), want)
+        wide = torch.full((len(orders), npts + 3), 7.0, dtype=torch.float64, device="cuda")
+        assert torch.equal(g.eval(q, orders, group=True, out=wide[:, :npts]), want)
+        assert bool((wide[:, npts:] == 7.0).all())
+        f32 = g.eval(q, orders, group=True, out_dtype=torch.float32)
+        assert torch.equal(f32, g.eval(q, orders, group=False, out_dtype=torch.float32))
