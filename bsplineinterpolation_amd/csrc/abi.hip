@@ -1576,9 +1576,10 @@ struct intp_proxy_s {
     bool uniform = false;  // device weights from the uniform-grid path
     std::vector<int32_t> first_h;
     std::vector<double> weights_h;
-    unsigned char* dev = nullptr;  // first (int32) then weights (double)
+    unsigned char* dev = nullptr;  // first (int32), weights (double), then the order of sorted points (uint32)
     int32_t* first_d = nullptr;
     double* weights_d = nullptr;
+    uint32_t* perm_d = nullptr;
     UseTracker uses;
     ~intp_proxy_s() {
         if (dev) release_after(grid->device, dev, uses);
@@ -1586,6 +1587,23 @@ struct intp_proxy_s {
 };
 
 namespace {
+
+// Whether a proxy sorts its points by brick: where applying it in caller
+// order would spend more than 60 us on the lines of its stencil rows
+// (group_pays counts them), about what sorting adds to its creation, so that
+// the first application already pays for it.  Creation + application, us,
+// caller order -> sorted: order 4, 97x120x83, 300,000 points 42+98 -> 97+44,
+// 2M 154+573 -> 195+240; cubic, 200^3, 300,000 points 39+111 -> 91+42; order
+// 5, 30^3, 1M points 87+185 -> 102+144.  Below the line: order 2, 100^3,
+// 300,000 points 43+42 -> 97+24.
+bool proxy_sorts(int dim, int order, int64_t elements, int64_t npts) {
+    if (dim != 3) return false;
+    const double table = static_cast<double>(elements) * 8;
+    const int row = order + 1;
+    const double lines = static_cast<double>(row) * row * (1.0 + order * 8 / 128.0);
+    const double missed = table > 0x1.4p22 ? 1.0 - 0x1.4p22 / table : 0.0;
+    return static_cast<double>(npts) * lines * (4.2 + 12.5 * missed) > 60e6;
+}
 
 // Splines on equal grids: the same tables, or equal dimension, order,
 // sizes, periodicity and knot vectors.
@@ -1639,12 +1657,34 @@ int intp_proxy_create(intp_template t, intp_spline s, int64_t npts, const double
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     DeviceScope scope(g.device);
     if (!scope.ok()) return fail(INTP_E_HIP, "cannot select device");
+    p->uniform = uniform_grid(g);
+    bool sorted = p->uniform && bin_scan_tiles(npts) <= 4096 && proxy_sorts(D, g.order, g.total, npts);
+    if (sorted) {
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) (void)hipGetLastError();
+        sorted = capturing == hipStreamCaptureStatusNone;
+    }
     const size_t first_bytes = (static_cast<size_t>(npts * D) * sizeof(int32_t) + 255) / 256 * 256;
-    const size_t bytes = first_bytes + static_cast<size_t>(npts * D * w) * sizeof(double) + 256;
-    HIP_TRY(device_alloc(reinterpret_cast<void**>(&p->dev), bytes, stream), "device allocation (proxy)");
+    const size_t weight_bytes = static_cast<size_t>(npts * D * w) * sizeof(double) + 256;
+    // the points' records, twice, and the histograms of two radix passes
+    const int64_t bin_entries = sorted ? bin_hist_entries(npts) : 0;
+    const int64_t bin_tiles = sorted ? (bin_scan_tiles(npts) + 3) / 4 * 4 : 0;
+    const size_t rec_bytes = static_cast<size_t>(npts) * sizeof(BinRecord);
+    unsigned char* sort = nullptr;
+    if (sorted &&
+        device_alloc(reinterpret_cast<void**>(&sort),
+                     2 * rec_bytes + static_cast<size_t>(2 * bin_entries + bin_tiles + (npts + 1) / 2) * 4, stream) !=
+            hipSuccess) {
+        (void)hipGetLastError();
+        sorted = false;
+    }
+    const size_t bytes = first_bytes + weight_bytes + (sorted ? static_cast<size_t>(npts) * sizeof(uint32_t) : 0);
+    hipError_t e = device_alloc(reinterpret_cast<void**>(&p->dev), bytes, stream);
+    if (e != hipSuccess && sort) (void)hipFreeAsync(sort, stream);
+    HIP_TRY(e, "device allocation (proxy)");
     p->first_d = reinterpret_cast<int32_t*>(p->dev);
     p->weights_d = reinterpret_cast<double*>(p->dev + first_bytes);
-    p->uniform = uniform_grid(g);
+    if (sorted) p->perm_d = reinterpret_cast<uint32_t*>(p->dev + first_bytes + weight_bytes);
     ProxyParams pp{};
     for (int d = 0; d < D; ++d) pp.dim[d] = dim_params(g, d);
     pp.npts = npts;
@@ -1653,14 +1693,32 @@ int intp_proxy_create(intp_template t, intp_spline s, int64_t npts, const double
     pp.cs_pt = cs_pt;
     pp.first = p->first_d;
     pp.weights = p->weights_d;
+    if (sorted) {
+        int64_t patch_volume = 0;
+        BinParams bp = bin_params(g, sizeof(double), &patch_volume);
+        bp.coords = coords;
+        bp.cs_dim = cs_dim;
+        bp.cs_pt = cs_pt;
+        bp.npts = npts;
+        BinRecord* const rec_a = reinterpret_cast<BinRecord*>(sort);
+        BinRecord* const rec_b = rec_a + npts;
+        uint32_t* const hist = reinterpret_cast<uint32_t*>(rec_b + npts);
+        e = launch_binning(bp, hist, hist + bin_entries, hist + 2 * bin_entries, hist + 2 * bin_entries + bin_tiles,
+                           rec_a, rec_b, stream);
+        pp.coords = reinterpret_cast<const double*>(rec_b);
+        pp.cs_dim = 1;
+        pp.cs_pt = sizeof(BinRecord) / sizeof(double);
+        pp.records = rec_b;
+        pp.perm = p->perm_d;
+    }
     int* dbad = nullptr;
-    hipError_t e = hipSuccess;
-    if (bounds) {
+    if (bounds && e == hipSuccess) {
         e = device_alloc(reinterpret_cast<void**>(&dbad), sizeof(int), stream);
         if (e == hipSuccess) e = hipMemsetAsync(dbad, 0, sizeof(int), stream);
         pp.bad = dbad;
     }
     if (e == hipSuccess) e = launch_proxy_create(D, g.order, p->uniform, pp, stream);
+    if (sort) (void)hipFreeAsync(sort, stream);
     if (e == hipSuccess) e = p->uses.record(stream);
     if (e == hipSuccess) e = gp->uses.record(stream);
     int bad = 0;
@@ -1697,6 +1755,7 @@ int intp_proxy_eval(intp_proxy p, intp_spline s, double* out, int64_t os_pt, uin
     pp.npts = p->npts;
     pp.first = p->first_d;
     pp.weights = p->weights_d;
+    pp.perm = p->perm_d;
     pp.ctrl = s->ctrl;
     if (flags & INTP_EVAL_OUT_F32)
         pp.out32 = reinterpret_cast<float*>(out);

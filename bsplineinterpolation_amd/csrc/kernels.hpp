@@ -131,8 +131,13 @@ struct ProxyParams {
     int64_t npts;
     const double* coords;
     int64_t cs_dim, cs_pt;
+    // one array per dimension (first) and per dimension and weight: the
+    // loads of consecutive points are consecutive
     int32_t* first;
     double* weights;
+    // sorted points: result position of each; made from `records`
+    uint32_t* perm;
+    const BinRecord* records;
     int* bad;
     const void* ctrl;
     double* out;

@@ -33,51 +33,57 @@ template <int D, int K, bool UNIFORM>
 __global__ __launch_bounds__(kProxyBlock) void proxy_create_kernel(ProxyParams p) {
     const int64_t pt = static_cast<int64_t>(blockIdx.x) * kProxyBlock + threadIdx.x;
     if (pt >= p.npts) return;
+    if (p.records) p.perm[pt] = p.records[pt].idx;
 #pragma unroll
     for (int d = 0; d < D; ++d) {
         const double x = p.coords[d * p.cs_dim + pt * p.cs_pt];
-        double* w = p.weights + (pt * D + d) * (K + 1);
+        double* w = p.weights + d * (K + 1) * p.npts + pt;
         int mu;
         if constexpr (UNIFORM) {
             DimW<K, uint32_t, double> dd;
             mu = uniform_weights<K, false, double>(p.dim[d], x, 0, p.bad, dd);
 #pragma unroll
-            for (int m = 0; m <= K; ++m) w[m] = dd.w[m];
+            for (int m = 0; m <= K; ++m) w[m * p.npts] = dd.w[m];
         } else {
             double b[K + 1];
             mu = general_span_weights<K>(p.dim[d], x, p.bad, b);
 #pragma unroll
-            for (int m = 0; m <= K; ++m) w[m] = b[m];
+            for (int m = 0; m <= K; ++m) w[m * p.npts] = b[m];
         }
-        p.first[pt * D + d] = mu - K;
+        p.first[d * p.npts + pt] = mu - K;
     }
 }
 
+// What bounds it is the gather, as in caller-order evaluation: 33 lines a
+// point at order 4, half of them from beyond L2 on a table of 8 MB.  Sorted
+// points share their lines, and each XCD's contiguous range of blocks reads
+// its own part of the table: 300,000 points on 97 x 120 x 83, order 4, 89 -> 33 us.
 template <int D, int K, bool LASTC, typename T, typename Off>
 __global__ __launch_bounds__(kProxyBlock) void proxy_apply_kernel(ProxyParams p) {
-    const int64_t pt = static_cast<int64_t>(blockIdx.x) * kProxyBlock + threadIdx.x;
+    const int64_t pt = xcd_chunk_index() * kProxyBlock + threadIdx.x;
     if (pt >= p.npts) return;
     DimW<K, Off, T> dd[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) {
         const DimParams& dp = p.dim[d];
-        const double* w = p.weights + (pt * D + d) * (K + 1);
-        const Off first = static_cast<Off>(p.first[pt * D + d]);
+        const double* w = p.weights + d * (K + 1) * p.npts + pt;
+        const Off first = static_cast<Off>(p.first[d * p.npts + pt]);
         const Off n = static_cast<Off>(dp.n), stride = static_cast<Off>(dp.stride);
 #pragma unroll
         for (int m = 0; m <= K; ++m) {
             Off id = first + static_cast<Off>(m);
             if (dp.periodic && id >= n) id -= n;
             dd[d].off[m] = id * stride;
-            dd[d].w[m] = static_cast<T>(w[m]);
+            dd[d].w[m] = static_cast<T>(w[m * p.npts]);
             dd[d].dw[m] = T(0);
         }
     }
     const T v = contract_single<D, K, LASTC, true>(static_cast<const T*>(p.ctrl), dd);
+    const int64_t at = (p.perm ? static_cast<int64_t>(p.perm[pt]) : pt) * p.os_pt;
     if (p.out32)
-        p.out32[pt * p.os_pt] = static_cast<float>(v);
+        p.out32[at] = static_cast<float>(v);
     else
-        p.out[pt * p.os_pt] = static_cast<double>(v);
+        p.out[at] = static_cast<double>(v);
 }
 
 template <void (*KF)(ProxyParams)>
