@@ -489,8 +489,13 @@ int solve_into(const GridData& g, const double* values, double* ctrl, hipStream_
 // Scratch: the correction (N floats), then c (N floats, gradient tables), then
 // two tables for the residual's passes where it does not take one
 // (refine_scratch).
+// One pass for 2D and 3D tables, but for small 3D ones of order 4 and more,
+// where its planes one after another take longer than short launches (builds,
+// us, one pass per dimension/one pass: order 5, 12^3 71/81, 100^3 158/159,
+// 200^3 428/380; order 4, 27x141x64 111/114, 150^3 241/224; cubic, 64^3
+// 103/100, 100^3 144/136; 2D 200^2 84/76, 1400x1300 order 5 177/163).
 bool fused_residual(const GridData& g) {
-    bool fused = (g.dim == 2 || g.dim == 3) && g.order >= 1;
+    bool fused = (g.dim == 2 || (g.dim == 3 && (g.order <= 3 || g.total >= (int64_t{1} << 21)))) && g.order >= 1;
     for (int d = 0; d < g.dim; ++d) fused = fused && g.setup[d].n < (1 << 30);
     return fused;
 }
@@ -1296,16 +1301,18 @@ int eval_call(intp_spline s, int64_t npts, const double* coords, int64_t cs_dim,
     const bool cells = any_grad && s->cells != nullptr;
     const int elem_bytes = cells ? cell_bytes(D) : s->ctrl_bytes;
     const bool forced = (flags & INTP_EVAL_GROUPED) != 0;
-    const bool two_ok = fast && D >= 2 && D <= kGroupDim && npts <= 0xFFFFFFFFll && bin_scan_tiles(npts) <= 4096;
+    const int launches = static_cast<int>(single.size()) + (any_grad ? 1 : 0);
+    // (at 2.1 ns a point, the most it can cost, fewer do not pay)
+    bool group = !(flags & INTP_EVAL_UNGROUPED) && (forced ? npts > 0 : npts * launches >= 32768 && fast && D >= 2 && D <= kGroupDim);
+    const bool two_ok = group && fast && D >= 2 && D <= kGroupDim && npts <= 0xFFFFFFFFll && bin_scan_tiles(npts) <= 4096;
     int64_t patch_volume = 0;
     BinParams bp{};
-    if (two_ok && !(flags & INTP_EVAL_UNGROUPED)) bp = bin_params(g, elem_bytes, &patch_volume);
-    int64_t bricks = 1;
-    for (int d = 0; d < bp.dim_count; ++d) bricks *= bp.bricks.nbrick[d];
-    bool group = forced ? npts > 0
-                        : !(flags & INTP_EVAL_UNGROUPED) &&
-                              group_pays(D, g.order, elem_bytes, g.total, npts,
-                                         static_cast<int>(single.size()) + (any_grad ? 1 : 0), nout, patch_volume > 0, bricks);
+    if (two_ok) bp = bin_params(g, elem_bytes, &patch_volume);
+    if (group && !forced) {
+        int64_t bricks = 1;
+        for (int d = 0; d < bp.dim_count; ++d) bricks *= bp.bricks.nbrick[d];
+        group = group_pays(D, g.order, elem_bytes, g.total, npts, launches, nout, patch_volume > 0, bricks);
+    }
     if (group && !forced && (npts < (int64_t{1} << 20) || g.total * s->ctrl_bytes < (int64_t{16} << 20))) {
         // a call that is being captured allocates only for large batches
         // on large tables

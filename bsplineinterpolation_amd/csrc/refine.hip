@@ -470,11 +470,13 @@ hipError_t launch_residual(int dim, int order, const ResidualParams& p_in, hipSt
     p.tiles1 = (p.n[1] + kResRows - 1) / kResRows;
     p.tiles2 = (p.n[2] + 63) / 64;
     // chunks along dimension 0: as many workgroups as the 256 CUs hold (two
-    // each up to order 4, by registers), if that leaves the chunks longer
-    // than the 2 w planes each multiplies again
+    // each up to order 4, by registers), down to three planes a chunk: each
+    // multiplies 2 w planes again, but a small table leaves CUs idle (builds,
+    // at least 8 planes -> 3: 32^3, order 5, 108 -> 97 us; 100^3, order 5, 172
+    // -> 159 us; cubic 145 -> 136 us)
     const int64_t tiles = static_cast<int64_t>(p.tiles1) * p.tiles2;
     const int64_t fill = (order <= 4 ? 512 : 256) / tiles;
-    const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(fill, p.n[0] / std::max(8, 2 * p.w[0])));
+    const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(fill, p.n[0] / 3));
     p.chunk = static_cast<int32_t>((p.n[0] + chunks - 1) / chunks);
     const int64_t blocks = tiles * ((p.n[0] + p.chunk - 1) / p.chunk);
     if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;

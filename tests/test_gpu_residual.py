@@ -44,3 +44,15 @@ def test_gpu_residual_tiles(amd, shape, order, periodic):
     got = amd.InterpolationFunction(order, f, precision="f32_refined", sweeps=3, **kw).control_points()
     bound = 2.0 ** -24 * np.abs(want) + 1e-4 * 2.0 ** -22 * np.abs(want).max()
     assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) - bound)
+
+
+@pytest.mark.parametrize("shape,order", [((128, 128, 128), 4), ((64, 200, 165), 6), ((130, 130, 130), 7)])
+def test_gpu_residual_large_orders(amd, shape, order):
+    """Orders 4 and up take the one pass from 2^21 control points on."""
+    rng = np.random.default_rng(order)
+    f = rng.standard_normal(shape)
+    kw = dict(periodic=[order == 6, False, True], ranges=[(0.0, 1.0)] * 3)
+    want = amd.InterpolationFunction(order, f, **kw).control_points()
+    got = amd.InterpolationFunction(order, f, precision="f32_refined", sweeps=3, **kw).control_points()
+    bound = 2.0 ** -24 * np.abs(want) + 1e-4 * 2.0 ** -22 * np.abs(want).max()
+    assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) - bound)
