@@ -1447,7 +1447,8 @@ int eval_call(intp_spline s, int64_t npts, const double* coords, int64_t cs_dim,
         EvalParams pg = p;
         int wanted = 0;
         for (int i = 0; i <= D; ++i) wanted += p.slot[i] >= 0 ? 1 : 0;
-        const bool records = two_pass && !p.out_packed && wanted >= 3 && npts >= kRecordMinPoints;
+        // (FP32 results stored as records are one line a point already)
+        const bool records = two_pass && !p.out_packed && wanted >= 3 && npts >= kRecordMinPoints && p.os_out >= 32;
         if (records) {
             // the first radix pass's records are done with
             pg.out = reinterpret_cast<double*>(rec_a);
