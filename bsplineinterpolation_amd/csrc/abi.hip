@@ -480,16 +480,8 @@ int solve_into(const GridData& g, const double* values, double* ctrl, hipStream_
     return solve_axes(g, false, values, ctrl, nullptr, stream);
 }
 
-// Refined-FP32 control points of `values` into `ctrl` (FP32): an FP32
-// solve, then `sweeps` rounds of an FP64 residual r = S f - (M_0 (x) ...) c
-// and an FP32 correction solve added to c; and the gradient table `cells`.
-// The last round's correction d is kept apart: with a gradient table the
-// rounds run on c in the scratch, and the cells' launch takes their
-// differences from c + d in FP64 and rounds c + d into `ctrl`.
-// Scratch: the correction (N floats), then c (N floats, gradient tables), then
-// two tables for the residual's passes where it does not take one
-// (refine_scratch).
-// One pass for 2D and 3D tables, but for small 3D ones of order 4 and more,
+// The residual takes one pass for 2D and 3D tables, but for small 3D ones of
+// order 4 and more,
 // where its planes one after another take longer than short launches (builds,
 // us, one pass per dimension/one pass: order 5, 12^3 71/81, 100^3 158/159,
 // 200^3 428/380; order 4, 27x141x64 111/114, 150^3 241/224; cubic, 64^3
@@ -512,6 +504,15 @@ RefineScratch refine_scratch(const GridData& g, bool cells) {
     return r;
 }
 
+// Refined-FP32 control points of `values` into `ctrl` (FP32): an FP32
+// solve, then `sweeps` rounds of an FP64 residual r = S f - (M_0 (x) ...) c
+// and an FP32 correction solve added to c; and the gradient table `cells`.
+// The last round's correction d is kept apart: with a gradient table the
+// rounds run on c in the scratch, and the cells' launch takes their
+// differences from c + d in FP64 and rounds c + d into `ctrl`.
+// Scratch: the correction (N floats), then c (N floats, gradient tables), then
+// two tables for the residual's passes where it does not take one
+// (refine_scratch).
 int refine_into(const GridData& g, const double* values, float* ctrl, void* cells, int sweeps,
                 unsigned char* scratch, hipStream_t stream) {
     const RefineScratch at = refine_scratch(g, cells != nullptr);

@@ -5,10 +5,11 @@
 // where M_d is dimension d's collocation matrix (the unfactored matrix the
 // reference factors, InterpolationTemplate.hpp:254-446) and S f the values
 // with the periodic index shift (InterpolationTemplate.hpp:452-462).  A
-// refinement sweep forms r = S f - (M_0 (x) ... ) c in FP64, one axis at a
-// time (band mat-vec along an axis: the FP64 counterpart of the
-// reference's BandMatrix product, BandMatrix.hpp:68-77, 148-172), solves
-// for the correction in FP32 with the LU factors, and adds it to c.
+// refinement sweep forms r = S f - (M_0 (x) ... ) c in FP64 (band mat-vecs
+// along the axes: the FP64 counterpart of the reference's BandMatrix
+// product, BandMatrix.hpp:68-77, 148-172; all axes in one pass where that is
+// faster, otherwise one axis at a time), solves for the correction in FP32
+// with the LU factors, and adds it to c.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
