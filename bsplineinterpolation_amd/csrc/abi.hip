@@ -1293,9 +1293,7 @@ int eval_call(intp_spline s, int64_t npts, const double* coords, int64_t cs_dim,
     BinRecord* rec_b = nullptr;
     uint32_t* bin_scratch = nullptr;
     auto free_bins = [&]() {
-        sc.put(rec_a);
-        sc.put(rec_b);
-        sc.put(bin_scratch);
+        sc.put(rec_a);  // the whole block
     };
     // refined builds: value and first partials come from the gradient table,
     // whose elements size the grouping's brick patches
@@ -1359,11 +1357,21 @@ int eval_call(intp_spline s, int64_t npts, const double* coords, int64_t cs_dim,
     if (one_pass) {
         e = sc.get(static_cast<size_t>(one_pass_scratch(npts, item_bins)), reinterpret_cast<void**>(&rec_a));
     } else if (two_pass) {
-        e = sc.get(static_cast<size_t>(npts) * sizeof(BinRecord), reinterpret_cast<void**>(&rec_a));
-        if (e == hipSuccess) e = sc.get(static_cast<size_t>(npts) * sizeof(BinRecord), reinterpret_cast<void**>(&rec_b));
-        if (e == hipSuccess)
-            e = sc.get(static_cast<size_t>(2 * bin_entries + bin_tiles + (npts + 1) / 2) * 4,
-                       reinterpret_cast<void**>(&bin_scratch));
+        // one block for both record arrays and the rest, of few sizes: a pool
+        // block that is freed serves the next call of about the same size
+        size_t bytes = static_cast<size_t>(two_pass_scratch(npts));
+        if (!sc.fixed()) {
+            size_t step = 4096;
+            while (step * 8 < bytes) step *= 2;
+            bytes = (bytes + step - 1) / step * step;
+        }
+        e = sc.get(bytes, reinterpret_cast<void**>(&rec_a));
+        if (e == hipSuccess) {
+            unsigned char* const base = reinterpret_cast<unsigned char*>(rec_a);
+            const size_t records = (static_cast<size_t>(npts) * sizeof(BinRecord) + 255) / 256 * 256;
+            rec_b = reinterpret_cast<BinRecord*>(base + records);
+            bin_scratch = reinterpret_cast<uint32_t*>(base + 2 * records);
+        }
     }
     if (e == hipErrorOutOfMemory && !forced) {
         // no room for the library's own choice: caller order (same results)
