@@ -443,14 +443,14 @@ __global__ __launch_bounds__(NT, 2) void batch_solve_kernel(const BatchSpline* s
 
 constexpr int kEvalStreams = 4;
 
-// LDS budget of one solve workgroup (two per CU).
-constexpr int64_t kBatchTileBudget = 80 * 1024 - 2 * kMaxTileLines * 8 - kEdgeMax * 8;
+// LDS budget of the tile of one solve workgroup (two per CU).
+constexpr int64_t kBatchTileBudget = kTileLdsBudget - kTileStaticLds - kEdgeMax * 8;
 
 int64_t tile_fit(int64_t n, int64_t inner, int cap) {
     int lpb = kMaxTileLines;
     while (lpb > 0 && (lpb > cap || tile_elements(n, lpb, inner) * 8 > kBatchTileBudget)) lpb /= 2;
     // one line may take most of a CU's LDS
-    if (lpb == 0 && tile_elements(n, 1, inner) * 8 <= kBatchTileBudget + 80 * 1024) lpb = 1;
+    if (lpb == 0 && tile_elements(n, 1, inner) * 8 <= kBatchTileBudget + kLdsBytes - kTileLdsBudget) lpb = 1;
     return lpb;
 }
 

@@ -10,10 +10,6 @@ namespace intp_amd {
 
 namespace {
 
-constexpr int kMaxTileThreads = 512;
-// LDS of a tiled workgroup: two workgroups per CU on gfx950 (160 KB).
-constexpr int64_t kTileLdsBudget = 80 * 1024;
-
 template <int BW, bool CYC, typename T, typename C, int B>
 __global__ __launch_bounds__(kSolveBlock) void solve_kernel(SolveParams sp) {
     const int64_t line = static_cast<int64_t>(blockIdx.x) * kSolveBlock + threadIdx.x;
@@ -47,9 +43,10 @@ hipError_t launch_lines(const SolveParams& p, int threads, hipStream_t s) {
         const int lpb = p.lines_per_block;
         const int64_t blocks = (p.nlines + lpb - 1) / lpb;
         if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
-        const size_t lds = static_cast<size_t>(tile_elements(p.n, lpb, p.inner) + edge_elements(p.n, BW, p)) * sizeof(C);
+        const int64_t lds = tile_lds(p, BW, sizeof(C));
+        if (lds + kTileStaticLds > kLdsBytes) return hipErrorInvalidValue;
         hipLaunchKernelGGL((solve_tile_kernel<BW, CYC, T, C>), dim3(static_cast<unsigned>(blocks)),
-                           dim3(static_cast<unsigned>(threads)), lds, s, p);
+                           dim3(static_cast<unsigned>(threads)), static_cast<size_t>(lds), s, p);
         return hipGetLastError();
     }
     const int64_t blocks = (p.nlines + kSolveBlock - 1) / kSolveBlock;
@@ -121,57 +118,11 @@ hipError_t launch_solve(int bw, bool cyclic, SolveTypes types, const SolveParams
 }
 
 TilePlan solve_tile_plan(const SolveParams& p, int bw, bool cyclic, int compute_bytes) {
-    TilePlan plan;
     int dev = 0, max_lds = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
-        return plan;
-    const int64_t n = p.n, inner = p.inner;
-    // lines long enough for rows of equal factors (and, cyclic, for the
-    // strips' prefix) to matter; shorter ones are substituted plainly
-    // (one axis, one segment against plain: n = 97, order 4 20.6 / 17.8 us;
-    // n = 150, order 3 28 / 29 us)
-    SolveParams cut = p;
-    cut.segs = (p.warm > 0 || bw == 0) && n >= kMinSegmentRows && (!cyclic || n >= 2 * p.warm) ? 1 : 0;
-    const int64_t extra = 2 * kMaxTileLines * sizeof(int64_t) + edge_elements(n, bw, cut) * compute_bytes;
-    auto fits = [&](int64_t lpb, int64_t budget) {
-        return tile_elements(n, lpb, inner) * compute_bytes + extra <= std::min<int64_t>(budget, max_lds);
-    };
-    // Segments for a tile of lpb lines: one per thread and line of 256
-    // threads, halved while that costs few rows (fewer warm-ups), and one
-    // where the warm-ups would not pay.
-    auto rows = [&](int64_t segs) { return segs == 1 ? n : p.warm + ((n + segs - 1) / segs + 7) / 8 * 8; };
-    auto segments = [&](int64_t lpb) -> int64_t {
-        int64_t segs = kTileThreads / lpb;
-        while (segs > 1 && (segs * 8 > n || rows(segs / 2) <= rows(segs) + rows(segs) / 8)) segs /= 2;
-        return segs > 1 && segs >= bw && 4 * rows(segs) <= 3 * n ? segs : 1;
-    };
-    // Lines per tile: the least estimated time over the rounds of resident
-    // workgroups.  A round copies its tiles (20 B/ns per CU; strided rows
-    // move whole 64-byte sectors) and substitutes rows(segs) rows twice at
-    // about 25 ns (60 cycles), workgroups on one CU sharing its SIMDs.
-    // Measured against every choice from 4 to 32 lines on the grids of 1 to
-    // 3 dimensions from 700 x 900 to 256^3: within 5 % of the fastest.
-    double best = 0.0;
-    for (int lpb = kTileLines; lpb >= 1; lpb /= 2) {
-        if (!fits(lpb, 2 * kTileLdsBudget)) continue;
-        if (inner >= 64 && lpb < 4) continue;  // in HBM instead
-        const int64_t tiles = (p.nlines + lpb - 1) / lpb;
-        const int64_t lds = tile_elements(n, lpb, inner) * compute_bytes + extra;
-        const int64_t resident = std::min<int64_t>(std::min<int64_t>(3, (2 * kTileLdsBudget) / lds), (tiles + 255) / 256);
-        const int64_t rounds = (tiles + 256 * resident - 1) / (256 * resident);
-        const int64_t width = inner == 1 ? lpb * compute_bytes : std::max<int64_t>(lpb * compute_bytes, 64);
-        const int64_t segs = cut.segs > 0 ? segments(lpb) : 1;
-        const double t = rounds * resident * (2.0 * width * n / 20.0 + rows(segs) * 50.0);
-        if (plan.lines == 0 || t < best) {
-            best = t;
-            plan.lines = lpb;
-            plan.segs = cut.segs > 0 ? static_cast<int>(segs) : 0;
-        }
-    }
-    if (plan.lines == 0) return plan;
-    plan.threads = plan.segs <= 1 ? kTileThreads : std::max(64, plan.segs * plan.lines);
-    return plan;
+        return TilePlan{};
+    return plan_tile(p, bw, cyclic, compute_bytes, max_lds);
 }
 
 hipError_t launch_shift_copy(const ShiftParams& p, bool dst_f32, hipStream_t s) {

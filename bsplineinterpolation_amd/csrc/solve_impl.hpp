@@ -31,17 +31,13 @@
 
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-
-#include "kernels.hpp"
+#include "solve_plan.hpp"
 
 namespace intp_amd {
 
 namespace {
 
 constexpr int kSolveBlock = 256;
-constexpr int kTileThreads = 256;
-constexpr int kMaxTileLines = 64;
 
 // Elements a lane moves per batch: their loads (values and factor
 // coefficients) are issued together, then substituted in order, then
@@ -355,23 +351,10 @@ __device__ __forceinline__ void warm_factors(const SolveParams& sp, int64_t n) {
 // all but the first ~8 * order rows and the last few) take them from
 // registers instead of memory: [flo, fhi) for the forward sweep and [blo,
 // bhi) for the backward one.
-constexpr int kSegRows = 8;  // segments and warm-ups are multiples of this
-
 __device__ __forceinline__ bool same_bits(double a, double b) {
     return __double_as_longlong(a) == __double_as_longlong(b);
 }
 __device__ __forceinline__ bool same_bits(float a, float b) { return __float_as_int(a) == __float_as_int(b); }
-
-// Factors of the rows outside [flo, fhi) and [blo, bhi), with one row of
-// each range for the rest, staged in LDS after the tile: a few rows on a
-// uniform grid.  On grids where that is more than kEdgeMax elements (the
-// non-uniform ones) nothing is staged and every row reads global memory.
-constexpr int kEdgeMax = 1024;
-
-__host__ __device__ __forceinline__ int edge_elements(int64_t n, int bw, const SolveParams& sp) {
-    const int64_t e = (sp.flo + 1 + n - sp.fhi) * bw + (sp.blo + 1 + n - sp.bhi) * (bw + 1);
-    return sp.segs > 0 && e <= kEdgeMax ? static_cast<int>(e) : 0;
-}
 
 // Row of the staged table that stands for row r, and its inverse.
 __device__ __forceinline__ int edge_row(int r, int lo, int hi) { return r < hi ? min(r, lo) : r - hi + lo + 1; }
@@ -794,21 +777,6 @@ __device__ __forceinline__ bool solve_segments(const SolveParams& sp, C* tile, i
         }
     }
     return !any_bad(bad);
-}
-
-// Row stride of a tile in elements: odd on the contiguous axis, so that
-// the coalesced runs along a line spread over the LDS banks, and for
-// kTileLines lines on any axis.
-constexpr int kTileLines = 32;
-constexpr int kTileStep = kTileLines + 1;
-__host__ __device__ __forceinline__ int64_t tile_step(int64_t lpb, int64_t inner) {
-    return inner == 1 || lpb == kTileLines ? lpb | 1 : lpb;
-}
-// Rows before and after the tile, zeroed: a segment's first or last batch
-// can read and write past the line's ends.
-constexpr int64_t kTilePad = kSegRows;
-__host__ __device__ __forceinline__ int64_t tile_elements(int64_t n, int64_t lpb, int64_t inner) {
-    return (n + 2 * kTilePad) * tile_step(lpb, inner);
 }
 
 // One workgroup: lines [first, first + lpb) staged through LDS in the

@@ -1,0 +1,69 @@
+// The host-side choices of the line solves (solve_plan.hpp): no plan may ask
+// for more LDS than a workgroup has.
+
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+
+#include "grid.hpp"
+#include "solve_plan.hpp"
+
+using namespace intp_amd;
+
+namespace {
+
+int failures = 0;
+
+void check(bool ok, const char* what, int order, int periodic, int bytes, int64_t n, int64_t inner, int64_t value) {
+    if (ok) return;
+    if (++failures <= 20)
+        std::printf("%s: order %d periodic %d bytes %d n %lld inner %lld: %lld\n", what, order, periodic, bytes,
+                    static_cast<long long>(n), static_cast<long long>(inner), static_cast<long long>(value));
+}
+
+// Solve parameters of a dimension of n points, from the setup of a shorter
+// one: on a uniform grid the rows of unequal factors at both ends stay as
+// they are.
+SolveParams stretched(const DimSetup& s, bool f32, int64_t n, int64_t inner, int64_t nlines) {
+    SolveParams p{};
+    set_segment_params(f32 ? s.lu.seg32 : s.lu.seg64, &p);
+    const int more = static_cast<int>(n - s.n);
+    if (p.fhi > p.flo + 1) p.fhi += more;
+    if (p.bhi > p.blo + 1) p.bhi += more;
+    p.n = n;
+    p.inner = inner;
+    p.nlines = nlines;
+    return p;
+}
+
+// Static LDS the kernels are built with is at most `static_lds` (read from
+// the code objects by the caller).
+void tiles(int64_t static_lds) {
+    for (int order = 1; order <= 7; ++order)
+        for (int periodic = 0; periodic < 2; ++periodic)
+            for (int f32 = 0; f32 < 2; ++f32) {
+                const int bytes = f32 ? 4 : 8;
+                DimSetup s;
+                if (!setup_dimension(order, periodic != 0, 3000, 0.0, 1.0, nullptr, s, true).empty()) std::abort();
+                const struct { int64_t inner, nlines; } lines[] = {{1, 1}, {1, 3}, {1, 70}, {3, 3}, {17, 34}, {64, 640}, {300, 300}};
+                for (const auto& l : lines)
+                    for (int64_t n = 3000; n < 42000; ++n) {
+                        const SolveParams base = stretched(s, f32 != 0, n, l.inner, l.nlines);
+                        SolveParams p = base;
+                        const TilePlan plan = plan_tile(p, s.lu.p, s.lu.cyclic, bytes, kLdsBytes);
+                        if (plan.lines == 0) continue;
+                        p.lines_per_block = plan.lines;
+                        p.segs = plan.segs;
+                        const int64_t lds = (tile_lds(p, s.lu.p, bytes) + 15) / 16 * 16 + static_lds;
+                        check(lds <= kLdsBytes, "tile LDS", order, periodic, bytes, n, l.inner, lds);
+                    }
+            }
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    tiles(argc > 1 ? std::atoll(argv[1]) : kTileStaticLds);
+    if (failures) std::printf("%d failures\n", failures);
+    return failures ? 1 : 0;
+}
