@@ -31,11 +31,6 @@ namespace intp_amd {
 
 namespace {
 
-// Rows of a chunk and threads of its workgroup, for lines side by side
-// (lpb 1: contiguous lines).
-constexpr int kLongThreads = 128;
-constexpr int kStridedLen = 32;
-
 template <typename C>
 struct LongParams {
     SolveParams sp;
@@ -473,23 +468,6 @@ __global__ __launch_bounds__(64) void long_join_backward_kernel(LongParams<C> p)
     }
 }
 
-struct LongShape {
-    int lpb, threads, segs, len, rows, chunks;
-};
-
-LongShape long_shape(const SolveParams& p, int64_t H) {
-    LongShape s{};
-    s.lpb = 1;
-    if (p.inner > 1)
-        while (s.lpb < kTileLines && 2 * s.lpb <= p.inner) s.lpb *= 2;
-    s.threads = s.lpb == 1 ? kLongThreads : 256;
-    s.segs = s.threads / s.lpb;
-    s.len = s.segs <= 8 ? kStridedLen : kSegRows;
-    s.rows = s.segs * s.len;
-    s.chunks = static_cast<int>((H + s.rows - 1) / s.rows);
-    return s;
-}
-
 template <typename C>
 size_t long_state_bytes(const SolveParams& p, int bw, const LongShape& s) {
     const size_t lines = static_cast<size_t>(p.nlines);
@@ -498,7 +476,8 @@ size_t long_state_bytes(const SolveParams& p, int bw, const LongShape& s) {
 
 template <int BW, bool CYC, typename T, typename C>
 hipError_t launch_long(const SolveParams& sp, void* scratch, hipStream_t s) {
-    const LongShape shape = long_shape(sp, CYC ? sp.n - BW : sp.n);
+    const LongShape shape = plan_long(sp, BW, CYC, sizeof(C));
+    if (shape.lpb == 0) return hipErrorInvalidValue;
     LongParams<C> p{};
     p.sp = sp;
     p.sp.lines_per_block = shape.lpb;
@@ -514,12 +493,12 @@ hipError_t launch_long(const SolveParams& sp, void* scratch, hipStream_t s) {
     p.corner = p.vmax + lines * shape.chunks;
     const int64_t groups = (sp.nlines + shape.lpb - 1) / shape.lpb;
     if (groups > 65535 || sp.nlines > 0x7FFFFFFF || sp.n >= (int64_t{1} << 28)) return hipErrorInvalidValue;
-    const size_t lds = static_cast<size_t>((shape.rows + sp.warm + 2 * kTilePad) * tile_step(shape.lpb, sp.inner) +
-                                           edge_elements(sp.n, BW, p.sp)) *
-                       sizeof(C);
+    const size_t lds = static_cast<size_t>(long_lds(p.sp, BW, shape, sizeof(C)));
     const dim3 grid(static_cast<unsigned>(shape.chunks), static_cast<unsigned>(groups)), block(shape.threads);
     const dim3 lgrid(static_cast<unsigned>(sp.nlines));
     hipLaunchKernelGGL((long_forward_kernel<BW, CYC, T, C>), grid, block, lds, s, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;  // the others read what it writes
     if (BW > 0) hipLaunchKernelGGL((long_join_forward_kernel<BW, CYC, T, C>), lgrid, dim3(64), 0, s, p);
     hipLaunchKernelGGL((long_backward_kernel<BW, CYC, T, C>), grid, block, lds, s, p);
     if (BW > 0) hipLaunchKernelGGL((long_join_backward_kernel<BW, CYC, T, C>), lgrid, dim3(64), 0, s, p);
@@ -554,11 +533,10 @@ hipError_t launch_long_typed(int bw, bool cyclic, const SolveParams& p, void* sc
 constexpr int64_t kLongScratchMax = int64_t{1} << 30;
 
 size_t solve_long_scratch(const SolveParams& p, int bw, bool cyclic, int compute_bytes) {
-    const int64_t H = cyclic ? p.n - bw : p.n;
     if ((p.warm == 0 && bw > 0) || p.n >= (int64_t{1} << 28) || (cyclic && p.n < 2 * p.warm)) return 0;
-    const LongShape s = long_shape(p, H);
+    const LongShape s = plan_long(p, bw, cyclic, compute_bytes);
     // a chunk at least, and every warm-up inside the line it warms up on
-    if (s.chunks < 2 || (p.nlines + s.lpb - 1) / s.lpb > 65535) return 0;
+    if (s.lpb == 0 || s.chunks < 2 || (p.nlines + s.lpb - 1) / s.lpb > 65535) return 0;
     if (p.nlines > kLongScratchMax / compute_bytes / p.n) return 0;
     const size_t state = compute_bytes == 4 ? long_state_bytes<float>(p, bw, s) : long_state_bytes<double>(p, bw, s);
     return static_cast<size_t>(p.nlines) * static_cast<size_t>(p.n) * compute_bytes + state;

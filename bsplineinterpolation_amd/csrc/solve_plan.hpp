@@ -105,4 +105,45 @@ inline TilePlan plan_tile(const SolveParams& p, int bw, bool cyclic, int compute
     return plan;
 }
 
+// Lines too long for a tile, in chunks (solve_long.hip): lines per workgroup
+// and its threads, segments of len rows per line, rows and number of chunks.
+// lpb 0: not even one line fits.
+struct LongShape {
+    int lpb = 0, threads = 0, segs = 0, len = 0, rows = 0, chunks = 0;
+};
+
+constexpr int kLongThreads = 128;  // contiguous lines (lpb 1); 256 for lines side by side
+constexpr int kStridedLen = 32;
+// Static LDS of the chunk kernels, at most: three arrays of an entry a line
+// and a flag.
+constexpr int64_t kLongStaticLds = 3 * kMaxTileLines * 8 + 16;
+
+// Dynamic LDS of a chunk's workgroup: its rows, the warm-up before them and a
+// pad on both sides, and the staged factors.
+inline int64_t long_lds(const SolveParams& p, int bw, const LongShape& s, int compute_bytes) {
+    SolveParams cut = p;
+    cut.segs = s.segs;
+    return ((s.rows + p.warm + 2 * kTilePad) * tile_step(s.lpb, p.inner) + edge_elements(p.n, bw, cut)) * compute_bytes;
+}
+
+inline LongShape plan_long(const SolveParams& p, int bw, bool cyclic, int compute_bytes) {
+    int lpb = 1;
+    if (p.inner > 1)
+        while (lpb < kTileLines && 2 * lpb <= p.inner) lpb *= 2;
+    // fewer lines side by side where a long warm-up (352 rows on nodes graded
+    // by 5 % a cell, order 7; at most 400) leaves no room for 32
+    for (; lpb >= 1; lpb /= 2) {
+        LongShape s;
+        s.lpb = lpb;
+        s.threads = lpb == 1 ? kLongThreads : 256;
+        s.segs = s.threads / lpb;
+        s.len = s.segs <= 8 ? kStridedLen : kSegRows;
+        s.rows = s.segs * s.len;
+        const int64_t H = cyclic ? p.n - bw : p.n;
+        s.chunks = static_cast<int>((H + s.rows - 1) / s.rows);
+        if (long_lds(p, bw, s, compute_bytes) + kLongStaticLds <= kLdsBytes) return s;
+    }
+    return LongShape{};
+}
+
 }  // namespace intp_amd

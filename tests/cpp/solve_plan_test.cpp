@@ -1,6 +1,7 @@
 // The host-side choices of the line solves (solve_plan.hpp): no plan may ask
 // for more LDS than a workgroup has.
 
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <vector>
@@ -60,10 +61,40 @@ void tiles(int64_t static_lds) {
             }
 }
 
+// Lines too long for a tile: every warm-up that segment_plan can give (at
+// most 400 rows), and nodes whose factors fade slowly.
+void chunks(int64_t static_lds) {
+    for (int bw = 0; bw <= 6; ++bw)
+        for (int cyclic = 0; cyclic < 2; ++cyclic)
+            for (int bytes : {4, 8})
+                for (int64_t inner : {1, 2, 3, 15, 16, 31, 32, 63, 64, 70, 1000})
+                    for (int warm = 0; warm <= 400; warm += 8)
+                        for (int edge = 1; edge < 200; edge += 11) {
+                            SolveParams p{};
+                            p.warm = warm;
+                            p.inner = inner;
+                            p.nlines = inner * 2;
+                            p.n = 30000;
+                            p.flo = p.blo = edge;
+                            p.fhi = p.bhi = 30000 - edge;
+                            const LongShape s = plan_long(p, bw, cyclic != 0, bytes);
+                            check(s.lpb > 0 && s.rows % kSegRows == 0 && s.threads == s.segs * s.lpb, "chunk shape", bw, cyclic, bytes,
+                                  warm, inner, s.lpb);
+                            const int64_t lds = (long_lds(p, bw, s, bytes) + 15) / 16 * 16 + static_lds;
+                            check(lds <= kLdsBytes, "chunk LDS", bw, cyclic, bytes, warm, inner, lds);
+                        }
+    std::vector<double> x;
+    for (int i = 0; i < 6000; ++i) x.push_back(i == 0 ? 0.0 : x.back() + std::pow(1.05, std::min(i % 400, 400 - i % 400)));
+    DimSetup s;
+    if (!setup_dimension(7, false, 6000, 0.0, 1.0, x.data(), s, true).empty()) std::abort();
+    check(s.lu.seg64.warm > 340, "warm-up of graded nodes", 7, 0, 8, 6000, 64, s.lu.seg64.warm);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     tiles(argc > 1 ? std::atoll(argv[1]) : kTileStaticLds);
+    chunks(argc > 2 ? std::atoll(argv[2]) : kLongStaticLds);
     if (failures) std::printf("%d failures\n", failures);
     return failures ? 1 : 0;
 }

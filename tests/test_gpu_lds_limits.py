@@ -53,3 +53,19 @@ def test_gpu_refined_lines_at_the_tile_limit(order, n):
     # a refined control point is the FP64 one rounded to FP32, up to an error
     # of the last correction far below an FP32 rounding of the largest value
     assert np.max(np.abs(got - want.reshape(got.shape))) <= 2.0 ** -23 * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("shape,growth,cells", [((6000, 70), 1.05, 200), ((5500, 64), 1.08, 100), ((5200, 33), 1.05, 200)])
+def test_gpu_long_lines_with_long_warm_ups(shape, growth, cells):
+    """Lines side by side, too long for a tile, on nodes whose factors fade so
+    slowly that 32 lines of a chunk and its warm-up would not fit LDS."""
+    import bsplineinterpolation_amd as amd
+    rng = np.random.default_rng(shape[0])
+    i = np.arange(shape[0])
+    steps = growth ** np.minimum(i % (2 * cells), 2 * cells - i % (2 * cells)).astype(float)
+    x = np.concatenate([[0.0], np.cumsum(steps[1:])])
+    y = np.linspace(0.0, 1.0, shape[1])
+    f = rng.standard_normal(shape)
+    want = OracleSpline(7, f, periodic=[False, False], coords=[x, y]).control_points()
+    got = amd.InterpolationFunction(7, f, coords=[x, y]).control_points()
+    assert np.array_equal(got, want.reshape(got.shape))
