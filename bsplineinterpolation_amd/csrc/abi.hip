@@ -377,6 +377,23 @@ SolveTypes axis_types(const GridData& g, bool refined, int d) {
 
 int compute_bytes(SolveTypes t) { return t == SolveTypes::kF32 ? 4 : 8; }
 
+// A block of the pool, freed on its stream at the end of the scope.
+struct StreamBlock {
+    hipStream_t stream;
+    void* p = nullptr;
+    explicit StreamBlock(hipStream_t s) : stream(s) {}
+    StreamBlock(const StreamBlock&) = delete;
+    StreamBlock& operator=(const StreamBlock&) = delete;
+    ~StreamBlock() {
+        if (p) (void)hipFreeAsync(p, stream);
+    }
+    hipError_t get(size_t bytes) {
+        const hipError_t e = device_alloc(&p, bytes, stream);
+        if (e != hipSuccess) p = nullptr;
+        return e;
+    }
+};
+
 // Line solves along every axis, last axis first (InterpolationTemplate.hpp:448-580),
 // on table x (FP64, or FP32 when `refined`).  With `values` set, the first
 // pass reads them (FP64) with the periodic shift applied; when its lines do
@@ -390,31 +407,39 @@ int solve_axes(const GridData& g, bool refined, const double* values, void* x, v
     bool any_shift = false;
     for (int d = 0; d < g.dim; ++d) any_shift = any_shift || shift[d] != 0;
     const size_t elem = refined ? sizeof(float) : sizeof(double);
-    // shape fields of axis a's line solve, and its tile
-    auto axis_params = [&](int a, SolveParams* sp) {
+    // every axis's line solve and its tile; lines too long for a tile are
+    // solved in chunks, through scratch (one block serves all axes)
+    SolveParams params[kMaxDim]{};
+    TilePlan plans[kMaxDim];
+    size_t chunk_bytes[kMaxDim] = {}, scratch_bytes = 0;
+    for (int a = 0; a < g.dim; ++a) {
         const DimSetup& s = g.setup[a];
         const SolveTypes types = axis_types(g, refined, a);
-        sp->n = s.n;
-        sp->div_n = make_fast_div(static_cast<uint32_t>(s.n));
-        sp->inner = 1;
-        for (int d = a + 1; d < g.dim; ++d) sp->inner *= g.setup[d].n;
-        sp->nlines = g.total / s.n;
-        set_segment_params(types == SolveTypes::kF32 ? s.lu.seg32 : s.lu.seg64, sp);
-        const TilePlan plan = solve_tile_plan(*sp, s.lu.p, s.lu.cyclic, compute_bytes(types));
-        sp->lines_per_block = plan.lines;
-        sp->segs = plan.segs;
-        return plan;
-    };
-    // lines too long for a tile are solved in chunks, through scratch
-    auto long_scratch = [&](int a, const SolveParams& sp) -> size_t {
-        const DimSetup& s = g.setup[a];
-        return sp.lines_per_block > 0
-                   ? 0
-                   : solve_long_scratch(sp, s.lu.p, s.lu.cyclic, compute_bytes(axis_types(g, refined, a)));
-    };
-    SolveParams last_params{};
-    const bool fused =
-        values != nullptr && (axis_params(last, &last_params).lines > 0 || long_scratch(last, last_params) > 0);
+        SolveParams& sp = params[a];
+        sp.n = s.n;
+        sp.div_n = make_fast_div(static_cast<uint32_t>(s.n));
+        sp.inner = 1;
+        for (int d = a + 1; d < g.dim; ++d) sp.inner *= g.setup[d].n;
+        sp.nlines = g.total / s.n;
+        set_segment_params(types == SolveTypes::kF32 ? s.lu.seg32 : s.lu.seg64, &sp);
+        plans[a] = solve_tile_plan(sp, s.lu.p, s.lu.cyclic, compute_bytes(types));
+        sp.lines_per_block = plans[a].lines;
+        sp.segs = plans[a].segs;
+        if (plans[a].lines == 0) chunk_bytes[a] = solve_long_scratch(sp, s.lu.p, s.lu.cyclic, compute_bytes(types));
+        scratch_bytes = std::max(scratch_bytes, chunk_bytes[a]);
+    }
+    StreamBlock scratch(stream);
+    if (scratch_bytes > 0) {
+        const hipError_t e = scratch.get(scratch_bytes);
+        if (e == hipErrorOutOfMemory) {
+            // no room: those lines are solved in place, one lane a line
+            (void)hipGetLastError();
+            std::fill(chunk_bytes, chunk_bytes + kMaxDim, size_t{0});
+        } else {
+            HIP_TRY(e, "device allocation (long lines)");
+        }
+    }
+    const bool fused = values != nullptr && (plans[last].lines > 0 || chunk_bytes[last] > 0);
     if (values != nullptr && !fused) {
         if (any_shift || refined) {
             ShiftParams sh{};
@@ -436,9 +461,8 @@ int solve_axes(const GridData& g, bool refined, const double* values, void* x, v
         const DimSetup& s = g.setup[a];
         const SolveTypes types = axis_types(g, refined, a);
         const bool f32 = types == SolveTypes::kF32;
-        SolveParams sp{};
+        SolveParams sp = params[a];
         sp.x = x;
-        const TilePlan plan = axis_params(a, &sp);
         sp.lower = f32 ? static_cast<const void*>(g.lower32[a]) : g.lower[a];
         sp.upper = f32 ? static_cast<const void*>(g.upper32[a]) : g.upper[a];
         sp.diag = f32 ? static_cast<const void*>(g.diag32[a]) : g.diag[a];
@@ -456,14 +480,10 @@ int solve_axes(const GridData& g, bool refined, const double* values, void* x, v
         const bool add_after = a == 0 && accum != nullptr && sp.lines_per_block == 0;
         if (a == 0 && accum != nullptr && !add_after) sp.accum = accum;
         hipError_t e;
-        if (const size_t bytes = long_scratch(a, sp)) {
-            void* scratch = nullptr;
-            HIP_TRY(device_alloc(&scratch, bytes, stream), "device allocation (long lines)");
-            e = launch_solve_long(s.lu.p, s.lu.cyclic, types, sp, scratch, stream);
-            (void)hipFreeAsync(scratch, stream);
-        } else {
-            e = launch_solve(s.lu.p, s.lu.cyclic, types, sp, plan.threads, stream);
-        }
+        if (chunk_bytes[a] > 0)
+            e = launch_solve_long(s.lu.p, s.lu.cyclic, types, sp, scratch.p, stream);
+        else
+            e = launch_solve(s.lu.p, s.lu.cyclic, types, sp, plans[a].threads, stream);
         if (e == hipErrorNotSupported) return fail(INTP_E_UNSUPPORTED, "band width without a compiled solver");
         HIP_TRY(e, "solve launch");
         if (add_after) {
