@@ -1703,21 +1703,30 @@ int intp_proxy_create(intp_template t, intp_spline s, int64_t npts, const double
     }
     const size_t first_bytes = (static_cast<size_t>(npts * D) * sizeof(int32_t) + 255) / 256 * 256;
     const size_t weight_bytes = static_cast<size_t>(npts * D * w) * sizeof(double) + 256;
-    // the points' records, twice, and the histograms of two radix passes
+    // the points' records, twice, and the histograms of two radix passes;
+    // where these, or the order they give, find no room, the points stay in
+    // caller order
     const int64_t bin_entries = sorted ? bin_hist_entries(npts) : 0;
     const int64_t bin_tiles = sorted ? (bin_scan_tiles(npts) + 3) / 4 * 4 : 0;
     const size_t rec_bytes = static_cast<size_t>(npts) * sizeof(BinRecord);
-    unsigned char* sort = nullptr;
-    if (sorted &&
-        device_alloc(reinterpret_cast<void**>(&sort),
-                     2 * rec_bytes + static_cast<size_t>(2 * bin_entries + bin_tiles + (npts + 1) / 2) * 4, stream) !=
-            hipSuccess) {
-        (void)hipGetLastError();
-        sorted = false;
+    StreamBlock sort(stream);
+    const size_t bytes = first_bytes + weight_bytes;
+    hipError_t e = hipErrorOutOfMemory;
+    if (sorted) {
+        e = device_alloc(reinterpret_cast<void**>(&p->dev), bytes + static_cast<size_t>(npts) * sizeof(uint32_t), stream);
+        if (e == hipSuccess &&
+            sort.get(2 * rec_bytes + static_cast<size_t>(2 * bin_entries + bin_tiles + (npts + 1) / 2) * 4) != hipSuccess)
+            sorted = false;
+        if (e != hipSuccess) {
+            p->dev = nullptr;
+            sorted = false;
+        }
+        if (!sorted) (void)hipGetLastError();
     }
-    const size_t bytes = first_bytes + weight_bytes + (sorted ? static_cast<size_t>(npts) * sizeof(uint32_t) : 0);
-    hipError_t e = device_alloc(reinterpret_cast<void**>(&p->dev), bytes, stream);
-    if (e != hipSuccess && sort) (void)hipFreeAsync(sort, stream);
+    if (!p->dev) {
+        e = device_alloc(reinterpret_cast<void**>(&p->dev), bytes, stream);
+        if (e != hipSuccess) p->dev = nullptr;
+    }
     HIP_TRY(e, "device allocation (proxy)");
     p->first_d = reinterpret_cast<int32_t*>(p->dev);
     p->weights_d = reinterpret_cast<double*>(p->dev + first_bytes);
@@ -1737,7 +1746,7 @@ int intp_proxy_create(intp_template t, intp_spline s, int64_t npts, const double
         bp.cs_dim = cs_dim;
         bp.cs_pt = cs_pt;
         bp.npts = npts;
-        BinRecord* const rec_a = reinterpret_cast<BinRecord*>(sort);
+        BinRecord* const rec_a = static_cast<BinRecord*>(sort.p);
         BinRecord* const rec_b = rec_a + npts;
         uint32_t* const hist = reinterpret_cast<uint32_t*>(rec_b + npts);
         e = launch_binning(bp, hist, hist + bin_entries, hist + 2 * bin_entries, hist + 2 * bin_entries + bin_tiles,
@@ -1755,7 +1764,6 @@ int intp_proxy_create(intp_template t, intp_spline s, int64_t npts, const double
         pp.bad = dbad;
     }
     if (e == hipSuccess) e = launch_proxy_create(D, g.order, p->uniform, pp, stream);
-    if (sort) (void)hipFreeAsync(sort, stream);
     if (e == hipSuccess) e = p->uses.record(stream);
     if (e == hipSuccess) e = gp->uses.record(stream);
     int bad = 0;

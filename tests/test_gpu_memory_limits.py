@@ -63,3 +63,35 @@ def test_gpu_long_lines_without_room_for_chunks(shim, shape, order, periodic, pr
         assert shim.alloc_refused() > 0
         assert np.array_equal(got, want)
     """ % (shape, order, periodic, precision))
+
+
+@pytest.mark.parametrize("room", ["weights", "weights and order", "all"])
+def test_gpu_proxy_without_room_to_sort(shim, room):
+    """A proxy's weights fit; what it takes to sort its points does not."""
+    _run(shim, """
+        room = %r
+        n = 1000000
+        t = amd.InterpolationFunctionTemplate(4, (60, 50, 40), ranges=[(0.0, 1.0)] * 3)
+        spline = t.interpolate(device(rng.standard_normal((60, 50, 40))))
+        pts = device(rng.random((n, 3)))
+        want = t.eval_proxy(pts)(spline).cpu().numpy()
+        weights = (n * 3 * 4 + 255) // 256 * 256 + n * 3 * 5 * 8 + 256
+        limit({"weights": weights + 1024, "weights and order": weights + 4 * n + 1024, "all": None}[room])
+        got = t.eval_proxy(pts)(spline).cpu().numpy()
+        assert (shim.alloc_refused() > 0) == (room != "all")
+        assert np.array_equal(got, want)
+    """ % room)
+
+
+def test_gpu_eval_without_room_to_group(shim):
+    """Points whose grouping scratch cannot be had stay in caller order."""
+    _run(shim, """
+        s = amd.InterpolationFunction(5, device(rng.standard_normal((100, 90, 80))), ranges=[(0.0, 1.0)] * 3)
+        pts = device(rng.random((1000000, 3)))
+        orders = [[0, 0, 0], [1, 0, 0], [0, 1, 0], [0, 0, 1]]
+        want = s.eval(pts, orders).cpu().numpy()
+        limit(4096)
+        got = s.eval(pts, orders).cpu().numpy()
+        assert shim.alloc_refused() > 0
+        assert np.array_equal(got, want)
+    """)
