@@ -336,8 +336,8 @@ __device__ __forceinline__ void warm_factors(const SolveParams& sp, int64_t n) {
 // is loaded again and solved with one segment per line.  That happens on
 // exactly constant lines (two starts can settle on neighbouring fixed
 // points: 0.7 to 16 % of the boundaries for orders 3 and 4, up to 40 % at
-// order 5), on long runs of zeros after data (a true state there is a tail
-// of the data) and on infinities and NaN.
+// order 5) and where data decays faster than the factors fade (a Gaussian's
+// flanks, zeros after data: a true state there is a tail of the data).
 //
 // The strips of a cyclic matrix are the other chain: x[n-BW+q] minus
 // bottom[q][j] * y[j] over all j.  The strip decays like the recurrence, so
@@ -345,7 +345,13 @@ __device__ __forceinline__ void warm_factors(const SolveParams& sp, int64_t n) {
 // below the rounding of the sum A.  That is checked too: with t the
 // largest remaining strip entry (strip_rest) times the largest |y|,
 // A - t == A and A + t == A make every later subtraction a no-op
-// (rounding is monotonic).
+// (rounding is monotonic).  Where they do not hold, the other rows are
+// summed too.
+//
+// Numerators too small for the two-operation division, infinities and NaN
+// are found after each batch of rows, which is then divided in full: a field
+// of 1e-290 costs 0.27 ms at 256^3 cubic, 0.25 at ordinary values (0.85 where
+// a tile that met one was solved again, twice).
 //
 // Rows whose factors repeat bit for bit (the interior of a uniform grid,
 // all but the first ~8 * order rows and the last few) take them from
@@ -516,13 +522,14 @@ __device__ __forceinline__ void seg_forward(C* line, int step, int origin, int l
 // 2004).  The host has checked every numerator whose quotient lies near
 // enough to a rounding boundary, so the result is the correctly rounded
 // quotient (zl >= 0 keeps the sign of a zero) unless v zl underflows,
-// which the caller's check of the smallest exponent finds, or v is
-// infinite, which its finite check finds.
+// which `least` finds, or v is infinite, which leaves a NaN in every later
+// row.  The caller looks for both after a batch of rows and divides that
+// batch in full.
 template <typename C>
 struct KnownDivisor {
-    C zh, zl;
-    // the smallest exponent of a numerator so far (a zero, an infinity and
-    // a NaN count as 0)
+    C zh, zl, d;
+    // least: the smallest exponent of a numerator so far (a zero, an infinity
+    // and a NaN count as 0)
     __device__ __forceinline__ C divide(C v, int& least) const {
 #pragma clang fp contract(off)
         if constexpr (sizeof(C) == 8) {
@@ -535,6 +542,13 @@ struct KnownDivisor {
     }
     __device__ __forceinline__ static bool underflows(int least) { return least < (sizeof(C) == 8 ? -900 : -90); }
 };
+
+template <typename C>
+__device__ __forceinline__ KnownDivisor<C> known_pivot(const SolveParams& sp) {
+    KnownDivisor<C> k{static_cast<C>(sp.zh), static_cast<C>(sp.zl), C(1)};
+    if (sp.fast_divide) k.d = ((GlobalPtr<C>)(sp.diag))[sp.blo];
+    return k;
+}
 
 // One batch of backward rows (row u at x - u * step, u downward from row j).
 template <int BW, bool CYC, bool STORE, typename C, int B, typename U, typename D, typename R>
@@ -566,8 +580,7 @@ __device__ __forceinline__ void seg_backward_rows(const C (&xb)[B], C* x, int st
 template <int BW, bool CYC, bool STORE, typename C, int B>
 __device__ __forceinline__ void seg_backward(C* line, int step, int origin, int n, int j0, int count, int end,
                                              bool mine, BatchRange eq, const SolveParams& sp, const EdgeTable<C>& edge,
-                                             const KnownDivisor<C>& kz, const C (&corner)[BW + 1], C (&nxt)[BW + 1],
-                                             int& least) {
+                                             const KnownDivisor<C>& kz, const C (&corner)[BW + 1], C (&nxt)[BW + 1]) {
     const GlobalPtr<C> __restrict__ upper = (GlobalPtr<C>)(sp.upper);
     const GlobalPtr<C> __restrict__ diag = (GlobalPtr<C>)(sp.diag);
     const GlobalPtr<C> __restrict__ right = (GlobalPtr<C>)(sp.right);
@@ -629,11 +642,25 @@ __device__ __forceinline__ void seg_backward(C* line, int step, int origin, int 
         };
         auto run = [&](const C (&xv)[B], const C (&rv)[B][BW + 1]) {
             const int j = j0 - t;
-            if (mine && j >= 0 && j < end)
-                seg_backward_rows<BW, CYC, STORE, C, B>(xv, line + at, step, n, j, corner, nxt,
-                                                        [&](int, int m) { return ku[m]; },
-                                                        [&](int, C v) { return kz.divide(v, least); },
-                                                        [&](int u, int c) { return rv[u][c]; });
+            if (mine && j >= 0 && j < end) {
+                auto rows = [&](auto divide) {
+                    seg_backward_rows<BW, CYC, STORE, C, B>(xv, line + at, step, n, j, corner, nxt,
+                                                            [&](int, int m) { return ku[m]; }, divide,
+                                                            [&](int u, int c) { return rv[u][c]; });
+                };
+                C before[BW + 1];
+                int least = 0;
+#pragma unroll
+                for (int m = 0; m < BW; ++m) before[m] = nxt[m];
+                auto finite = [&]() { return nxt[0] - nxt[0] == C(0); };
+                const bool fast = finite();  // (infinities and NaN stay in every row)
+                if (fast) rows([&](int, C v) { return kz.divide(v, least); });
+                if (!fast || kz.underflows(least) || !finite()) {
+#pragma unroll
+                    for (int m = 0; m < BW; ++m) nxt[m] = before[m];
+                    rows([&](int, C v) { return v / kz.d; });
+                }
+            }
             t += B;
             at -= stride;
             asm volatile("" : "+v"(at));  // one running index, not one per row
@@ -657,7 +684,7 @@ __device__ __forceinline__ void seg_backward(C* line, int step, int origin, int 
 // undefined.  Every thread of the workgroup takes part.
 template <int BW, bool CYC, typename C, int B>
 __device__ __forceinline__ bool solve_segments(const SolveParams& sp, C* tile, int step, int nl, int lpb, int segs,
-                                               const EdgeTable<C>& edge, int tid, int* failed) {
+                                               const EdgeTable<C>& edge, int tid, int (&failed)[2]) {
     const int n = static_cast<int>(sp.n);
     const int shift = __builtin_ctz(static_cast<unsigned>(lpb));
     const int line = tid & (lpb - 1), seg = tid >> shift;
@@ -676,11 +703,11 @@ __device__ __forceinline__ bool solve_segments(const SolveParams& sp, C* tile, i
     // whether any thread's `bad` is set (LDS flag, cleared below between
     // barriers)
     auto any_bad = [&](bool bad) {
-        if (__any(bad) && (threadIdx.x & 63) == 0) *failed = 1;
+        if (__any(bad) && (threadIdx.x & 63) == 0) failed[0] = 1;
         __syncthreads();
-        return *failed != 0;
+        return failed[0] != 0;
     };
-    if (tid == 0) *failed = 0;
+    if (tid < 2) failed[tid] = 0;
     // forward
     const int a = seg * len;
     C strip_row = C(0);  // x[n-BW+q] of the thread that sums strip q (the forward sweep stores past row H)
@@ -705,28 +732,35 @@ __device__ __forceinline__ bool solve_segments(const SolveParams& sp, C* tile, i
         for (int m = 0; m < BW; ++m) bad = bad || !same_bits(start[m], x[(a - 1 - m) * step]);
     }
     if constexpr (CYC && BW > 0) {
-        if (mine) bad = bad || !(hist[0] - hist[0] == C(0));  // infinities and NaN
-        if (line < nl) {
 #pragma clang fp contract(off)
-            const GlobalPtr<C> __restrict__ bottom = (GlobalPtr<C>)(sp.bottom);
-            if (seg < BW) {
-                C acc = strip_row;
-                const int last = min(warm, n - 2 * BW + seg);
+        // x[n-BW+q] minus the terms of rows a .. e - 1, by thread q of a line
+        const GlobalPtr<C> __restrict__ bottom = (GlobalPtr<C>)(sp.bottom);
+        auto strip = [&](C acc, int a, int e) {
 #pragma unroll 8
-                for (int j = 0; j < last; ++j) acc = acc - bottom[seg * n + j] * x[j * step];
-                x[(H + seg) * step] = acc;
-            }
-        }
+            for (int j = a; j < e; ++j) acc = acc - bottom[seg * n + j] * x[j * step];
+            x[(H + seg) * step] = acc;
+        };
+        const int rows = n - 2 * BW + seg, prefix = min(warm, rows);
+        if (line < nl && seg < BW) strip(strip_row, 0, prefix);
         __syncthreads();
+        // terms that are not below the rounding of the sums, infinities and
+        // NaN: the rest of the rows are summed too
+        bool rest = false;
         if (mine) {
+            rest = !(hist[0] - hist[0] == C(0));
 #pragma unroll
             for (int q = 0; q < BW; ++q) {
                 const C A = x[(H + q) * step];
                 const C t = static_cast<C>(sp.strip_rest) * vmax;
-                bad = bad || !(A - t == A && A + t == A) || same_bits(A, C(-0.0));
+                rest = rest || !(A - t == A && A + t == A) || same_bits(A, C(-0.0));
             }
         }
+        if (__any(rest) && (threadIdx.x & 63) == 0) failed[1] = 1;
         if (any_bad(bad)) return false;
+        if (failed[1]) {
+            if (line < nl && seg < BW) strip(x[(H + seg) * step], prefix, rows);
+            __syncthreads();
+        }
         if (line < nl && seg == 0) {
             // the last rows, then the backward rows that fix the corners
             LineState<BW, CYC, C> st;
@@ -750,8 +784,7 @@ __device__ __forceinline__ bool solve_segments(const SolveParams& sp, C* tile, i
     // backward: segment `seg` from the end; in sweep order row r is H - 1 - r
     const int top = H - seg * len;
     const int blo = H - min(sp.bhi, H), bhi = H - sp.blo;
-    const KnownDivisor<C> kz{static_cast<C>(sp.zh), static_cast<C>(sp.zl)};
-    int least = 0;
+    const KnownDivisor<C> kz = known_pivot<C>(sp);
     C nxt[BW + 1];
     nxt[BW] = C(0);
 #pragma unroll
@@ -759,22 +792,20 @@ __device__ __forceinline__ bool solve_segments(const SolveParams& sp, C* tile, i
     if (segs > 1) {
         seg_backward<BW, CYC, false, C, B>(x, step, 0, n, top + warm - 1, warm, H, mine && seg > 0,
                                            equal_batches(max(seg0, 1), seg1, len, warm, warm, blo, bhi, H, B), sp,
-                                           edge, kz, corner, nxt, least);
+                                           edge, kz, corner, nxt);
 #pragma unroll
         for (int m = 0; m < BW; ++m) start[m] = nxt[m];
         __syncthreads();
     }
     seg_backward<BW, CYC, true, C, B>(x, step, 0, n, top - 1, len, H, mine,
                                       equal_batches(seg0, seg1, len, 0, len, blo, bhi, H, B), sp, edge, kz, corner,
-                                      nxt, least);
+                                      nxt);
     __syncthreads();
-    bad = kz.underflows(least);
-    if (mine) {
-        if (BW > 0) bad = bad || !(nxt[0] - nxt[0] == C(0));  // infinities and NaN
-        if (seg > 0) {
+    if (segs == 1) return true;
+    bad = false;
+    if (mine && seg > 0) {
 #pragma unroll
-            for (int m = 0; m < BW; ++m) bad = bad || !same_bits(start[m], x[(top + m) * step]);
-        }
+        for (int m = 0; m < BW; ++m) bad = bad || !same_bits(start[m], x[(top + m) * step]);
     }
     return !any_bad(bad);
 }
@@ -913,7 +944,7 @@ __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first,
     };
     bool done = false;
     if constexpr (SEG) {
-        __shared__ int failed;
+        __shared__ int failed[2];
         EdgeTable<C> edge;
         if (sp.segs > 0) {
             const int pad = static_cast<int>(kTilePad) * step;
@@ -921,17 +952,16 @@ __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first,
             edge = stage_edges<BW, C>(sp, reinterpret_cast<C*>(tile_bytes) + tile_elements(n, lpb, inner), tid, NT);
         }
         load();
-        // segmented; then, if a comparison failed, one segment per line;
-        // then, if the strips or a pivot's division need it, the plain
-        // substitution
+        // segmented; then, if a comparison failed, one segment per line,
+        // which has nothing to compare
 #pragma unroll 1
         for (int segs = sp.segs; segs > 0 && !done; segs = segs > 1 ? 1 : 0) {
             // the usual row stride of many lines as a constant: row offsets
             // become immediates of the LDS instructions
             if (FIXED && step == kTileStep)
-                done = solve_segments<BW, CYC, C, B>(sp, tile, kTileStep, nl, lpb, segs, edge, tid, &failed);
+                done = solve_segments<BW, CYC, C, B>(sp, tile, kTileStep, nl, lpb, segs, edge, tid, failed);
             else
-                done = solve_segments<BW, CYC, C, B>(sp, tile, step, nl, lpb, segs, edge, tid, &failed);
+                done = solve_segments<BW, CYC, C, B>(sp, tile, step, nl, lpb, segs, edge, tid, failed);
             if (!done) load();
         }
     } else {

@@ -362,7 +362,7 @@ __global__ __launch_bounds__(256) void long_backward_kernel(LongParams<C> p) {
     corner[BW] = C(0);
 #pragma unroll
     for (int c = 0; c < BW; ++c) corner[c] = CYC && line < nl ? p.corner[(first + line) * BW + c] : C(0);
-    const KnownDivisor<C> kz{static_cast<C>(sp.zh), static_cast<C>(sp.zl)};
+    const KnownDivisor<C> kz = known_pivot<C>(sp);
     const int blo = H - min(sp.bhi, H), bhi = H - sp.blo;
     C start[BW + 1], nxt[BW + 1];
     nxt[BW] = C(0);
@@ -372,38 +372,29 @@ __global__ __launch_bounds__(256) void long_backward_kernel(LongParams<C> p) {
         const bool mine = line < nl && seg < segs && top > 0;
         const int wave = __builtin_amdgcn_readfirstlane(tid) & ~63;
         const int seg0 = wave >> shift, seg1 = min((wave + 63) >> shift, min(segs, (e0 + len - 1) / len) - 1);
-        // the second attempt divides in full everywhere
-        const BatchRange none{0, 0};
         const int before = H - e0;
 #pragma unroll
         for (int m = 0; m < BW; ++m) nxt[m] = CYC && top + warm >= H ? corner[m] : C(0);
-        int least = 0;
         if (tid == 0) failed = 0;
-        seg_backward<BW, CYC, false, C, B>(
-            x, step, origin, n, top + warm - 1, warm, H, mine && top < H,
-            attempt > 0 ? none : equal_batches(seg0, seg1, len, warm - before, warm, blo, bhi, H, B), sp, edge, kz,
-            corner, nxt, least);
+        seg_backward<BW, CYC, false, C, B>(x, step, origin, n, top + warm - 1, warm, H, mine && top < H,
+                                           equal_batches(seg0, seg1, len, warm - before, warm, blo, bhi, H, B), sp,
+                                           edge, kz, corner, nxt);
 #pragma unroll
         for (int m = 0; m < BW; ++m) start[m] = nxt[m];
         __syncthreads();
-        seg_backward<BW, CYC, true, C, B>(
-            x, step, origin, n, top - 1, len, H, mine,
-            attempt > 0 ? none : equal_batches(seg0, seg1, len, -before, len, blo, bhi, H, B), sp, edge, kz, corner,
-            nxt, least);
+        seg_backward<BW, CYC, true, C, B>(x, step, origin, n, top - 1, len, H, mine,
+                                          equal_batches(seg0, seg1, len, -before, len, blo, bhi, H, B), sp, edge, kz,
+                                          corner, nxt);
         __syncthreads();
-        bool bad = kz.underflows(least);
-        if (mine) {
-            if (BW > 0) bad = bad || !(nxt[0] - nxt[0] == C(0));  // infinities and NaN
-            if (seg > 0) {
+        bool bad = false;
+        if (mine && seg > 0) {
 #pragma unroll
-                for (int m = 0; m < BW; ++m) bad = bad || !same_bits(start[m], x[(top + m - origin) * step]);
-            }
+            for (int m = 0; m < BW; ++m) bad = bad || !same_bits(start[m], x[(top + m - origin) * step]);
         }
         if (__any(bad) && (tid & 63) == 0) failed = 1;
         __syncthreads();
-        const bool again = failed != 0 && attempt == 0;
-        __syncthreads();
-        if (!again) break;
+        const bool again = failed != 0;
+        if (!again) break;  // one segment has no cuts: the second attempt ends here
         load();
     }
     T* __restrict__ X = static_cast<T*>(sp.x);

@@ -19,9 +19,9 @@ constexpr int kSegRows = 8;  // segments and warm-ups are multiples of this
 constexpr int64_t kLdsBytes = 160 * 1024;
 constexpr int64_t kTileLdsBudget = 80 * 1024;
 // Static LDS of the kernels that call solve_tile, at most: two offsets a
-// line and, for each variant the kernel holds, a flag; rounded up to the 16
+// line and, for each variant the kernel holds, two flags; rounded up to the 16
 // bytes at which the dynamic part (the tile) starts.
-constexpr int64_t kTileStaticLds = 2 * kMaxTileLines * 8 + 64;
+constexpr int64_t kTileStaticLds = 2 * kMaxTileLines * 8 + 128;
 
 // Row stride of a tile in elements: odd on the contiguous axis, so that
 // the coalesced runs along a line spread over the LDS banks, and for

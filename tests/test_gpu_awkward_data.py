@@ -1,0 +1,73 @@
+"""Builds on data whose segments do not join (solve_impl.hpp): fields that
+decay faster than the factors fade, zeros after data, values near underflow.
+They may cost a second pass over the tiles, not more, and refined (FP32) lines
+must come out right on them too."""
+import numpy as np
+import pytest
+
+from oracle import OracleSpline
+
+pytestmark = pytest.mark.gpu
+
+
+def _field(kind, n):
+    import torch
+    rng = torch.Generator(device="cuda").manual_seed(n)
+    noise = torch.randn((n, n, n), dtype=torch.float64, device="cuda", generator=rng)
+    if kind == "noise":
+        return noise
+    if kind == "tiny":
+        return noise * 1e-290
+    x = torch.linspace(0, 1, n, dtype=torch.float64, device="cuda")
+    g = torch.exp(-((x - 0.5) / 0.02) ** 2) if kind == "gaussian" else ((x - 0.5).abs() < 0.2).double() * (1 + x)
+    return (g[:, None, None] * g[:, None] * g).contiguous()
+
+
+def _microseconds(build):
+    import torch
+    best = float("inf")
+    for _ in range(15):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        spline = build()
+        end.record()
+        torch.cuda.synchronize()
+        best = min(best, start.elapsed_time(end) * 1e3)
+    return best
+
+
+@pytest.mark.parametrize("order,n", [(3, 256), (3, 180)])
+def test_gpu_values_near_underflow_cost_no_multiple(order, n):
+    """A batch of rows whose division would underflow is divided in full:
+    about 70 more cycles a row beside the 40 of the substitution and the
+    copying of the tile, and no second pass over it."""
+    import bsplineinterpolation_amd as amd
+    t = amd.InterpolationFunctionTemplate(order, (n, n, n), ranges=[(0.0, 1.0)] * 3)
+    base = _microseconds(lambda f=_field("noise", n): t.interpolate(f))
+    us = _microseconds(lambda f=_field("tiny", n): t.interpolate(f))
+    print("order %d %d^3: %.0f and %.0f us" % (order, n, base, us), flush=True)
+    assert us <= 1.85 * base
+
+
+@pytest.mark.parametrize("order,shape,periodic", [(3, (1000,), "0"), (5, (700,), "0"), (3, (1001,), "1"), (3, (70, 300), "00"),
+                                                  (4, (300, 70), "10")])
+@pytest.mark.parametrize("kind", ["constant", "zero_tail", "impulse", "gaussian"])
+def test_gpu_awkward_refined_lines(order, shape, periodic, kind):
+    import bsplineinterpolation_amd as amd
+    rng = np.random.default_rng(order)
+    f = rng.standard_normal(shape)
+    if kind == "constant":
+        f[:] = 0.7372
+    elif kind == "zero_tail":
+        f[..., shape[-1] // 3:] = 0.0
+    elif kind == "impulse":
+        f[:] = 0.0
+        f.flat[f.size // 2] = 1.0
+    else:
+        f = np.exp(-((np.indices(shape)[-1] / shape[-1] - 0.5) / 0.02) ** 2)
+    kw = dict(periodic=[c == "1" for c in periodic], ranges=[(0.0, 1.0)] * len(shape))
+    want = OracleSpline(order, f, **kw).control_points()
+    got = amd.InterpolationFunction(order, f, precision="f32_refined", sweeps=2, **kw).control_points()
+    # a refined control point is the FP64 one rounded to FP32, up to an error
+    # of the last correction far below an FP32 rounding of the largest value
+    assert np.max(np.abs(got - want.reshape(got.shape))) <= 2.0 ** -23 * np.max(np.abs(want))
