@@ -422,10 +422,12 @@ int solve_axes(const GridData& g, bool refined, const double* values, void* x, v
         for (int d = a + 1; d < g.dim; ++d) sp.inner *= g.setup[d].n;
         sp.nlines = g.total / s.n;
         set_segment_params(types == SolveTypes::kF32 ? s.lu.seg32 : s.lu.seg64, &sp);
+        if (a == 0) sp.accum = accum;
         plans[a] = solve_tile_plan(sp, s.lu.p, s.lu.cyclic, compute_bytes(types));
         sp.lines_per_block = plans[a].lines;
         sp.segs = plans[a].segs;
-        if (plans[a].lines == 0) chunk_bytes[a] = solve_long_scratch(sp, s.lu.p, s.lu.cyclic, compute_bytes(types));
+        if (plans[a].lines == 0 && !plans[a].in_place)
+            chunk_bytes[a] = solve_long_scratch(sp, s.lu.p, s.lu.cyclic, compute_bytes(types));
         scratch_bytes = std::max(scratch_bytes, chunk_bytes[a]);
     }
     StreamBlock scratch(stream);
@@ -477,8 +479,8 @@ int solve_axes(const GridData& g, bool refined, const double* values, void* x, v
             }
             sp.shift_last = shift[last];
         }
-        const bool add_after = a == 0 && accum != nullptr && sp.lines_per_block == 0;
-        if (a == 0 && accum != nullptr && !add_after) sp.accum = accum;
+        const bool add_after = sp.accum != nullptr && sp.lines_per_block == 0;
+        if (add_after) sp.accum = nullptr;
         hipError_t e;
         if (chunk_bytes[a] > 0)
             e = launch_solve_long(s.lu.p, s.lu.cyclic, types, sp, scratch.p, stream);

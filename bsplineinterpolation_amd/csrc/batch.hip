@@ -444,13 +444,13 @@ __global__ __launch_bounds__(NT, 2) void batch_solve_kernel(const BatchSpline* s
 constexpr int kEvalStreams = 4;
 
 // LDS budget of the tile of one solve workgroup (two per CU).
-constexpr int64_t kBatchTileBudget = kTileLdsBudget - kTileStaticLds - kEdgeMax * 8;
+constexpr int64_t kBatchTileBudget = kTileLdsBudget - kBatchStaticLds - kEdgeMax * 8;
 
 int64_t tile_fit(int64_t n, int64_t inner, int cap) {
     int lpb = kMaxTileLines;
-    while (lpb > 0 && (lpb > cap || tile_elements(n, lpb, inner) * 8 > kBatchTileBudget)) lpb /= 2;
+    while (lpb > 0 && (lpb > cap || tile_elements(n, lpb, inner, 1) * 8 > kBatchTileBudget)) lpb /= 2;
     // one line may take most of a CU's LDS
-    if (lpb == 0 && tile_elements(n, 1, inner) * 8 <= kBatchTileBudget + kLdsBytes - kTileLdsBudget) lpb = 1;
+    if (lpb == 0 && tile_elements(n, 1, inner, 1) * 8 <= kBatchTileBudget + kLdsBytes - kTileLdsBudget) lpb = 1;
     return lpb;
 }
 
@@ -651,7 +651,7 @@ int make_solve_work(intp_batch b, hipStream_t stream) {
             if (D == 1) {
                 // batch_line_kernel, beside the passes
                 if (bs.lines_per_block[0] > 0)
-                    b->line_lds = std::max(b->line_lds, static_cast<size_t>((tile_elements(ds.n, 1, 1) +
+                    b->line_lds = std::max(b->line_lds, static_cast<size_t>((tile_elements(ds.n, 1, 1, 1) +
                                                                              edge_rows(ds, bs.segs[0])) * 8));
                 continue;
             } else if (bs.lines_per_block[a] == 0) {
@@ -660,7 +660,7 @@ int make_solve_work(intp_batch b, hipStream_t stream) {
                         {cost, BatchSolveItem{s, static_cast<int16_t>(a), kind_of(ds, kSolveLanes), first}});
             } else {
                 const int64_t lpb = bs.lines_per_block[a];
-                const int64_t bytes = (tile_elements(ds.n, lpb, inner) + edge_rows(ds, bs.segs[a])) * 8;
+                const int64_t bytes = (tile_elements(ds.n, lpb, inner, 1) + edge_rows(ds, bs.segs[a])) * 8;
                 // lines cut into segments keep every wave busy; the others one
                 const bool small = bytes <= kSmallTileBytes && bs.segs[a] == 0;
                 const bool medium = !small && bytes <= kMediumTileBytes && bs.segs[a] == 0;

@@ -231,11 +231,12 @@ struct SolveParams {
 // Lines shorter than this are not cut into segments.
 constexpr int64_t kMinSegmentRows = 128;
 
-// Shape of the LDS-tiled kernel for one axis: lines per workgroup (0: the
-// tile does not fit, solve in HBM), segments per line (0: plain
-// substitution), threads.
+// Shape of the LDS-tiled kernel for one axis: lines per workgroup, segments
+// per line (0: plain substitution), threads.  lines 0: in HBM, one lane a
+// line, because that is faster (in_place) or because no tile fits.
 struct TilePlan {
     int lines = 0, segs = 0, threads = 256;
+    bool in_place = false;
 };
 
 struct ShiftParams {

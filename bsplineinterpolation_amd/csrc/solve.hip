@@ -19,22 +19,30 @@ __global__ __launch_bounds__(kSolveBlock) void solve_kernel(SolveParams sp) {
     substitute<BW, CYC, C, T, B>(static_cast<T*>(sp.x) + o * sp.n * sp.inner + ii, sp.inner, sp.n, sp);
 }
 
-// Waves per SIMD the tile kernel is built for: three (168 VGPRs) where that
+// Waves per SIMD the tile kernels are built for: three (168 VGPRs) where that
 // does not spill, so that tiles of short lines share a CU three at a time
-// (150^3 cubic, one axis: 34 us at two, 27 us at three; four spill).
-template <int BW, bool CYC, typename C>
+// (150^3 cubic, one axis: 34 us at two, 27 us at three; four spill).  Uncut
+// lines have a kernel of their own, with about half the registers (orders 4
+// and 7, 136^3, the contiguous axis, us: 48 and 64 as the cut kernel's plain
+// path, 35 and 37); wide FP64 bands are held to three waves, or the compiler
+// spends the rest on more waves and not on loads in flight (order 7, 256^3:
+// 250 us unbounded, 215).
+template <int BW, bool CYC, typename C, bool SEG>
 constexpr int tile_waves() {
+    if (!SEG) return sizeof(C) == 8 && (BW == 4 || (CYC && BW == 2)) ? 2 : 3;
     return !CYC && (sizeof(C) == 4 || BW <= 2) ? 3 : 2;
 }
 
-template <int BW, bool CYC, typename T, typename C>
-__global__ __launch_bounds__(kMaxTileThreads, (tile_waves<BW, CYC, C>())) void solve_tile_kernel(SolveParams sp) {
+template <int BW, bool CYC, typename T, typename C, bool SEG>
+__global__ __launch_bounds__(SEG ? kMaxTileThreads : kTileThreads)
+    __attribute__((amdgpu_waves_per_eu((tile_waves<BW, CYC, C, SEG>()), !SEG && BW >= 4 && sizeof(C) == 8 ? 3 : 8))) void solve_tile_kernel(SolveParams sp) {
     extern __shared__ __align__(16) unsigned char tile_bytes[];
     __shared__ int64_t dst_base[kMaxTileLines];
     __shared__ int64_t src_base[kMaxTileLines];
     const int nt = static_cast<int>(blockDim.x);  // a power of two
-    solve_tile<BW, CYC, T, C>(sp, static_cast<int64_t>(blockIdx.x) * sp.lines_per_block, tile_bytes, dst_base,
-                              src_base, static_cast<int>(threadIdx.x + 64 * blockIdx.x) & (nt - 1), nt);
+    solve_tile<BW, CYC, T, C, batch_rows<BW, CYC>(), SEG>(
+        sp, static_cast<int64_t>(blockIdx.x) * sp.lines_per_block, tile_bytes, dst_base, src_base,
+        static_cast<int>(threadIdx.x + 64 * blockIdx.x) & (nt - 1), nt);
 }
 
 template <int BW, bool CYC, typename T, typename C>
@@ -45,8 +53,11 @@ hipError_t launch_lines(const SolveParams& p, int threads, hipStream_t s) {
         if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
         const int64_t lds = tile_lds(p, BW, sizeof(C));
         if (lds + kTileStaticLds > kLdsBytes) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((solve_tile_kernel<BW, CYC, T, C>), dim3(static_cast<unsigned>(blocks)),
-                           dim3(static_cast<unsigned>(threads)), static_cast<size_t>(lds), s, p);
+        const dim3 grid(static_cast<unsigned>(blocks)), block(static_cast<unsigned>(threads));
+        if (p.segs > 0)
+            hipLaunchKernelGGL((solve_tile_kernel<BW, CYC, T, C, true>), grid, block, static_cast<size_t>(lds), s, p);
+        else
+            hipLaunchKernelGGL((solve_tile_kernel<BW, CYC, T, C, false>), grid, block, static_cast<size_t>(lds), s, p);
         return hipGetLastError();
     }
     const int64_t blocks = (p.nlines + kSolveBlock - 1) / kSolveBlock;
@@ -78,9 +89,9 @@ hipError_t launch_bw(bool cyclic, const SolveParams& p, int threads, hipStream_t
     if (p.lines_per_block > 0) {
         // whole lanes per line, every segment's lane present, rows in 32 bits
         const int lpb = p.lines_per_block;
-        if (lpb > kMaxTileLines || threads > kMaxTileThreads || threads % lpb != 0 || threads % 64 != 0 ||
+        if (lpb > kMaxTileLines || threads > (p.segs > 0 ? kMaxTileThreads : kTileThreads) || threads % lpb != 0 || threads % 64 != 0 ||
             (threads & (threads - 1)) != 0 ||
-            (lpb & (lpb - 1)) != 0 || p.segs < 0 || p.segs > threads / lpb || (p.segs > 1 && p.segs < BW) || threads / lpb < BW ||
+            (lpb & (lpb - 1)) != 0 || p.segs < 0 || p.segs > threads / lpb || (p.segs > 1 && p.segs < BW) || (p.segs > 0 && threads / lpb < BW) ||
             p.n >= (int64_t{1} << 24))
             return hipErrorInvalidValue;
     } else if (p.src || p.accum) {

@@ -333,7 +333,7 @@ __device__ __forceinline__ void warm_factors(const SolveParams& sp, int64_t n) {
 // the state it started from with the rows its neighbour stored, bit for
 // bit.  Equal states mean equal rows, so a line that passes holds exactly
 // the sequential result.  If any comparison of a workgroup fails, the tile
-// is loaded again and solved with one segment per line.  That happens on
+// is loaded again and solved in one piece.  That happens on
 // exactly constant lines (two starts can settle on neighbouring fixed
 // points: 0.7 to 16 % of the boundaries for orders 3 and 4, up to 40 % at
 // order 5) and where data decays faster than the factors fade (a Gaussian's
@@ -813,11 +813,12 @@ __device__ __forceinline__ bool solve_segments(const SolveParams& sp, C* tile, i
 // One workgroup: lines [first, first + lpb) staged through LDS in the
 // compute type C; the table holds T.  Row j of line l sits at
 // tile[j * step + l].  With sp.accum set, the solved lines are added into
-// accum instead of being stored to x.  segs == 0: plain substitution.
+// accum instead of being stored to x.
 // tid: the thread's place in the workgroup of NT threads, whole waves of it
 // in any order (the callers rotate the waves: where one wave substitutes,
 // neighbouring workgroups on a CU then use different SIMDs).
-// SEG false: kernels whose lines are never cut.  FIXED: with a copy of the
+// SEG false: plain substitution (sp.segs 0), without the segments' pad rows.
+// SEG true with sp.segs 0 (the batch's 256-thread kernel): plain, with them.  FIXED: with a copy of the
 // segment code for the row stride kTileStep.
 template <int BW, bool CYC, typename T, typename C, int B = batch_rows<BW, CYC>(), bool SEG = true,
           bool FIXED = true>
@@ -826,7 +827,7 @@ __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first,
     const int lpb = sp.lines_per_block;
     const int64_t n = sp.n, inner = sp.inner;
     const int step = static_cast<int>(tile_step(lpb, inner));
-    C* tile = reinterpret_cast<C*>(tile_bytes) + kTilePad * step;
+    C* tile = reinterpret_cast<C*>(tile_bytes) + (SEG ? kTilePad : 0) * step;
     T* __restrict__ X = static_cast<T*>(sp.x);
     const int nl = static_cast<int>(min(static_cast<int64_t>(lpb), sp.nlines - first));
     if (tid < nl) {
@@ -949,13 +950,15 @@ __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first,
         if (sp.segs > 0) {
             const int pad = static_cast<int>(kTilePad) * step;
             for (int i = tid; i < pad; i += NT) tile[i - pad] = tile[static_cast<int>(n) * step + i] = C(0);
-            edge = stage_edges<BW, C>(sp, reinterpret_cast<C*>(tile_bytes) + tile_elements(n, lpb, inner), tid, NT);
+            edge = stage_edges<BW, C>(sp, reinterpret_cast<C*>(tile_bytes) + tile_elements(n, lpb, inner, 1), tid, NT);
         }
         load();
-        // segmented; then, if a comparison failed, one segment per line,
-        // which has nothing to compare
+        // segmented; then, if a comparison failed, in one piece: as one
+        // segment, which has nothing to compare, or plainly where the rows of
+        // equal factors do not make up for its steps (plan_tile)
+        const bool one = CYC || (sp.fast_divide && BW <= 2);
 #pragma unroll 1
-        for (int segs = sp.segs; segs > 0 && !done; segs = segs > 1 ? 1 : 0) {
+        for (int segs = sp.segs; segs > 0 && !done; segs = segs > 1 && one ? 1 : 0) {
             // the usual row stride of many lines as a constant: row offsets
             // become immediates of the LDS instructions
             if (FIXED && step == kTileStep)

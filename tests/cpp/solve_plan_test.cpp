@@ -90,11 +90,44 @@ void chunks(int64_t static_lds) {
     check(s.lu.seg64.warm > 340, "warm-up of graded nodes", 7, 0, 8, 6000, 64, s.lu.seg64.warm);
 }
 
+// How lines are solved where the fastest way is clear from measurement: cut
+// where few lines leave the chip idle, in place where many lie side by side.
+void choices() {
+    enum { kCut, kWhole, kInPlace };
+    const struct {
+        int order, periodic;
+        int64_t n, nlines, inner;
+        int want;
+    } cases[] = {
+        {3, 0, 8192, 1, 1, kCut},         {6, 1, 8192, 1, 1, kCut},         {3, 0, 2000, 2000, 1, kCut},
+        {3, 0, 2000, 2000, 2000, kCut},   {5, 0, 1021, 769, 769, kCut},     {3, 0, 1000, 4096, 64, kCut},
+        {3, 0, 256, 65536, 1, kCut},      {5, 0, 256, 65536, 1, kWhole},    {7, 0, 200, 40000, 1, kWhole},
+        {3, 0, 256, 65536, 256, kInPlace}, {5, 0, 256, 65536, 65536, kInPlace}, {7, 0, 180, 32400, 180, kInPlace},
+        {6, 1, 180, 32400, 180, kInPlace}, {5, 0, 64, 65536, 65536, kInPlace}, {5, 0, 100, 50000, 100, kInPlace},
+        {3, 0, 20, 90000, 300, kInPlace},  {3, 0, 100, 10000, 100, kWhole},  {5, 0, 80, 6400, 80, kWhole},
+        {3, 0, 64, 64, 64, kWhole},        {3, 0, 64, 4096, 64, kWhole},
+    };
+    for (const auto& c : cases) {
+        DimSetup s;
+        if (!setup_dimension(c.order, c.periodic != 0, c.n, 0.0, 1.0, nullptr, s, true).empty()) std::abort();
+        SolveParams p{};
+        set_segment_params(s.lu.seg64, &p);
+        p.n = c.n;
+        p.nlines = c.nlines;
+        p.inner = c.inner;
+        const TilePlan plan = plan_tile(p, s.lu.p, s.lu.cyclic, 8, kLdsBytes);
+        const int got = plan.in_place ? kInPlace : plan.lines == 0 ? -1 : plan.segs > 1 ? kCut : kWhole;
+        check(got == c.want, "choice", c.order, c.periodic, 8, c.n, c.inner, got);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     tiles(argc > 1 ? std::atoll(argv[1]) : kTileStaticLds);
+    choices();
     chunks(argc > 2 ? std::atoll(argv[2]) : kLongStaticLds);
+    check(argc < 4 || std::atoll(argv[3]) <= kBatchStaticLds, "batch kernels' static LDS", 0, 0, 0, 0, 0, argc < 4 ? 0 : std::atoll(argv[3]));
     if (failures) std::printf("%d failures\n", failures);
     return failures ? 1 : 0;
 }

@@ -43,7 +43,8 @@ def _static_lds(tmp, kernels):
 
 
 def test_solve_plans_fit_lds(plan_test, tmp_path):
-    static = _static_lds(str(tmp_path), ("solve_tile_kernel", "batch_solve_kernel", "batch_line_kernel"))
+    static = _static_lds(str(tmp_path), ("solve_tile_kernel",))
+    batch = _static_lds(str(tmp_path), ("batch_solve_kernel", "batch_line_kernel"))
     chunks = _static_lds(str(tmp_path), ("long_forward_kernel", "long_backward_kernel"))
-    out = subprocess.run([plan_test, str(static), str(chunks)], capture_output=True, text=True, timeout=110)
+    out = subprocess.run([plan_test, str(static), str(chunks), str(batch)], capture_output=True, text=True, timeout=110)
     assert out.returncode == 0, out.stdout

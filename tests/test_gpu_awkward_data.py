@@ -49,6 +49,22 @@ def test_gpu_values_near_underflow_cost_no_multiple(order, n):
     assert us <= 1.85 * base
 
 
+@pytest.mark.parametrize("order,n,periodic", [(3, 256, False), (5, 256, False), (3, 256, True), (3, 200, False)])
+def test_gpu_awkward_fields_cost_no_multiple(order, n, periodic):
+    """Lines are cut only where that gains though half of the tiles fail, and
+    a failed tile costs its own time and less than that of uncut ones: less
+    than 1 + 0.6 / 0.7 of what cut ones cost, on the axes that are cut."""
+    import bsplineinterpolation_amd as amd
+    t = amd.InterpolationFunctionTemplate(order, (n, n, n), periodic=[periodic] * 3, ranges=[(0.0, 1.0)] * 3)
+    base = None
+    for kind in ("noise", "gaussian", "box"):
+        f = _field(kind, n)
+        us = _microseconds(lambda: t.interpolate(f))
+        print("order %d %d^3 %s: %.0f us" % (order, n, kind, us), flush=True)
+        base = base or us
+        assert us <= 1.85 * base, kind
+
+
 @pytest.mark.parametrize("order,shape,periodic", [(3, (1000,), "0"), (5, (700,), "0"), (3, (1001,), "1"), (3, (70, 300), "00"),
                                                   (4, (300, 70), "10")])
 @pytest.mark.parametrize("kind", ["constant", "zero_tail", "impulse", "gaussian"])
