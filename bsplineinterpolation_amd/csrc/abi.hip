@@ -20,6 +20,7 @@
 #include "../../include/intp_amd.h"
 #include "kernels.hpp"
 #include "grid.hpp"
+#include "group_rule.hpp"
 #include "host_eval.hpp"
 #include "runtime.hpp"
 #include "setup.hpp"
@@ -621,43 +622,6 @@ DimParams dim_params(const GridData& g, int d) {
     int64_t stride = 1;
     for (int e = d + 1; e < g.dim; ++e) stride *= g.setup[e].n;
     return make_dim_params(g.setup[d], g.order, stride, g.knots[d], g.recip[d], g.poly[d]);
-}
-
-// Whether grouping by brick before evaluation pays.  In caller order a point
-// costs the cache lines of its stencil rows: 4.2 ps a line from L2 and 12.5
-// ps more for the share of the table beyond it.  Grouped, a call costs
-// about 85 us and 30 ps a point, each result 16 ps and each stencil element
-// of a launch 0.0125 ps a byte; 30 ps more where the patches come from
-// beyond L2, 100 us and 200 ps more where they do not fit LDS (`staged`
-// false), and the caller-order cost of the points that leave their chunk's
-// brick, about 5 a brick.  Measured on both sides of the line (us, caller order / grouped,
-// 3D, value and first partials unless said):
-//   cubic,   100^3:        400,000 points 84/110, 1M 187/155, 10M 1717/1252
-//   cubic,   48^3:         3M points 248/269, 10M 807/1037
-//   order 4, 48^3, value:  400,000 points 66/83, 1M 143/112, 10M 1269/684
-//   order 5, 100^3:        131,072 points 63/98, 400,000 185/134, 10M 3984/1429
-//   order 5, 160x140x150:  131,072 points 101/105, 400,000 300/154
-//   order 5, 100^3, refined: 131,072 points 107/112, 400,000 319/149
-//   order 5, 256^3, refined: 131,072 points 157/190, 400,000 463/334
-//   order 2, 160x140x150:  1M points 172/156, 10M 1565/1261
-//   order 1, 256^3:        1M points 100/176, 10M 915/1352
-// 2D stencils have k + 1 rows only: 2D tables gain beyond the 256 MB
-// Infinity Cache, from 2^20 points on (2^24 points on 1024^2, cubic: 0.87
-// ms in caller order, 2.15 ms grouped).
-bool group_pays(int dim, int order, int elem_bytes, int64_t elements, int64_t npts, int launches, int results,
-                bool staged, int64_t bricks) {
-    const double table = static_cast<double>(elements) * elem_bytes;
-    if (dim != 3) return npts >= (int64_t{1} << 20) && table >= 0x1p28;
-    const int row = order + 1;
-    const double lines = static_cast<double>(row) * row * (1.0 + order * elem_bytes / 128.0);
-    const double missed = table > 0x1.4p22 ? 1.0 - 0x1.4p22 / table : 0.0;  // 5 MB
-    const double n = static_cast<double>(npts);
-    const double caller_order = n * launches * lines * (4.2 + 12.5 * missed);
-    const double grouped = 85e6 + n * (30.0 + 16.0 * results + launches * 0.0125 * elem_bytes * row * row * row +
-                                       30.0 * missed) +
-                           (staged ? 0.0 : 100e6 + 200.0 * n) +
-                           caller_order * std::min(1.0, 5.0 * static_cast<double>(bricks) / n);
-    return caller_order > grouped;
 }
 
 // Grouped results go to their callers' positions in random order.  Three or
@@ -1323,38 +1287,55 @@ int eval_call(intp_spline s, int64_t npts, const double* coords, int64_t cs_dim,
     const int elem_bytes = cells ? cell_bytes(D) : s->ctrl_bytes;
     const bool forced = (flags & INTP_EVAL_GROUPED) != 0;
     const int launches = static_cast<int>(single.size()) + (any_grad ? 1 : 0);
-    // (at 2.1 ns a point, the most it can cost, fewer do not pay)
-    bool group = !(flags & INTP_EVAL_UNGROUPED) && (forced ? npts > 0 : npts * launches >= 32768 && fast && D >= 2 && D <= kGroupDim);
-    const bool two_ok = group && fast && D >= 2 && D <= kGroupDim && npts <= 0xFFFFFFFFll && bin_scan_tiles(npts) <= 4096;
+    const bool uniform3 = fast && D >= 2 && D <= kGroupDim && npts <= 0xFFFFFFFFll;
+    bool group = uniform3 && !(flags & INTP_EVAL_UNGROUPED) &&
+                 (forced || group_considered(npts, launches, sc.fixed()));
+    const bool two_ok = group && bin_scan_tiles(npts) <= 4096;
     int64_t patch_volume = 0;
     BinParams bp{};
     if (two_ok) bp = bin_params(g, elem_bytes, &patch_volume);
+    BrickGrid ib{};
+    int64_t item_patch = 0;
+    int32_t item_bins = 0;
+    const bool bricks_ok = group && item_bricks(g, elem_bytes, &ib, &item_patch, &item_bins);
+    // Two radix passes by default (measured faster at 256^3); one pass on
+    // request, for a fixed scratch buffer, where it needs half the memory,
+    // and at the widest stencils where the radix bricks' patches exceed LDS
+    // and the bricks of the one pass hold enough points for its counters
+    // (order 7, value, us in two passes/one: 200x220x210, 1M points 429/568,
+    // 3M 1101/1059; 256^3, 3M 1198/1459, 10M 3614/3334).  Narrower stencils
+    // gain more from the small bricks also without patches (400^3, 2^24
+    // points, value and partials: order 2 2153/3304, cubic 2633/3322).
+    bool one_pass = bricks_ok && ((flags & INTP_EVAL_GROUP_ONE_PASS) || sc.fixed() || !two_ok ||
+                                  (!forced && g.order >= 6 && patch_volume == 0 &&
+                                   npts >= 384 * static_cast<int64_t>(item_bins)));
     if (group && !forced) {
-        int64_t bricks = 1;
-        for (int d = 0; d < bp.dim_count; ++d) bricks *= bp.bricks.nbrick[d];
-        group = group_pays(D, g.order, elem_bytes, g.total, npts, launches, nout, patch_volume > 0, bricks);
+        GroupCase gc;
+        gc.dim = D;
+        gc.order = g.order;
+        gc.elem_bytes = elem_bytes;
+        gc.elements = g.total;
+        gc.npts = npts;
+        gc.launches = launches;
+        gc.results = nout;
+        gc.one_pass = one_pass;
+        gc.staged = patch_volume > 0;
+        gc.bricks = item_bins;
+        if (!one_pass) {
+            gc.bricks = 1;
+            for (int d = 0; d < bp.dim_count; ++d) gc.bricks *= bp.bricks.nbrick[d];
+        }
+        group = group_pays(gc);
     }
-    if (group && !forced && (npts < (int64_t{1} << 20) || g.total * s->ctrl_bytes < (int64_t{16} << 20))) {
+    if (group && !forced && !sc.fixed() && (npts < (int64_t{1} << 20) || g.total * s->ctrl_bytes < (int64_t{16} << 20))) {
         // a call that is being captured allocates only for large batches
         // on large tables
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(stream, &capturing) != hipSuccess) (void)hipGetLastError();
         group = capturing == hipStreamCaptureStatusNone;
     }
-    BrickGrid ib{};
-    int64_t item_patch = 0;
-    int32_t item_bins = 0;
-    const bool groupable = fast && D >= 2 && D <= kGroupDim && group && npts <= 0xFFFFFFFFll;
-    const bool bricks_ok = groupable && item_bricks(g, elem_bytes, &ib, &item_patch, &item_bins);
-    // Two radix passes by default (measured faster at 256^3); one pass on
-    // request, for a fixed scratch buffer, where it needs half the memory,
-    // and where the radix bricks' patches exceed LDS and the bricks of the
-    // one pass hold enough points for its counters (order 7, value, us in
-    // two passes/one: 200x220x210, 1M points 429/568, 3M 1101/1059; 256^3,
-    // 3M 1198/1459, 10M 3614/3334).
-    bool one_pass = bricks_ok && ((flags & INTP_EVAL_GROUP_ONE_PASS) || sc.fixed() || !two_ok ||
-                                  (!forced && patch_volume == 0 && npts >= 384 * static_cast<int64_t>(item_bins)));
-    bool two_pass = !one_pass && groupable && two_ok;
+    one_pass = one_pass && group;
+    bool two_pass = group && !one_pass && two_ok;
     if (sc.fixed() && (one_pass || two_pass)) {
         // the grouping's scratch must fit the fixed buffer; otherwise the
         // points are evaluated in caller order (same results), unless the
