@@ -7,6 +7,8 @@
 
 #include <cstdint>
 
+#include "setup.hpp"
+
 namespace intp_amd {
 
 constexpr int kMaxDim = 6;    // dimensions of a spline
@@ -227,9 +229,6 @@ struct SolveParams {
     double strip_rest;             // the largest bottom strip entry from row `warm` on (cyclic)
     double eq_lower[kMaxOrder], eq_upper[kMaxOrder];  // the factors of those rows
 };
-
-// Lines shorter than this are not cut into segments.
-constexpr int64_t kMinSegmentRows = 128;
 
 // Shape of the LDS-tiled kernel for one axis: lines per workgroup, segments
 // per line (0: plain substitution), threads.  lines 0: in HBM, one lane a

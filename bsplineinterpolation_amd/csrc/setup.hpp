@@ -10,6 +10,9 @@
 
 namespace intp_amd {
 
+// Lines shorter than this are not cut into segments.
+constexpr int64_t kMinSegmentRows = 128;
+
 // Row-oriented LU factors of one dimension's collocation matrix A = L U,
 // L unit lower with p sub-diagonals, U upper with q super-diagonals, plus
 // the cyclic fill of a periodic matrix:

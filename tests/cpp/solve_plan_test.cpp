@@ -123,9 +123,28 @@ void choices() {
 
 }  // namespace
 
+// Lines that are never cut get no segment plan; others do, also where their
+// factors differ from row to row.
+void segment_plans() {
+    for (int order = 2; order <= 7; ++order)
+        for (int periodic = 0; periodic < 2; ++periodic)
+            for (int uniform = 0; uniform < 2; ++uniform)
+                for (int64_t n : {int64_t{20}, kMinSegmentRows - 1, kMinSegmentRows, int64_t{1000}}) {
+                    std::vector<double> x(static_cast<size_t>(n + 1));
+                    for (int64_t i = 0; i <= n; ++i) x[static_cast<size_t>(i)] = 0.3 * i + 0.1 * ((i * 7) % 3);
+                    DimSetup s;
+                    if (!setup_dimension(order, periodic != 0, n, -0.4, 1.7, uniform ? nullptr : x.data(), s, true).empty())
+                        std::abort();
+                    for (const SegmentPlan* seg : {&s.lu.seg64, &s.lu.seg32})
+                        check((seg->warm > 0) == (n >= kMinSegmentRows) && seg->warm % 8 == 0, "warm-up", order, periodic,
+                              seg == &s.lu.seg64 ? 8 : 4, n, uniform, seg->warm);
+                }
+}
+
 int main(int argc, char** argv) {
     tiles(argc > 1 ? std::atoll(argv[1]) : kTileStaticLds);
     choices();
+    segment_plans();
     chunks(argc > 2 ? std::atoll(argv[2]) : kLongStaticLds);
     check(argc < 4 || std::atoll(argv[3]) <= kBatchStaticLds, "batch kernels' static LDS", 0, 0, 0, 0, 0, argc < 4 ? 0 : std::atoll(argv[3]));
     if (failures) std::printf("%d failures\n", failures);
