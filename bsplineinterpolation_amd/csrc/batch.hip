@@ -45,9 +45,9 @@ namespace {
 // two workgroups per CU).
 constexpr int kMergedRows = 4;
 // the segmented tile kernel holds a batch's factors next to its loop state
-template <int BW, bool CYC, int NT>
+template <int BW, bool CYC, bool SEG>
 constexpr int merged_rows() {
-    return NT == 256 && BW * (CYC ? 2 : 1) >= 4 ? 2 : kMergedRows;
+    return SEG && BW * (CYC ? 2 : 1) >= 4 ? 2 : kMergedRows;
 }
 // Small tiles (at most kSmallTileBytes of LDS) are solved by one-wave
 // workgroups, so that every resident wave substitutes a tile of its own
@@ -68,11 +68,19 @@ constexpr int kMaxBatchBand = 6;
 // 1D splines of at least this many points are split (INTP_BATCH_SPLIT_LINES)
 constexpr int64_t kSplitMinRows = 256;
 
-template <int BW, bool CYC, int NT>
+// How the items of one launch are solved: whole lines or lines cut into
+// segments, in LDS tiles, or one line per lane in HBM.
+enum class BatchSolveForm { kWhole, kCut, kLanes };
+
+// Launches of a pass, each with items of one class.
+enum SolveClass { kCutTiles, kLargeTiles, kLanes, kMediumTiles, kSmallTiles, kSolveClasses };
+
+template <int BW, bool CYC, int NT, BatchSolveForm FORM>
 __device__ __forceinline__ void batch_solve_item(const BatchSpline* specs, const BatchSolveItem& w, const double* values, double* ctrl,
                                                  int32_t first_pass, unsigned char* tile_bytes, int64_t* dst_base,
                                                  int64_t* src_base) {
-    if ((w.kind >> 4) == kSolveTile) {
+    if constexpr (FORM != BatchSolveForm::kLanes) {
+        constexpr bool SEG = FORM == BatchSolveForm::kCut;
         const BatchSpline& b = specs[w.spline];
         const int a = w.axis;
         SolveParams sp{};
@@ -89,7 +97,7 @@ __device__ __forceinline__ void batch_solve_item(const BatchSpline* specs, const
         sp.bottom = b.bottom[a];
         sp.right = b.right[a];
         sp.lines_per_block = b.lines_per_block[a];
-        if constexpr (NT == kTileThreads) {
+        if constexpr (SEG) {
             sp.segs = b.segs[a];
             set_segment_params(b.seg[a], &sp);
         }
@@ -104,26 +112,26 @@ __device__ __forceinline__ void batch_solve_item(const BatchSpline* specs, const
             }
             sp.shift_last = b.shift[a];
         }
-        solve_tile<BW, CYC, double, double, merged_rows<BW, CYC, NT>(), NT == kTileThreads, false>(sp, w.first_line, tile_bytes, dst_base, src_base,
-                                                       static_cast<int>(threadIdx.x), NT);
-        return;
+        solve_tile<BW, CYC, double, double, merged_rows<BW, CYC, SEG>(), SEG, false>(
+            sp, w.first_line, tile_bytes, dst_base, src_base, static_cast<int>(threadIdx.x), NT);
+    } else {
+        // one line per lane, in place
+        const BatchSpline& b = specs[w.spline];
+        const int a = w.axis;
+        const int64_t n = b.ep.dim[a].n;
+        const int64_t line = w.first_line + threadIdx.x;
+        if (line >= b.total / n) return;
+        int64_t inner = 1;
+        for (int d = a + 1; d < b.dim; ++d) inner *= b.ep.dim[d].n;
+        SolveParams sp{};
+        sp.lower = b.lower[a];
+        sp.upper = b.upper[a];
+        sp.diag = b.diag[a];
+        sp.bottom = b.bottom[a];
+        sp.right = b.right[a];
+        const int64_t o = line / inner, ii = line - o * inner;
+        substitute<BW, CYC, double, double, kMergedRows>(ctrl + b.offset + o * n * inner + ii, inner, n, sp);
     }
-    // kSolveLanes: one line per lane, in place
-    const BatchSpline& b = specs[w.spline];
-    const int a = w.axis;
-    const int64_t n = b.ep.dim[a].n;
-    const int64_t line = w.first_line + threadIdx.x;
-    if (line >= b.total / n) return;
-    int64_t inner = 1;
-    for (int d = a + 1; d < b.dim; ++d) inner *= b.ep.dim[d].n;
-    SolveParams sp{};
-    sp.lower = b.lower[a];
-    sp.upper = b.upper[a];
-    sp.diag = b.diag[a];
-    sp.bottom = b.bottom[a];
-    sp.right = b.right[a];
-    const int64_t o = line / inner, ii = line - o * inner;
-    substitute<BW, CYC, double, double, kMergedRows>(ctrl + b.offset + o * n * inner + ii, inner, n, sp);
 }
 
 // One-dimensional splines: one spline per 64-thread workgroup, longest
@@ -403,26 +411,26 @@ __global__ __launch_bounds__(kLineThreads) void batch_line_split_kernel(const Ba
 #undef INTP_LINE_CASE
 }
 
-// One launch per pass: workgroup g solves items g, g + gridDim.x, ...
+// One launch per pass and form: workgroup g solves items g, g + gridDim.x, ...
 // (tiles of lines of one spline along one axis, of any band width; the
 // items are ordered longest line first, so the long sequential lines
 // start at once and the short tiles fill in around them).
-template <int NT>
-__global__ __launch_bounds__(NT, 2) void batch_solve_kernel(const BatchSpline* specs,
-                                                                   const BatchSolveItem* items, int32_t nitems,
-                                                                   const double* values, double* ctrl,
-                                                                   int32_t first_pass) {
+template <int NT, BatchSolveForm FORM>
+__global__ __launch_bounds__(NT, NT == kTileThreads && FORM != BatchSolveForm::kCut ? 1 : 2) void batch_solve_kernel(
+    const BatchSpline* specs, const BatchSolveItem* items, int32_t nitems, const double* values, double* ctrl,
+    int32_t first_pass) {
     extern __shared__ __align__(16) unsigned char tile_bytes[];
-    __shared__ int64_t dst_base[kMaxTileLines];
-    __shared__ int64_t src_base[kMaxTileLines];
+    constexpr int kBases = FORM == BatchSolveForm::kLanes ? 1 : kMaxTileLines;
+    __shared__ int64_t dst_base[kBases];
+    __shared__ int64_t src_base[kBases];
     for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
         const BatchSolveItem w = items[it];
 #define INTP_SOLVE_CASE(BW, CYC)                                                                                  \
     case 2 * BW + CYC:                                                                                            \
-        batch_solve_item<BW, CYC, NT>(specs, w, values, ctrl, first_pass, tile_bytes, dst_base, src_base);        \
+        batch_solve_item<BW, CYC, NT, FORM>(specs, w, values, ctrl, first_pass, tile_bytes, dst_base, src_base);  \
         break;
         // periodic band widths are floor(k/2) <= 3, clamped ones k - 1 <= 6
-        switch (w.kind & 15) {
+        switch (w.kind) {
             INTP_SOLVE_CASE(0, false)
             INTP_SOLVE_CASE(0, true)
             INTP_SOLVE_CASE(1, false)
@@ -446,13 +454,18 @@ constexpr int kEvalStreams = 4;
 // LDS budget of the tile of one solve workgroup (two per CU).
 constexpr int64_t kBatchTileBudget = kTileLdsBudget - kBatchStaticLds - kEdgeMax * 8;
 
-int64_t tile_fit(int64_t n, int64_t inner, int cap) {
+int64_t tile_fit(int64_t n, int64_t inner, int cap, int segs) {
     int lpb = kMaxTileLines;
-    while (lpb > 0 && (lpb > cap || tile_elements(n, lpb, inner, 1) * 8 > kBatchTileBudget)) lpb /= 2;
+    while (lpb > 0 && (lpb > cap || tile_elements(n, lpb, inner, segs) * 8 > kBatchTileBudget)) lpb /= 2;
     // one line may take most of a CU's LDS
-    if (lpb == 0 && tile_elements(n, 1, inner, 1) * 8 <= kBatchTileBudget + kLdsBytes - kTileLdsBudget) lpb = 1;
+    if (lpb == 0 && tile_elements(n, 1, inner, segs) * 8 <= kBatchTileBudget + kLdsBytes - kTileLdsBudget) lpb = 1;
     return lpb;
 }
+
+// Waves per CU, of one line per lane, that keep it busy; tiles per CU up to
+// which a pass's tiles are one launch.
+constexpr double kFullWaves = 2.0;
+constexpr int kMergeTilesPerCu = 16;
 
 // Elements of the staged edge factors of an axis (after the tile in LDS).
 int64_t edge_rows(const DimSetup& ds, int segs) {
@@ -464,9 +477,9 @@ int64_t edge_rows(const DimSetup& ds, int segs) {
 
 struct SolveGroup {
     int pass;
-    int64_t offset, count;
-    size_t lds;
-    int threads;  // kSmallSolveThreads, kMediumSolveThreads or kTileThreads
+    SolveClass cls;
+    int64_t offset = 0, count = 0;
+    size_t lds = 0;
 };
 
 struct EvalGroup {
@@ -476,7 +489,7 @@ struct EvalGroup {
 
 // Tunables (picked by the autotuner).
 struct Tuning {
-    int tile_cap = kTileLines;   // lines per solve tile, at most
+    int tile_cap = kMaxTileLines;  // lines per solve tile, at most
     int solve_blocks_per_cu = 4;  // persistent 256-thread solve workgroups per CU
     int eval_threads = 256;       // points per eval item (= workgroup size)
     int eval_blocks_per_cu = 8;   // persistent eval workgroups per CU
@@ -514,8 +527,8 @@ struct intp_batch_s {
     hipStream_t side = nullptr;        // runs the 1D splines beside the passes
     hipStream_t side2 = nullptr;       // the split 1D lines, beside both
     // a pass's solve groups run side by side: all but its last on these
-    hipStream_t solve_side[2] = {};
-    hipEvent_t solve_fork = nullptr, solve_join[2] = {};
+    hipStream_t solve_side[kSolveClasses - 1] = {};
+    hipEvent_t solve_fork = nullptr, solve_join[kSolveClasses - 1] = {};
     hipEvent_t fork = nullptr, join = nullptr, join2 = nullptr;
     // the (dimension, order) eval classes run side by side on these
     hipStream_t eval_side[kEvalStreams] = {};
@@ -558,7 +571,7 @@ struct intp_batch_s {
             (void)hipStreamSynchronize(side2);
             (void)hipStreamDestroy(side2);
         }
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < kSolveClasses - 1; ++i) {
             if (solve_side[i]) {
                 (void)hipStreamSynchronize(solve_side[i]);
                 (void)hipStreamDestroy(solve_side[i]);
@@ -590,52 +603,87 @@ void drop_graph(intp_batch b);
 // bakes in the work-item buffers and their contents, so it is dropped,
 // and the upload waits for every launch still reading the old items.
 int make_solve_work(intp_batch b, hipStream_t stream) {
-    // per spline tile sizes (tiles serve the axes with fewer than 64
-    // adjacent lines)
+    // per pass, waves per CU that solve its lines one per lane: the lines of
+    // strided axes (64 or more adjacent lines, [1]) and the others
+    double waves[2][kBatchDim] = {};
+    auto inner_of = [&](int s, int d) {
+        int64_t inner = 1;
+        for (int e = d + 1; e < b->dims[static_cast<size_t>(s)]; ++e)
+            inner *= b->setups[static_cast<size_t>(s) * kBatchDim + e].n;
+        return inner;
+    };
+    for (int s = 0; s < b->count; ++s) {
+        const int D = b->dims[static_cast<size_t>(s)];
+        for (int d = 0; D > 1 && d < D; ++d)
+            waves[inner_of(s, d) >= 64 ? 1 : 0][D - 1 - d] +=
+                static_cast<double>(b->host_specs[static_cast<size_t>(s)].total) /
+                (64.0 * b->num_cus * b->setups[static_cast<size_t>(s) * kBatchDim + d].n);
+    }
+    // Segments per line where they pay.  A cut line takes about its warm-up
+    // and one segment of its rows, but all four waves of its tile do, and
+    // data on which the segments do not meet are solved twice: where the
+    // pass's lines fill the chip, only contiguous lines are cut, from 2.5
+    // times that on, elsewhere all from 1.5 times on (us, noise / constant
+    // data, 2D of orders 1 to 5: 500 of 300..400 squared, cut from 2.5 1164 /
+    // 1679, from 4 1476 / 1659; 1500 of 128..160, from 2.5 557 / 675, from
+    // 1.3 581 / 724; all axes in tiles instead, cut or not, 2500 / 2600 and
+    // 784 / 852; 60 of 200..300 from 1.5 100 / 193, from 3 284 / 326).
+    bool any_cut[kBatchDim] = {};
     for (int s = 0; s < b->count; ++s) {
         BatchSpline& bs = b->host_specs[static_cast<size_t>(s)];
         const int D = b->dims[static_cast<size_t>(s)];
         for (int d = 0; d < D; ++d) {
-            int64_t inner = 1;
-            for (int e = d + 1; e < D; ++e) inner *= b->setups[static_cast<size_t>(s) * kBatchDim + e].n;
             const DimSetup& ds = b->setups[static_cast<size_t>(s) * kBatchDim + d];
-            // a 1D spline is a tile of its own; an axis with 64 or more
-            // adjacent lines and no room for four of them is solved in HBM
-            int64_t lpb = tile_fit(ds.n, inner, D == 1 ? 1 : b->tune.tile_cap);
-            if (D > 1 && inner >= 64 && lpb < 4) lpb = 0;
-            // segments where they pay: one lane of the 256-thread tile
-            // workgroup (of the 64-thread line workgroup) per segment and line
+            const int64_t inner = inner_of(s, d);
+            // one lane of the 256-thread tile workgroup (of the 64-thread
+            // line workgroup) per segment and line
+            const int lpb = tile_fit(ds.n, inner, D == 1 ? 1 : std::min(b->tune.tile_cap, kTileLines), 1);
+            bs.lines_per_block[d] = lpb;
             bs.segs[d] = 0;
-            if (lpb > 0 && ds.n >= kMinSegmentRows && (ds.lu.seg64.warm > 0 || ds.lu.p == 0) &&
-                (!ds.lu.cyclic || ds.n >= 2 * ds.lu.seg64.warm)) {
-                int64_t segs = D == 1 ? kLineThreads : kTileThreads / lpb;
-                while (segs > 1 && segs * 8 > ds.n) segs /= 2;
-                if (segs < ds.lu.p || 4 * (ds.lu.seg64.warm + ds.n / segs) > 3 * ds.n) segs = D == 1 ? 1 : 0;
-                bs.segs[d] = static_cast<int32_t>(segs);
-            }
-            if (lpb == 0 && inner < 64 && D > 1)
+            if (lpb < (D > 1 && inner >= 64 ? 4 : 1) || ds.n < kMinSegmentRows ||
+                (ds.lu.seg64.warm == 0 && ds.lu.p > 0) || (ds.lu.cyclic && ds.n < 2 * ds.lu.seg64.warm))
+                continue;
+            int64_t segs = D == 1 ? kLineThreads : kTileThreads / lpb;
+            while (segs > 1 && segs * 8 > ds.n) segs /= 2;
+            const bool full = D > 1 && waves[inner >= 64 ? 1 : 0][D - 1 - d] >= kFullWaves;
+            if (full && inner >= 64) continue;
+            const double factor = D == 1 ? 4.0 / 3 : full ? 2.5 : 1.5;
+            if (segs < ds.lu.p || factor * static_cast<double>(ds.lu.seg64.warm + ds.n / segs) > static_cast<double>(ds.n))
+                segs = D == 1 ? 1 : 0;
+            bs.segs[d] = static_cast<int32_t>(segs);
+            if (D > 1 && segs > 0) any_cut[D - 1 - d] = true;
+        }
+    }
+    // The other lines: tiles, and on strided axes one line per lane in HBM,
+    // whose loads are coalesced; where other lines of the pass are cut and
+    // the chip has room, in tiles as well, of the same launch.
+    for (int s = 0; s < b->count; ++s) {
+        BatchSpline& bs = b->host_specs[static_cast<size_t>(s)];
+        const int D = b->dims[static_cast<size_t>(s)];
+        for (int d = 0; D > 1 && d < D; ++d) {
+            if (bs.segs[d] > 0) continue;
+            const DimSetup& ds = b->setups[static_cast<size_t>(s) * kBatchDim + d];
+            const int64_t inner = inner_of(s, d);
+            int lpb = tile_fit(ds.n, inner, b->tune.tile_cap, 0);
+            if (inner >= 64 && (lpb < 4 || !any_cut[D - 1 - d] || waves[1][D - 1 - d] >= kFullWaves)) lpb = 0;
+            if (lpb == 0 && inner < 64)
                 return fail(INTP_E_UNSUPPORTED, "spline " + std::to_string(s) + ": line too long for a batch");
-            bs.lines_per_block[d] = static_cast<int32_t>(lpb);
+            bs.lines_per_block[d] = lpb;
         }
     }
     b->solve_host.clear();
     b->solve_groups.clear();
     // a workgroup's time is about its longest line times the work per row
     auto row_cost = [](const DimSetup& ds) { return int64_t{4} + ds.lu.p * (ds.lu.cyclic ? 4 : 2); };
-    auto kind_of = [](const DimSetup& ds, int mode) {
-        return static_cast<int16_t>((mode << 4) | (2 * ds.lu.p + (ds.lu.cyclic ? 1 : 0)));
+    auto kind_of = [](const DimSetup& ds) {
+        return static_cast<int16_t>(2 * ds.lu.p + (ds.lu.cyclic ? 1 : 0));
     };
-    // per pass: the large tiles with the in-place runs (256-thread
-    // workgroups), the medium tiles (two-wave workgroups) and the small
-    // tiles (one-wave workgroups), each longest first
-    std::vector<std::pair<int64_t, BatchSolveItem>> large_items, medium_items, small_items;
+    // per pass and class, longest first
+    std::vector<std::pair<int64_t, BatchSolveItem>> items[kSolveClasses];
     for (int pass = 0; pass < kBatchDim; ++pass) {
-        SolveGroup gl{pass, 0, 0, 0, kTileThreads};
-        SolveGroup gm{pass, 0, 0, 0, kMediumSolveThreads};
-        SolveGroup gs{pass, 0, 0, 0, kSmallSolveThreads};
-        large_items.clear();
-        medium_items.clear();
-        small_items.clear();
+        size_t lds[kSolveClasses] = {};
+        int64_t cut_lds[kSolveClasses] = {};
+        for (auto& i : items) i.clear();
         for (int s = 0; s < b->count; ++s) {
             const int D = b->dims[static_cast<size_t>(s)];
             if (D <= pass) continue;
@@ -656,28 +704,52 @@ int make_solve_work(intp_batch b, hipStream_t stream) {
                 continue;
             } else if (bs.lines_per_block[a] == 0) {
                 for (int64_t first = 0; first < nlines; first += kTileThreads)
-                    large_items.push_back(
-                        {cost, BatchSolveItem{s, static_cast<int16_t>(a), kind_of(ds, kSolveLanes), first}});
+                    items[kLanes].push_back({cost, BatchSolveItem{s, static_cast<int16_t>(a), kind_of(ds), first}});
             } else {
                 const int64_t lpb = bs.lines_per_block[a];
-                const int64_t bytes = (tile_elements(ds.n, lpb, inner, 1) + edge_rows(ds, bs.segs[a])) * 8;
-                // lines cut into segments keep every wave busy; the others one
-                const bool small = bytes <= kSmallTileBytes && bs.segs[a] == 0;
-                const bool medium = !small && bytes <= kMediumTileBytes && bs.segs[a] == 0;
-                auto& to_items = small ? small_items : medium ? medium_items : large_items;
+                const int64_t edges = edge_rows(ds, bs.segs[a]);
+                const int64_t bytes = (tile_elements(ds.n, lpb, inner, bs.segs[a]) + edges) * 8;
+                const SolveClass cls = bs.segs[a] > 0              ? kCutTiles
+                                       : bytes <= kSmallTileBytes  ? kSmallTiles
+                                       : bytes <= kMediumTileBytes ? kMediumTiles
+                                                                   : kLargeTiles;
                 for (int64_t first = 0; first < nlines; first += lpb)
-                    to_items.push_back({cost, BatchSolveItem{s, static_cast<int16_t>(a), kind_of(ds, kSolveTile), first}});
-                SolveGroup& to = small ? gs : medium ? gm : gl;
-                to.lds = std::max(to.lds, static_cast<size_t>(bytes));
+                    items[cls].push_back({cost, BatchSolveItem{s, static_cast<int16_t>(a), kind_of(ds), first}});
+                lds[cls] = std::max(lds[cls], static_cast<size_t>(bytes));
+                // of a launch that cuts lines, whose tiles have spare rows
+                cut_lds[cls] = std::max(cut_lds[cls], (tile_elements(ds.n, lpb, inner, 1) + edges) * 8);
             }
         }
-        for (auto* items : {&large_items, &medium_items, &small_items}) {
-            SolveGroup& grp = items == &large_items ? gl : items == &medium_items ? gm : gs;
-            std::stable_sort(items->begin(), items->end(),
+        // few tiles go into the class of the largest, which solves them all:
+        // a second launch costs more, with its fork and join, than workgroups
+        // of the right size save (us, 40 splines of 16..256 squared 234 in
+        // four launches a pass, 83; 4096 mixed ones, 20 to 40 tiles per CU,
+        // 1340 and 1660)
+        constexpr SolveClass kTiles[] = {kCutTiles, kLargeTiles, kMediumTiles, kSmallTiles};
+        size_t tiles = 0;
+        for (SolveClass c : kTiles) tiles += items[c].size();
+        if (tiles <= static_cast<size_t>(b->num_cus) * kMergeTilesPerCu) {
+            SolveClass to = kSolveClasses;
+            for (SolveClass c : kTiles) {
+                if (items[c].empty()) continue;
+                if (to == kSolveClasses) {
+                    to = c;
+                    continue;
+                }
+                if (to == kCutTiles && cut_lds[c] + kBatchStaticLds > kLdsBytes) continue;
+                items[to].insert(items[to].end(), items[c].begin(), items[c].end());
+                items[c].clear();
+                lds[to] = std::max(lds[to], to == kCutTiles ? static_cast<size_t>(cut_lds[c]) : lds[c]);
+            }
+        }
+        for (int cls = 0; cls < kSolveClasses; ++cls) {
+            std::stable_sort(items[cls].begin(), items[cls].end(),
                              [](const auto& x, const auto& y) { return x.first > y.first; });
+            SolveGroup grp{pass, static_cast<SolveClass>(cls)};
+            grp.lds = lds[cls];
             grp.offset = static_cast<int64_t>(b->solve_host.size());
-            for (const auto& pi : *items) b->solve_host.push_back(pi.second);
-            grp.count = static_cast<int64_t>(b->solve_host.size()) - grp.offset;
+            for (const auto& pi : items[cls]) b->solve_host.push_back(pi.second);
+            grp.count = static_cast<int64_t>(items[cls].size());
             if (grp.count > 0) b->solve_groups.push_back(grp);
         }
     }
@@ -838,34 +910,37 @@ int launch_build(intp_batch b, const double* values, hipStream_t stream, bool sp
         HIP_TRY(hipEventRecord(b->join, b->side), "hipEventRecord");
     }
     if (!b->solve_fork) {
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < kSolveClasses - 1; ++i) {
             HIP_TRY(hipStreamCreateWithFlags(&b->solve_side[i], hipStreamNonBlocking), "hipStreamCreate");
             HIP_TRY(hipEventCreateWithFlags(&b->solve_join[i], hipEventDisableTiming), "hipEventCreate");
         }
         HIP_TRY(hipEventCreateWithFlags(&b->solve_fork, hipEventDisableTiming), "hipEventCreate");
     }
+    // small tiles: one wave each, 8 resident per CU at 2 waves per SIMD;
+    // medium tiles: two waves each, 4 resident per CU
     auto launch_group = [&](const SolveGroup& g, hipStream_t s) -> hipError_t {
         const int32_t first_pass = g.pass == 0 ? 1 : 0;
-        if (g.threads == kSmallSolveThreads) {
-            // one wave each: 8 resident per CU at 2 waves per SIMD
-            const int blocks = static_cast<int>(std::min<int64_t>(g.count, int64_t{b->num_cus} * 16));
-            hipLaunchKernelGGL(batch_solve_kernel<kSmallSolveThreads>, dim3(static_cast<unsigned>(blocks)),
-                               dim3(kSmallSolveThreads), g.lds, s, b->specs, b->solve_items + g.offset,
-                               static_cast<int32_t>(g.count), values, b->ctrl, first_pass);
-        } else if (g.threads == kMediumSolveThreads) {
-            // two waves each: 4 resident per CU (LDS and 2 waves per SIMD)
-            const int blocks = static_cast<int>(std::min<int64_t>(g.count, int64_t{b->num_cus} * 8));
-            hipLaunchKernelGGL(batch_solve_kernel<kMediumSolveThreads>, dim3(static_cast<unsigned>(blocks)),
-                               dim3(kMediumSolveThreads), g.lds, s, b->specs, b->solve_items + g.offset,
-                               static_cast<int32_t>(g.count), values, b->ctrl, first_pass);
-        } else {
-            const int blocks =
-                static_cast<int>(std::min<int64_t>(g.count, int64_t{b->num_cus} * b->tune.solve_blocks_per_cu));
-            hipLaunchKernelGGL(batch_solve_kernel<kTileThreads>, dim3(static_cast<unsigned>(blocks)),
-                               dim3(kTileThreads), g.lds, s, b->specs, b->solve_items + g.offset,
-                               static_cast<int32_t>(g.count), values, b->ctrl, first_pass);
+        if (static_cast<int64_t>(g.lds) + kBatchStaticLds > kLdsBytes) return hipErrorInvalidValue;
+        auto launch = [&](auto kernel, int threads, int per_cu) {
+            const int blocks = static_cast<int>(std::min<int64_t>(g.count, int64_t{b->num_cus} * per_cu));
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(static_cast<unsigned>(threads)), g.lds,
+                               s, b->specs, b->solve_items + g.offset, static_cast<int32_t>(g.count), values, b->ctrl,
+                               first_pass);
+            return hipGetLastError();
+        };
+        constexpr BatchSolveForm kWhole = BatchSolveForm::kWhole;
+        switch (g.cls) {
+            case kSmallTiles: return launch(batch_solve_kernel<kSmallSolveThreads, kWhole>, kSmallSolveThreads, 16);
+            case kMediumTiles: return launch(batch_solve_kernel<kMediumSolveThreads, kWhole>, kMediumSolveThreads, 8);
+            case kLargeTiles:
+                return launch(batch_solve_kernel<kTileThreads, kWhole>, kTileThreads, b->tune.solve_blocks_per_cu);
+            case kCutTiles:
+                return launch(batch_solve_kernel<kTileThreads, BatchSolveForm::kCut>, kTileThreads,
+                              b->tune.solve_blocks_per_cu);
+            default:
+                return launch(batch_solve_kernel<kTileThreads, BatchSolveForm::kLanes>, kTileThreads,
+                              b->tune.solve_blocks_per_cu);
         }
-        return hipGetLastError();
     };
     // a pass's groups run side by side (a spline's lines along one axis
     // are all in one size class, so the groups touch different splines):
@@ -874,8 +949,8 @@ int launch_build(intp_batch b, const double* values, hipStream_t stream, bool sp
     for (size_t i = 0; i < b->solve_groups.size();) {
         size_t end = i + 1;
         while (end < b->solve_groups.size() && b->solve_groups[end].pass == b->solve_groups[i].pass) ++end;
-        const size_t nside = end - i - 1;  // at most 2: three size classes per pass
-        if (nside > 2) return fail(INTP_E_INVALID, "more solve groups in a pass than side streams");
+        const size_t nside = end - i - 1;  // at most one group per class
+        if (nside > kSolveClasses - 1) return fail(INTP_E_INVALID, "more solve groups in a pass than side streams");
         if (nside > 0) {
             HIP_TRY(hipEventRecord(b->solve_fork, stream), "hipEventRecord");
             for (size_t k = 0; k < nside; ++k) {
@@ -986,7 +1061,7 @@ int autotune(intp_batch b, const double* values, const double* coords, const int
     // the solve knobs dominate and interact: they are visited twice
     int rc;
     for (int round = 0; round < 2; ++round) {
-        if ((rc = try_values("tile_cap", &Tuning::tile_cap, {8, 16, 32})) != INTP_OK) return rc;
+        if ((rc = try_values("tile_cap", &Tuning::tile_cap, {8, 16, 32, 64})) != INTP_OK) return rc;
         if ((rc = try_values("solve_blocks_per_cu", &Tuning::solve_blocks_per_cu, {1, 2, 4, 8})) != INTP_OK) return rc;
         if (round == 0) {
             if ((rc = try_values("eval_threads", &Tuning::eval_threads, {64, 128, 256})) != INTP_OK) return rc;

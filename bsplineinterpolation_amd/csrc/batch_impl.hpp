@@ -39,15 +39,9 @@ struct BatchSpline {
     int32_t nseg;
 };
 
-// Work of one solve workgroup.  kind & 15 = 2 * band width + cyclic
-// selects the substitution; kind >> 4 the mode:
-//   kSolveTile: lines first_line .. of `spline` along `axis`, staged
-//     through LDS;
-//   kSolveLanes: 256 adjacent lines first_line .. of `spline` along a
-//     strided `axis` too long for a tile, one per lane, substituted in
-//     place.
-enum : int16_t { kSolveTile = 0, kSolveLanes = 1 };
-
+// Work of one solve workgroup: the lines first_line .. of `spline` along
+// `axis`, a tile of them or one per lane (the launch's form).  kind = 2 *
+// band width + cyclic selects the substitution.
 struct BatchSolveItem {
     int32_t spline;
     int16_t axis;

@@ -1,0 +1,91 @@
+"""How a batch's lines are solved (batch.hip): tiles in one launch or by size,
+lines cut into segments or whole, strided axes one line per lane.  Control
+points are those of single splines bit for bit on any data, and a few splines
+together cost about what the largest of them costs alone."""
+import random
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _specs(seed, count, dim, lo, hi, orders=(1, 5)):
+    rng = random.Random(seed)
+    return [dict(order=rng.randint(*orders), shape=tuple(rng.randint(lo, hi) for _ in range(dim)),
+                 periodic=[rng.random() < 0.3 for _ in range(dim)], ranges=[(0.0, 1.0)] * dim) for _ in range(count)]
+
+
+def _batches():
+    return {
+        "few_short": _specs(1, 12, 2, 16, 120),
+        "few_long": _specs(2, 10, 2, 280, 700),
+        "few_mixed": _specs(3, 40, 2, 16, 256, (1, 7)) + _specs(4, 6, 3, 8, 64),
+        "many_mixed": _specs(5, 1500, 2, 16, 256),       # above 16 tiles per CU: a launch per size
+        "many_long": _specs(6, 420, 2, 200, 420),        # strided lines fill the chip
+        "three": _specs(7, 40, 3, 12, 150),
+        "thin": _specs(8, 30, 2, 700, 1200, (2, 4)) + _specs(9, 30, 3, 8, 24, (6, 7)),
+        "unequal_lines": _specs(10, 300, 1, 16, 400) + [dict(order=k, shape=(n,), periodic=[p], ranges=[(0.0, 1.0)])
+                                                        for k, n, p in ((3, 9000, False), (5, 17000, False), (4, 6000, True),
+                                                                        (2, 30000, False))],
+    }
+
+
+def _data(kind, specs, total):
+    rng = np.random.default_rng(total)
+    if kind == "constant":
+        return np.full(total, 0.7372)
+    v = rng.standard_normal(total)
+    if kind == "zero_tail":
+        v[np.arange(total) % 400 >= 60] = 0.0
+    return v
+
+
+@pytest.mark.parametrize("name", ["few_short", "few_long", "few_mixed", "many_mixed", "many_long", "three", "thin",
+                                  "unequal_lines"])
+def test_gpu_batch_forms_equal_single_splines(name):
+    import torch
+    import bsplineinterpolation_amd as amd
+    specs = _batches()[name]
+    batch = amd.Batch(specs)
+    sizes = [int(np.prod(s["shape"])) for s in specs]
+    first = np.concatenate([[0], np.cumsum(sizes)])
+    sample = sorted({int(i) for i in np.linspace(0, len(specs) - 1, 24)} | {int(np.argmax(sizes)), int(np.argmin(sizes))})
+    for kind in ("noise", "constant", "zero_tail"):
+        v = _data(kind, specs, batch.total)
+        batch.build(torch.from_numpy(v).cuda())
+        torch.cuda.synchronize()
+        for s in sample:
+            spec = specs[s]
+            one = amd.InterpolationFunction(spec["order"], v[first[s]:first[s + 1]].reshape(spec["shape"]),
+                                            periodic=spec["periodic"], ranges=spec["ranges"])
+            assert np.array_equal(batch.control_points(s), one.control_points().ravel()), (kind, s, spec)
+
+
+def _microseconds(build):
+    import torch
+    best = float("inf")
+    for _ in range(20):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        build()
+        end.record()
+        torch.cuda.synchronize()
+        best = min(best, start.elapsed_time(end) * 1e3)
+    return best
+
+
+def test_gpu_batch_of_a_few_costs_its_largest():
+    """Forty splines are fewer tiles than the chip holds at once: beside the
+    longest line there is the start of the workgroups and the contention for
+    the caches, less than the line again."""
+    import torch
+    import bsplineinterpolation_amd as amd
+    specs = [dict(order=o, shape=(n, n + 4), periodic=[False] * 2, ranges=[(0.0, 1.0)] * 2)
+             for o in (2, 3, 4, 5) for n in range(30, 250, 22)]
+    many, one = amd.Batch(specs), amd.Batch([specs[-1]])
+    v = torch.randn(many.total, dtype=torch.float64, device="cuda")
+    w = v[:one.total].clone()
+    us, base = _microseconds(lambda: many.build(v)), _microseconds(lambda: one.build(w))
+    print("%d splines %.0f us, the largest %.0f us" % (len(specs), us, base), flush=True)
+    assert us <= 2.0 * base
