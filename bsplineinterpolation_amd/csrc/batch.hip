@@ -475,6 +475,14 @@ int64_t edge_rows(const DimSetup& ds, int segs) {
     return edge_elements(ds.n, ds.lu.p, sp);
 }
 
+// A run of list1d, solved by one launch; a launch allocates the LDS of its
+// longest line for every workgroup.
+constexpr int kLineClasses = 3;
+struct LineGroup {
+    int64_t offset, count;
+    size_t lds;
+};
+
 struct SolveGroup {
     int pass;
     SolveClass cls;
@@ -519,7 +527,10 @@ struct intp_batch_s {
     int64_t solve_cap = 0;
     std::vector<int32_t> list1d_host;  // the 1D splines, longest first
     int32_t* list1d = nullptr;
-    size_t line_lds = 0;               // LDS of batch_line_kernel
+    // batch_line_kernel's launches, without and with lines split
+    std::vector<LineGroup> line_groups[2];
+    hipStream_t line_side[kLineClasses - 1] = {};  // all but the first launch on these
+    hipEvent_t line_join[kLineClasses - 1] = {};
     double* split_tables = nullptr;    // segment responses of the split 1D lines
     std::vector<int32_t> split_host;   // the split lines, longest first
     int32_t* split_list = nullptr;
@@ -571,6 +582,13 @@ struct intp_batch_s {
             (void)hipStreamSynchronize(side2);
             (void)hipStreamDestroy(side2);
         }
+        for (int i = 0; i < kLineClasses - 1; ++i) {
+            if (line_side[i]) {
+                (void)hipStreamSynchronize(line_side[i]);
+                (void)hipStreamDestroy(line_side[i]);
+            }
+            if (line_join[i]) (void)hipEventDestroy(line_join[i]);
+        }
         for (int i = 0; i < kSolveClasses - 1; ++i) {
             if (solve_side[i]) {
                 (void)hipStreamSynchronize(solve_side[i]);
@@ -597,6 +615,44 @@ struct intp_batch_s {
 namespace {
 
 void drop_graph(intp_batch b);
+
+// The launches of the 1D lines: up to three, by the workgroups per CU that
+// their LDS admits (registers admit eight), where one with the longest
+// line's LDS would take the lines in more than four turns (us, in one launch
+// and now: 8000 lines of 50 to 500 rows and one of 18,900 508 and 127, 60,000
+// and one 3825 and 669; in fewer turns the launches cost more than they give,
+// 1000 lines and one of 9000 79 and 89).
+void make_line_groups(intp_batch b, bool split) {
+    constexpr int64_t kLdsPerClass[kLineClasses - 1] = {kLdsBytes / 3, kLdsBytes / 8};
+    const auto& list = b->list1d_host;
+    auto& groups = b->line_groups[split ? 1 : 0];
+    groups.clear();
+    std::vector<int64_t> lds(list.size() + 1, 0);  // of this line and all after it
+    int64_t start = 0, end = static_cast<int64_t>(list.size());
+    for (int64_t i = end - 1; i >= 0; --i) {
+        const size_t s = static_cast<size_t>(list[static_cast<size_t>(i)]);
+        const BatchSpline& bs = b->host_specs[s];
+        const DimSetup& ds = b->setups[s * kBatchDim];
+        const bool skipped = split && bs.nseg > 0;
+        const int64_t need = skipped || bs.lines_per_block[0] == 0
+                                 ? 0
+                                 : (tile_elements(ds.n, 1, 1, 1) + edge_rows(ds, bs.segs[0])) * 8 + kBatchStaticLds;
+        lds[static_cast<size_t>(i)] = std::max(lds[static_cast<size_t>(i) + 1], need);
+    }
+    while (start < end && split && b->host_specs[static_cast<size_t>(list[static_cast<size_t>(start)])].nseg > 0) ++start;
+    for (int c = 0; c < kLineClasses && start < end; ++c) {
+        int64_t stop = end;
+        const int64_t most = lds[static_cast<size_t>(start)];
+        const bool few = most == 0 || end - start <= 4 * b->num_cus * std::min<int64_t>(8, kLdsBytes / most);
+        if (c < kLineClasses - 1 && !few) {
+            stop = start;
+            while (stop < end && lds[static_cast<size_t>(stop)] > kLdsPerClass[c]) ++stop;
+        }
+        if (stop > start)
+            groups.push_back({start, stop - start, static_cast<size_t>(std::max<int64_t>(0, most - kBatchStaticLds))});
+        start = stop;
+    }
+}
 
 // (Re)builds the solve work items for the current tuning; uploads them on
 // `stream` (the host copy stays alive in the batch).  A captured graph
@@ -697,11 +753,7 @@ int make_solve_work(intp_batch b, hipStream_t stream) {
             for (int d = a + 1; d < D; ++d) inner *= b->setups[static_cast<size_t>(s) * kBatchDim + d].n;
             const int64_t cost = ds.n * row_cost(ds);
             if (D == 1) {
-                // batch_line_kernel, beside the passes
-                if (bs.lines_per_block[0] > 0)
-                    b->line_lds = std::max(b->line_lds, static_cast<size_t>((tile_elements(ds.n, 1, 1, 1) +
-                                                                             edge_rows(ds, bs.segs[0])) * 8));
-                continue;
+                continue;  // batch_line_kernel, beside the passes
             } else if (bs.lines_per_block[a] == 0) {
                 for (int64_t first = 0; first < nlines; first += kTileThreads)
                     items[kLanes].push_back({cost, BatchSolveItem{s, static_cast<int16_t>(a), kind_of(ds), first}});
@@ -753,6 +805,8 @@ int make_solve_work(intp_batch b, hipStream_t stream) {
             if (grp.count > 0) b->solve_groups.push_back(grp);
         }
     }
+    make_line_groups(b, false);
+    if (b->split_ready) make_line_groups(b, true);
     drop_graph(b);
     b->uses.order_before(stream);
     const int64_t need = std::max<int64_t>(1, static_cast<int64_t>(b->solve_host.size()));
@@ -887,6 +941,7 @@ int prepare_split(intp_batch b, hipStream_t stream) {
         HIP_TRY(hipStreamSynchronize(stream), "hipStreamSynchronize");
     }
     b->split_ready = true;
+    make_line_groups(b, true);
     return INTP_OK;
 }
 
@@ -904,9 +959,16 @@ int launch_build(intp_batch b, const double* values, hipStream_t stream, bool sp
             HIP_TRY(hipGetLastError(), "batch split line launch");
             HIP_TRY(hipEventRecord(b->join2, b->side2), "hipEventRecord");
         }
-        hipLaunchKernelGGL(batch_line_kernel, dim3(static_cast<unsigned>(b->list1d_host.size())), dim3(kLineThreads),
-                           b->line_lds, b->side, b->specs, b->list1d, values, b->ctrl, seg ? 1 : 0);
-        HIP_TRY(hipGetLastError(), "batch line launch");
+        const auto& groups = b->line_groups[seg ? 1 : 0];
+        for (size_t i = 0; i < groups.size(); ++i) {
+            const LineGroup& g = groups[i];
+            hipStream_t s = i == 0 ? b->side : b->line_side[i - 1];
+            if (i > 0) HIP_TRY(hipStreamWaitEvent(s, b->fork, 0), "hipStreamWaitEvent");
+            hipLaunchKernelGGL(batch_line_kernel, dim3(static_cast<unsigned>(g.count)), dim3(kLineThreads), g.lds, s,
+                               b->specs, b->list1d + g.offset, values, b->ctrl, seg ? 1 : 0);
+            HIP_TRY(hipGetLastError(), "batch line launch");
+            if (i > 0) HIP_TRY(hipEventRecord(b->line_join[i - 1], s), "hipEventRecord");
+        }
         HIP_TRY(hipEventRecord(b->join, b->side), "hipEventRecord");
     }
     if (!b->solve_fork) {
@@ -963,7 +1025,12 @@ int launch_build(intp_batch b, const double* values, hipStream_t stream, bool sp
         for (size_t k = 0; k < nside; ++k) HIP_TRY(hipStreamWaitEvent(stream, b->solve_join[k], 0), "hipStreamWaitEvent");
         i = end;
     }
-    if (lines) HIP_TRY(hipStreamWaitEvent(stream, b->join, 0), "hipStreamWaitEvent");
+    if (lines) {
+        HIP_TRY(hipStreamWaitEvent(stream, b->join, 0), "hipStreamWaitEvent");
+        const size_t launches = b->line_groups[split && !b->split_host.empty() ? 1 : 0].size();
+        for (size_t i = 1; i < launches; ++i)
+            HIP_TRY(hipStreamWaitEvent(stream, b->line_join[i - 1], 0), "hipStreamWaitEvent");
+    }
     if (lines && split && !b->split_host.empty()) HIP_TRY(hipStreamWaitEvent(stream, b->join2, 0), "hipStreamWaitEvent");
     return INTP_OK;
 }
@@ -1246,6 +1313,10 @@ int intp_batch_create(intp_ctx ctx_, int32_t count, const intp_grid_desc* descs,
         HIP_TRY(hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking), "hipStreamCreate");
         HIP_TRY(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming), "hipEventCreate");
         HIP_TRY(hipEventCreateWithFlags(&b->join, hipEventDisableTiming), "hipEventCreate");
+        for (int i = 0; i < kLineClasses - 1; ++i) {
+            HIP_TRY(hipStreamCreateWithFlags(&b->line_side[i], hipStreamNonBlocking), "hipStreamCreate");
+            HIP_TRY(hipEventCreateWithFlags(&b->line_join[i], hipEventDisableTiming), "hipEventCreate");
+        }
         HIP_TRY(hipStreamCreateWithFlags(&b->side2, hipStreamNonBlocking), "hipStreamCreate");
         HIP_TRY(hipEventCreateWithFlags(&b->join2, hipEventDisableTiming), "hipEventCreate");
     }

@@ -25,6 +25,8 @@ def _batches():
         "many_long": _specs(6, 420, 2, 200, 420),        # strided lines fill the chip
         "three": _specs(7, 40, 3, 12, 150),
         "thin": _specs(8, 30, 2, 700, 1200, (2, 4)) + _specs(9, 30, 3, 8, 24, (6, 7)),
+        "many_unequal_lines": _specs(11, 6000, 1, 16, 500) + [dict(order=3, shape=(n,), periodic=[False], ranges=[(0.0, 1.0)])
+                                                              for n in (3000, 5000, 9000, 17000)],
         "unequal_lines": _specs(10, 300, 1, 16, 400) + [dict(order=k, shape=(n,), periodic=[p], ranges=[(0.0, 1.0)])
                                                         for k, n, p in ((3, 9000, False), (5, 17000, False), (4, 6000, True),
                                                                         (2, 30000, False))],
@@ -42,7 +44,7 @@ def _data(kind, specs, total):
 
 
 @pytest.mark.parametrize("name", ["few_short", "few_long", "few_mixed", "many_mixed", "many_long", "three", "thin",
-                                  "unequal_lines"])
+                                  "unequal_lines", "many_unequal_lines"])
 def test_gpu_batch_forms_equal_single_splines(name):
     import torch
     import bsplineinterpolation_amd as amd
@@ -89,3 +91,19 @@ def test_gpu_batch_of_a_few_costs_its_largest():
     us, base = _microseconds(lambda: many.build(v)), _microseconds(lambda: one.build(w))
     print("%d splines %.0f us, the largest %.0f us" % (len(specs), us, base), flush=True)
     assert us <= 2.0 * base
+
+
+def test_gpu_batch_long_line_beside_short_ones():
+    """A launch that gives every line the LDS of the longest holds few at a
+    time; side by side they take no longer than one after the other."""
+    import torch
+    import bsplineinterpolation_amd as amd
+    long = dict(order=3, shape=(18000,), periodic=[False], ranges=[(0.0, 1.0)])
+    short = _specs(12, 8000, 1, 50, 500)
+    us = []
+    for specs in ([long], short, short + [long]):
+        batch = amd.Batch(specs)
+        v = torch.randn(batch.total, dtype=torch.float64, device="cuda")
+        us.append(_microseconds(lambda: batch.build(v)))
+    print("long %.0f us, short %.0f us, together %.0f us" % tuple(us), flush=True)
+    assert us[2] <= us[0] + us[1]
