@@ -49,6 +49,12 @@ template <int BW, bool CYC, bool SEG>
 constexpr int merged_rows() {
     return SEG && BW * (CYC ? 2 : 1) >= 4 ? 2 : kMergedRows;
 }
+// a 1D line that is solved in one piece is one lane's chain: more rows
+// between the checks of the division
+template <int BW, bool CYC>
+constexpr int line_rows() {
+    return BW * (CYC ? 2 : 1) <= 2 ? 8 : kMergedRows;
+}
 // Small tiles (at most kSmallTileBytes of LDS) are solved by one-wave
 // workgroups, so that every resident wave substitutes a tile of its own
 // (a 256-thread workgroup has one substituting wave and three waiting at
@@ -161,7 +167,7 @@ __device__ __forceinline__ void batch_line(const BatchSpline& b, const double* v
         sp.lines_per_block = 1;
         sp.segs = b.segs[0];
         set_segment_params(b.seg[0], &sp);
-        solve_tile<BW, CYC, double, double, kMergedRows, true, false>(sp, 0, tile_bytes, dst_base, src_base,
+        solve_tile<BW, CYC, double, double, line_rows<BW, CYC>(), true, false, true>(sp, 0, tile_bytes, dst_base, src_base,
                                                          static_cast<int>(threadIdx.x), kLineThreads);
         return;
     }

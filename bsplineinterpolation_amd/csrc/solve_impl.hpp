@@ -819,9 +819,10 @@ __device__ __forceinline__ bool solve_segments(const SolveParams& sp, C* tile, i
 // neighbouring workgroups on a CU then use different SIMDs).
 // SEG false: plain substitution (sp.segs 0), without the segments' pad rows.
 // SEG true with sp.segs 0 (the batch's 256-thread kernel): plain, with them.  FIXED: with a copy of the
-// segment code for the row stride kTileStep.
+// segment code for the row stride kTileStep.  ONE: lines of known pivots that
+// fail are solved as one segment at any band width.
 template <int BW, bool CYC, typename T, typename C, int B = batch_rows<BW, CYC>(), bool SEG = true,
-          bool FIXED = true>
+          bool FIXED = true, bool ONE = false>
 __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first, unsigned char* tile_bytes,
                                            int64_t* dst_base, int64_t* src_base, int tid, int NT) {
     const int lpb = sp.lines_per_block;
@@ -956,7 +957,7 @@ __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first,
         // segmented; then, if a comparison failed, in one piece: as one
         // segment, which has nothing to compare, or plainly where the rows of
         // equal factors do not make up for its steps (plan_tile)
-        const bool one = CYC || (sp.fast_divide && BW <= 2);
+        const bool one = CYC || (sp.fast_divide && (BW <= 2 || ONE));
 #pragma unroll 1
         for (int segs = sp.segs; segs > 0 && !done; segs = segs > 1 && one ? 1 : 0) {
             // the usual row stride of many lines as a constant: row offsets
