@@ -58,8 +58,8 @@ constexpr int line_rows() {
 // Small tiles (at most kSmallTileBytes of LDS) are solved by one-wave
 // workgroups, so that every resident wave substitutes a tile of its own
 // (a 256-thread workgroup has one substituting wave and three waiting at
-// the barrier); larger tiles and the in-place runs keep 256 threads, whose
-// four waves share the loads and stores of a large tile.
+// the barrier); larger tiles keep 256 threads, whose four waves share their
+// loads and stores.
 constexpr int kSmallSolveThreads = 64;
 constexpr int64_t kSmallTileBytes = 20 * 1024;
 // Medium tiles (at most kMediumTileBytes: with the 1 KB of line bases,

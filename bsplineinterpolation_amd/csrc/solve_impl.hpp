@@ -3,12 +3,13 @@
 // is an independent band (or cyclic band) system sharing one LU
 // factorization (InterpolationTemplate.hpp:448-580).
 //
-// solve_tile: a workgroup copies up to 32 lines into LDS with coalesced
-// loads, substitutes them there, each line cut into segments of one lane
+// solve_tile: a workgroup copies up to 64 lines into LDS with coalesced
+// loads, substitutes them there, whole or cut into segments of one lane
 // each (solve_segments), and writes the tile back.  The first pass reads
 // the caller's values with the periodic index shift applied
 // (InterpolationTemplate.hpp:452-462), so no separate copy precedes it.
-// Lines too long for LDS are cut into chunks first (solve_long.hip).
+// Lines too long for LDS are cut into chunks first (solve_long.hip); strided
+// axes with many lines are substituted in HBM, one line per lane.
 //
 // What bounds it.  Substituting a line is a chain of dependent rows: 16
 // cycles forward (order 3), and backward 16 and an IEEE division of 70.
@@ -17,11 +18,11 @@
 // lanes or more on a line; the division by a pivot that repeats takes two
 // operations (KnownDivisor); rows whose factors repeat take them from
 // scalar registers.  Whole solves, before -> after:
-//   1D 8192 cubic 643 -> 49 us (clamped), order 6 periodic FP32 storage,
-//   two solves, 3314 -> 199 us; 2D 1021 x 769 order 5 364 -> 74 us, 2000^2
-//   cubic 655 -> 80 us; 3D 128^3 cubic 100 -> 70 us, 256^3 cubic 300 -> 273
-//   us (one axis 76 to 100 us, of which copying the tile in and out is 44,
-//   6.1 TB/s).
+//   1D 8192 cubic 643 -> 50 us (clamped), order 6 periodic FP32 storage,
+//   two solves, 3314 -> 199 us; 2D 1021 x 769 order 5 364 -> 72 us, 2000^2
+//   cubic 655 -> 83 us; 3D 128^3 cubic 102 -> 81 us, 256^3 cubic 300 -> 256
+//   us (the contiguous axis 101 us, of which copying the tile in and out is
+//   44, 6.1 TB/s; the strided ones 75 us each in place).
 //
 // The substitution is the reference's (BandLU.hpp:121-143, 216-259)
 // reordered by rows: each entry receives the same updates in the same

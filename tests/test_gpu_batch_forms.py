@@ -107,3 +107,28 @@ def test_gpu_batch_long_line_beside_short_ones():
         us.append(_microseconds(lambda: batch.build(v)))
     print("long %.0f us, short %.0f us, together %.0f us" % tuple(us), flush=True)
     assert us[2] <= us[0] + us[1]
+
+
+def test_gpu_batch_forms_in_a_graph():
+    """The launches side by side, captured and replayed with other values,
+    with split lines and without."""
+    import torch
+    import bsplineinterpolation_amd as amd
+    specs = _specs(13, 6000, 1, 50, 400) + [dict(order=3, shape=(n,), periodic=[False], ranges=[(0.0, 1.0)])
+                                            for n in (9000, 3000)] + _specs(14, 200, 2, 16, 300) + _specs(15, 10, 3, 8, 90)
+    batch, rng = amd.Batch(specs), np.random.default_rng(3)
+    q = 8
+    po = np.arange(len(specs) + 1) * q
+    pts = torch.from_numpy(rng.random((q * len(specs), 3)) * 0.999).cuda()
+    vals = torch.from_numpy(rng.standard_normal(batch.total)).cuda()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        for split in (False, True):
+            plain = batch.run(vals, pts, po, split_lines=split).clone()
+            out = torch.empty_like(plain)
+            for scale in (1.0, 2.0, 0.5):  # exact scalings
+                torch.mul(vals, scale, out=vals)
+                torch.mul(plain, scale, out=plain)
+                batch.run(vals, pts, po, out=out, graph=True, split_lines=split)
+                stream.synchronize()
+                assert torch.equal(out, plain), (split, scale)
