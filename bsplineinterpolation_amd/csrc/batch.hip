@@ -78,8 +78,9 @@ constexpr int64_t kSplitMinRows = 256;
 // segments, in LDS tiles, or one line per lane in HBM.
 enum class BatchSolveForm { kWhole, kCut, kLanes };
 
-// Launches of a pass, each with items of one class.
-enum SolveClass { kCutTiles, kLargeTiles, kLanes, kMediumTiles, kSmallTiles, kSolveClasses };
+// Launches of a pass, each with items of one class (kLongTiles: one line takes
+// more than half of a CU's LDS).
+enum SolveClass { kLongTiles, kCutTiles, kLargeTiles, kLanes, kMediumTiles, kSmallTiles, kSolveClasses };
 
 template <int BW, bool CYC, int NT, BatchSolveForm FORM>
 __device__ __forceinline__ void batch_solve_item(const BatchSpline* specs, const BatchSolveItem& w, const double* values, double* ctrl,
@@ -767,15 +768,17 @@ int make_solve_work(intp_batch b, hipStream_t stream) {
                 const int64_t lpb = bs.lines_per_block[a];
                 const int64_t edges = edge_rows(ds, bs.segs[a]);
                 const int64_t bytes = (tile_elements(ds.n, lpb, inner, bs.segs[a]) + edges) * 8;
-                const SolveClass cls = bs.segs[a] > 0              ? kCutTiles
+                // of a launch that cuts lines, whose tiles have spare rows
+                const int64_t cut_bytes = (tile_elements(ds.n, lpb, inner, 1) + edges) * 8;
+                const SolveClass cls = bytes > kTileLdsBudget - kBatchStaticLds ? kLongTiles
+                                       : bs.segs[a] > 0              ? kCutTiles
                                        : bytes <= kSmallTileBytes  ? kSmallTiles
                                        : bytes <= kMediumTileBytes ? kMediumTiles
                                                                    : kLargeTiles;
                 for (int64_t first = 0; first < nlines; first += lpb)
                     items[cls].push_back({cost, BatchSolveItem{s, static_cast<int16_t>(a), kind_of(ds), first}});
-                lds[cls] = std::max(lds[cls], static_cast<size_t>(bytes));
-                // of a launch that cuts lines, whose tiles have spare rows
-                cut_lds[cls] = std::max(cut_lds[cls], (tile_elements(ds.n, lpb, inner, 1) + edges) * 8);
+                lds[cls] = std::max(lds[cls], static_cast<size_t>(cls == kLongTiles ? cut_bytes : bytes));
+                cut_lds[cls] = std::max(cut_lds[cls], cut_bytes);
             }
         }
         // few tiles go into the class of the largest, which solves them all:
@@ -783,21 +786,22 @@ int make_solve_work(intp_batch b, hipStream_t stream) {
         // of the right size save (us, 40 splines of 16..256 squared 234 in
         // four launches a pass, 83; 4096 mixed ones, 20 to 40 tiles per CU,
         // 1340 and 1660)
-        constexpr SolveClass kTiles[] = {kCutTiles, kLargeTiles, kMediumTiles, kSmallTiles};
+        // (beside long tiles one per CU has room)
+        constexpr SolveClass kTiles[] = {kLongTiles, kCutTiles, kLargeTiles, kMediumTiles, kSmallTiles};
         size_t tiles = 0;
         for (SolveClass c : kTiles) tiles += items[c].size();
         if (tiles <= static_cast<size_t>(b->num_cus) * kMergeTilesPerCu) {
             SolveClass to = kSolveClasses;
             for (SolveClass c : kTiles) {
-                if (items[c].empty()) continue;
+                if (items[c].empty() || (c == kLongTiles && tiles > static_cast<size_t>(b->num_cus))) continue;
                 if (to == kSolveClasses) {
                     to = c;
                     continue;
                 }
-                if (to == kCutTiles && cut_lds[c] + kBatchStaticLds > kLdsBytes) continue;
+                if (to <= kCutTiles && cut_lds[c] + kBatchStaticLds > kLdsBytes) continue;
                 items[to].insert(items[to].end(), items[c].begin(), items[c].end());
                 items[c].clear();
-                lds[to] = std::max(lds[to], to == kCutTiles ? static_cast<size_t>(cut_lds[c]) : lds[c]);
+                lds[to] = std::max(lds[to], to <= kCutTiles ? static_cast<size_t>(cut_lds[c]) : lds[c]);
             }
         }
         for (int cls = 0; cls < kSolveClasses; ++cls) {
@@ -1002,6 +1006,7 @@ int launch_build(intp_batch b, const double* values, hipStream_t stream, bool sp
             case kMediumTiles: return launch(batch_solve_kernel<kMediumSolveThreads, kWhole>, kMediumSolveThreads, 8);
             case kLargeTiles:
                 return launch(batch_solve_kernel<kTileThreads, kWhole>, kTileThreads, b->tune.solve_blocks_per_cu);
+            case kLongTiles:
             case kCutTiles:
                 return launch(batch_solve_kernel<kTileThreads, BatchSolveForm::kCut>, kTileThreads,
                               b->tune.solve_blocks_per_cu);

@@ -279,17 +279,16 @@ __device__ __forceinline__ void substitute(P* __restrict__ x, int64_t step, int6
     backward_range<BW, CYC, C, P, B>(x, step, n, 0, n, sp, st, z);
 }
 
-// A launch of a few long lines (a long 1D spline, say) substitutes each
+// A launch of a few long lines (lines beyond a tile whose factors fade too
+// slowly to be cut, or without room for the chunks' table) substitutes each
 // line with one lane whose factor loads run one batch of rows ahead: from
 // HBM every batch would wait a full memory latency.  When the launch has
 // at most kWarmLines lines and the factors fit kWarmBytes, every thread of
 // the workgroup first reads the factor arrays once (one 4-byte word per
-// 64 bytes), so that the substitution finds them in L2.  The arithmetic is
-// unchanged.
+// 64 bytes), so that the substitution finds them in L2, or past its 4 MB in
+// the device's last-level cache (one cubic line of 100,000 rows: 12.8 ms at
+// a limit of 2 MB, 12.0).  The arithmetic is unchanged.
 constexpr int64_t kWarmLines = 8;
-// 32 MB: past the 4 MB L2 of an XCD the factors still land in the
-// device's last-level cache (1D n = 100,000 cubic: 12.8 -> 12.0 ms
-// against a 2 MB limit; n <= 20,000 unchanged).
 constexpr int64_t kWarmBytes = int64_t{32} << 20;
 
 template <int BW, bool CYC, typename C, int NT>

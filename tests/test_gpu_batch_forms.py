@@ -24,6 +24,8 @@ def _batches():
         "many_mixed": _specs(5, 1500, 2, 16, 256),       # above 16 tiles per CU: a launch per size
         "many_long": _specs(6, 420, 2, 200, 420),        # strided lines fill the chip
         "three": _specs(7, 40, 3, 12, 150),
+        "one_long_axis": _specs(16, 300, 2, 16, 160) + [dict(order=k, shape=shape, periodic=[False] * 2, ranges=[(0.0, 1.0)] * 2)
+                                                        for k, shape in ((3, (9, 15000)), (4, (12000, 5)), (5, (14000, 40)))],
         "thin": _specs(8, 30, 2, 700, 1200, (2, 4)) + _specs(9, 30, 3, 8, 24, (6, 7)),
         "many_unequal_lines": _specs(11, 6000, 1, 16, 500) + [dict(order=3, shape=(n,), periodic=[False], ranges=[(0.0, 1.0)])
                                                               for n in (3000, 5000, 9000, 17000)],
@@ -43,7 +45,7 @@ def _data(kind, specs, total):
     return v
 
 
-@pytest.mark.parametrize("name", ["few_short", "few_long", "few_mixed", "many_mixed", "many_long", "three", "thin",
+@pytest.mark.parametrize("name", ["few_short", "few_long", "few_mixed", "many_mixed", "many_long", "three", "thin", "one_long_axis",
                                   "unequal_lines", "many_unequal_lines"])
 def test_gpu_batch_forms_equal_single_splines(name):
     import torch
@@ -132,3 +134,18 @@ def test_gpu_batch_forms_in_a_graph():
                 batch.run(vals, pts, po, out=out, graph=True, split_lines=split)
                 stream.synchronize()
                 assert torch.equal(out, plain), (split, scale)
+
+
+def test_gpu_batch_long_axis_beside_short_ones():
+    """As above, for the tiles of a pass."""
+    import torch
+    import bsplineinterpolation_amd as amd
+    long = dict(order=3, shape=(4, 15000), periodic=[False] * 2, ranges=[(0.0, 1.0)] * 2)
+    short = _specs(17, 1500, 2, 128, 160)
+    us = []
+    for specs in ([long], short, short + [long]):
+        batch = amd.Batch(specs)
+        v = torch.randn(batch.total, dtype=torch.float64, device="cuda")
+        us.append(_microseconds(lambda: batch.build(v)))
+    print("long %.0f us, short %.0f us, together %.0f us" % tuple(us), flush=True)
+    assert us[2] <= us[0] + us[1]
