@@ -84,8 +84,8 @@ enum SolveClass { kLongTiles, kCutTiles, kLargeTiles, kLanes, kMediumTiles, kSma
 
 template <int BW, bool CYC, int NT, BatchSolveForm FORM>
 __device__ __forceinline__ void batch_solve_item(const BatchSpline* specs, const BatchSolveItem& w, const double* values, double* ctrl,
-                                                 int32_t first_pass, unsigned char* tile_bytes, int64_t* dst_base,
-                                                 int64_t* src_base) {
+                                                 int32_t first_pass, unsigned char* tile_bytes,
+                                                 int64_t* line_base) {
     if constexpr (FORM != BatchSolveForm::kLanes) {
         constexpr bool SEG = FORM == BatchSolveForm::kCut;
         const BatchSpline& b = specs[w.spline];
@@ -120,7 +120,7 @@ __device__ __forceinline__ void batch_solve_item(const BatchSpline* specs, const
             sp.shift_last = b.shift[a];
         }
         solve_tile<BW, CYC, double, double, merged_rows<BW, CYC, SEG>(), SEG, false>(
-            sp, w.first_line, tile_bytes, dst_base, src_base, static_cast<int>(threadIdx.x), NT);
+            sp, w.first_line, tile_bytes, line_base, static_cast<int>(threadIdx.x), NT);
     } else {
         // one line per lane, in place
         const BatchSpline& b = specs[w.spline];
@@ -148,7 +148,7 @@ __device__ __forceinline__ void batch_solve_item(const BatchSpline* specs, const
 // multi-dimensional splines.
 template <int BW, bool CYC>
 __device__ __forceinline__ void batch_line(const BatchSpline& b, const double* values, double* ctrl,
-                                           unsigned char* tile_bytes, int64_t* dst_base, int64_t* src_base) {
+                                           unsigned char* tile_bytes, int64_t* line_base) {
     const int64_t n = b.ep.dim[0].n, shift = b.shift[0];
     double* x = ctrl + b.offset;
     const double* f = values + b.offset;
@@ -168,7 +168,7 @@ __device__ __forceinline__ void batch_line(const BatchSpline& b, const double* v
         sp.lines_per_block = 1;
         sp.segs = b.segs[0];
         set_segment_params(b.seg[0], &sp);
-        solve_tile<BW, CYC, double, double, line_rows<BW, CYC>(), true, false, true>(sp, 0, tile_bytes, dst_base, src_base,
+        solve_tile<BW, CYC, double, double, line_rows<BW, CYC>(), true, false, true>(sp, 0, tile_bytes, line_base,
                                                          static_cast<int>(threadIdx.x), kLineThreads);
         return;
     }
@@ -367,14 +367,13 @@ __global__ __launch_bounds__(kLineThreads, 2) void batch_line_kernel(const Batch
                                                                   const double* values, double* ctrl,
                                                                   int32_t skip_split) {
     extern __shared__ __align__(16) unsigned char tile_bytes[];
-    __shared__ int64_t dst_base[kMaxTileLines];
-    __shared__ int64_t src_base[kMaxTileLines];
+    __shared__ int64_t line_base[kMaxTileLines];
     const BatchSpline& b = specs[list1d[blockIdx.x]];
     if (skip_split && b.nseg > 0) return;
     const int kind = 2 * b.band[0] + (b.ep.dim[0].periodic ? 1 : 0);
 #define INTP_LINE_CASE(BW, CYC) \
     case 2 * BW + CYC:          \
-        batch_line<BW, CYC>(b, values, ctrl, tile_bytes, dst_base, src_base); \
+        batch_line<BW, CYC>(b, values, ctrl, tile_bytes, line_base); \
         break;
     switch (kind) {
         INTP_LINE_CASE(0, false)
@@ -428,13 +427,12 @@ __global__ __launch_bounds__(NT, NT == kTileThreads && FORM != BatchSolveForm::k
     int32_t first_pass) {
     extern __shared__ __align__(16) unsigned char tile_bytes[];
     constexpr int kBases = FORM == BatchSolveForm::kLanes ? 1 : kMaxTileLines;
-    __shared__ int64_t dst_base[kBases];
-    __shared__ int64_t src_base[kBases];
+    __shared__ int64_t line_base[kBases];
     for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
         const BatchSolveItem w = items[it];
 #define INTP_SOLVE_CASE(BW, CYC)                                                                                  \
     case 2 * BW + CYC:                                                                                            \
-        batch_solve_item<BW, CYC, NT, FORM>(specs, w, values, ctrl, first_pass, tile_bytes, dst_base, src_base);  \
+        batch_solve_item<BW, CYC, NT, FORM>(specs, w, values, ctrl, first_pass, tile_bytes, line_base);            \
         break;
         // periodic band widths are floor(k/2) <= 3, clamped ones k - 1 <= 6
         switch (w.kind) {

@@ -37,11 +37,10 @@ template <int BW, bool CYC, typename T, typename C, bool SEG>
 __global__ __launch_bounds__(SEG ? kMaxTileThreads : kTileThreads)
     __attribute__((amdgpu_waves_per_eu((tile_waves<BW, CYC, C, SEG>()), !SEG && BW >= 4 && sizeof(C) == 8 ? 3 : 8))) void solve_tile_kernel(SolveParams sp) {
     extern __shared__ __align__(16) unsigned char tile_bytes[];
-    __shared__ int64_t dst_base[kMaxTileLines];
-    __shared__ int64_t src_base[kMaxTileLines];
+    __shared__ int64_t line_base[kMaxTileLines];
     const int nt = static_cast<int>(blockDim.x);  // a power of two
     solve_tile<BW, CYC, T, C, batch_rows<BW, CYC>(), SEG>(
-        sp, static_cast<int64_t>(blockIdx.x) * sp.lines_per_block, tile_bytes, dst_base, src_base,
+        sp, static_cast<int64_t>(blockIdx.x) * sp.lines_per_block, tile_bytes, line_base,
         static_cast<int>(threadIdx.x + 64 * blockIdx.x) & (nt - 1), nt);
 }
 
@@ -92,7 +91,7 @@ hipError_t launch_bw(bool cyclic, const SolveParams& p, int threads, hipStream_t
         if (lpb > kMaxTileLines || threads > (p.segs > 0 ? kMaxTileThreads : kTileThreads) || threads % lpb != 0 || threads % 64 != 0 ||
             (threads & (threads - 1)) != 0 ||
             (lpb & (lpb - 1)) != 0 || p.segs < 0 || p.segs > threads / lpb || (p.segs > 1 && p.segs < BW) || (p.segs > 0 && threads / lpb < BW) ||
-            p.n >= (int64_t{1} << 24))
+            p.n >= (int64_t{1} << 24) || (p.src && p.inner != 1))
             return hipErrorInvalidValue;
     } else if (p.src || p.accum) {
         return hipErrorInvalidValue;  // the HBM kernel solves in place only

@@ -824,7 +824,7 @@ __device__ __forceinline__ bool solve_segments(const SolveParams& sp, C* tile, i
 template <int BW, bool CYC, typename T, typename C, int B = batch_rows<BW, CYC>(), bool SEG = true,
           bool FIXED = true, bool ONE = false>
 __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first, unsigned char* tile_bytes,
-                                           int64_t* dst_base, int64_t* src_base, int tid, int NT) {
+                                           int64_t* line_base, int tid, int NT) {
     const int lpb = sp.lines_per_block;
     const int64_t n = sp.n, inner = sp.inner;
     const int step = static_cast<int>(tile_step(lpb, inner));
@@ -834,8 +834,11 @@ __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first,
     if (tid < nl) {
         const int64_t line = first + tid;
         const int64_t o = line / inner, ii = line - o * inner;
-        dst_base[tid] = o * n * inner + ii;
-        if (sp.src) {
+        // the line's place in the values (first pass, contiguous lines), or in
+        // the table
+        if (!sp.src) {
+            line_base[tid] = o * n * inner + ii;
+        } else {
             // inner == 1: o runs over the outer dims in C order
             // constant indices (a runtime-indexed loop would force a
             // SolveParams built in registers out to scratch memory)
@@ -851,7 +854,7 @@ __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first,
                 off += w * mul;
                 mul *= nd;
             }
-            src_base[tid] = off;
+            line_base[tid] = off;
         }
     }
     __syncthreads();
@@ -885,7 +888,7 @@ __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first,
                     const uint32_t l = fast_div(e, sp.div_n), jj = e - l * un;
                     int64_t js = static_cast<int64_t>(jj) - sp.shift_last;
                     if (js < 0) js += n;
-                    v[u] = static_cast<C>(__builtin_nontemporal_load(&sp.src[src_base[l] + js]));
+                    v[u] = static_cast<C>(__builtin_nontemporal_load(&sp.src[line_base[l] + js]));
                     at[u] = jj * static_cast<uint32_t>(step) + l;
                 }
 #pragma unroll
@@ -909,7 +912,7 @@ __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first,
             }
         } else if (vec) {
             if (static_cast<int>(my_v) < nl) {
-                const T* __restrict__ line = X + dst_base[my_v];
+                const T* __restrict__ line = X + line_base[my_v];
                 const uint32_t rows = NT >> vshift;
                 for (uint32_t j0 = static_cast<uint32_t>(tid) >> vshift; j0 < un; j0 += rows * kCopyBatch) {
                     VecT v[kCopyBatch];
@@ -927,7 +930,7 @@ __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first,
                 }
             }
         } else if (static_cast<int>(my_l) < nl) {
-            const T* __restrict__ line = X + dst_base[my_l];
+            const T* __restrict__ line = X + line_base[my_l];
             for (uint32_t e0 = tid; e0 < count; e0 += NT * kCopyBatch) {
                 C v[kCopyBatch];
 #pragma unroll
@@ -998,7 +1001,7 @@ __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first,
         }
     } else if (vec) {
         if (static_cast<int>(my_v) < nl) {
-            T* __restrict__ line = Y + dst_base[my_v];
+            T* __restrict__ line = Y + line_base[my_v];
             const uint32_t rows = NT >> vshift;
 #pragma unroll 4
             for (uint32_t j = static_cast<uint32_t>(tid) >> vshift; j < un; j += rows) {
@@ -1011,7 +1014,7 @@ __device__ __forceinline__ void solve_tile(const SolveParams& sp, int64_t first,
             }
         }
     } else if (static_cast<int>(my_l) < nl) {
-        T* __restrict__ line = Y + dst_base[my_l];
+        T* __restrict__ line = Y + line_base[my_l];
         for (uint32_t e0 = tid; e0 < count; e0 += NT * kBatch) {
             C v[kBatch];
 #pragma unroll

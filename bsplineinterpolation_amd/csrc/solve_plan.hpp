@@ -18,12 +18,12 @@ constexpr int kSegRows = 8;  // segments and warm-ups are multiples of this
 // LDS of a workgroup on gfx950, and of one of two workgroups that share a CU.
 constexpr int64_t kLdsBytes = 160 * 1024;
 constexpr int64_t kTileLdsBudget = 80 * 1024;
-// Static LDS of the kernels that call solve_tile, at most: two offsets a
+// Static LDS of the kernels that call solve_tile, at most: one offset a
 // line and two flags, a pair for each variant that the batch's merged kernel
 // holds; rounded up to the 16 bytes at which the dynamic part (the tile)
 // starts.
-constexpr int64_t kTileStaticLds = 2 * kMaxTileLines * 8 + 16;
-constexpr int64_t kBatchStaticLds = 2 * kMaxTileLines * 8 + 128;
+constexpr int64_t kTileStaticLds = kMaxTileLines * 8 + 16;
+constexpr int64_t kBatchStaticLds = kMaxTileLines * 8 + 128;
 
 // Row stride of a tile in elements: odd on the contiguous axis, so that
 // the coalesced runs along a line spread over the LDS banks, and for
@@ -56,6 +56,11 @@ inline int64_t tile_lds(const SolveParams& p, int bw, int compute_bytes) {
     return (tile_elements(p.n, p.lines_per_block, p.inner, p.segs) + edge_elements(p.n, bw, p)) * compute_bytes;
 }
 
+// Workgroups whose LDS a CU holds: it is given out in 1280-byte granules (a
+// contiguous cubic axis in whole lines, 32 a tile: at 200 rows with 53,328
+// bytes, three a CU, 66 us; with 53,840, two, 89).
+inline int64_t resident_by_lds(int64_t lds) { return kLdsBytes / ((lds + 1279) / 1280 * 1280); }
+
 // Estimated time of one axis, us, by the ways to solve its lines: plain
 // tiles, tiles of one segment a line, tiles cut into segments, the same where comparisons fail in every
 // tile (which are then solved again in one piece), and in place in HBM with
@@ -80,7 +85,7 @@ inline LineTimes line_times(const SolveParams& p, int bw, bool cyclic, int compu
         SolveParams q = p;
         q.segs = segs;
         const int64_t lds = tile_lds(q, bw, compute_bytes) + kTileStaticLds;
-        const int64_t resident = std::max<int64_t>(1, std::min<int64_t>(by_registers * 256 / threads, kLdsBytes / lds));
+        const int64_t resident = std::max<int64_t>(1, std::min<int64_t>(by_registers * 256 / threads, resident_by_lds(lds)));
         const int64_t tiles = (p.nlines + p.lines_per_block - 1) / p.lines_per_block;
         // a last round that is not full overlaps the one before in part
         const int64_t whole = (tiles + 256 * resident - 1) / (256 * resident);
@@ -145,7 +150,7 @@ inline TilePlan plan_tile(const SolveParams& p, int bw, bool cyclic, int compute
         if (lds > std::min(kLdsBytes, max_lds)) continue;
         if (inner >= 64 && lpb < 4) continue;  // in HBM instead
         const int64_t tiles = (p.nlines + lpb - 1) / lpb;
-        const int64_t resident = std::min<int64_t>(std::min<int64_t>(3, kLdsBytes / lds), (tiles + 255) / 256);
+        const int64_t resident = std::min<int64_t>(std::min<int64_t>(3, resident_by_lds(lds)), (tiles + 255) / 256);
         const int64_t rounds = (tiles + 256 * resident - 1) / (256 * resident);
         const int64_t width = inner == 1 ? lpb * compute_bytes : std::max<int64_t>(lpb * compute_bytes, 64);
         const int64_t segs = can_cut ? segments(lpb) : 1;
@@ -167,8 +172,12 @@ inline TilePlan plan_tile(const SolveParams& p, int bw, bool cyclic, int compute
     // fade (a Gaussian, zeros after a box) fail in many tiles, which are then
     // solved twice.  Lines are cut where that gains though every second tile
     // fails (256^3 cubic, the contiguous axis, us: plain 146, cut 92 on noise
-    // and 179 on a Gaussian; order 5: 167, 150, 244, so plain).
-    const double expected = 0.5 * (t.cut + t.failed);
+    // and 179 on a Gaussian; order 5: 167, 150, 244, so plain).  In FP32 every
+    // fourth: half of those solves are corrections, whose right-hand sides are
+    // rounding errors, and noise does not fail (order 5, 256^3 refined, the
+    // build, us: plain 575 on any data, cut 535 on noise, 574 on a Gaussian).
+    const double fails = compute_bytes == 4 ? 0.25 : 0.5;
+    const double expected = t.cut + fails * (t.failed - t.cut);
     const bool cut_pays = plan.segs > 1 && expected < t.plain;
     double tiled = cut_pays ? expected : t.plain;
     if (!cut_pays) {

@@ -98,6 +98,7 @@ void choices() {
         int order, periodic;
         int64_t n, nlines, inner;
         int want;
+        bool f32 = false;
     } cases[] = {
         {3, 0, 8192, 1, 1, kCut},         {6, 1, 8192, 1, 1, kCut},         {3, 0, 2000, 2000, 1, kCut},
         {3, 0, 2000, 2000, 2000, kCut},   {5, 0, 1021, 769, 769, kCut},     {3, 0, 1000, 4096, 64, kCut},
@@ -106,16 +107,18 @@ void choices() {
         {6, 1, 180, 32400, 180, kInPlace}, {5, 0, 64, 65536, 65536, kInPlace}, {5, 0, 100, 50000, 100, kInPlace},
         {3, 0, 20, 90000, 300, kInPlace},  {3, 0, 100, 10000, 100, kWhole},  {5, 0, 80, 6400, 80, kWhole},
         {3, 0, 64, 64, 64, kWhole},        {3, 0, 64, 4096, 64, kWhole},
+        {3, 0, 200, 40000, 1, kWhole},      {3, 0, 204, 41616, 1, kCut},
+        {5, 0, 256, 65536, 1, kCut, true}, {5, 0, 256, 65536, 256, kInPlace, true},
     };
     for (const auto& c : cases) {
         DimSetup s;
         if (!setup_dimension(c.order, c.periodic != 0, c.n, 0.0, 1.0, nullptr, s, true).empty()) std::abort();
         SolveParams p{};
-        set_segment_params(s.lu.seg64, &p);
+        set_segment_params(c.f32 ? s.lu.seg32 : s.lu.seg64, &p);
         p.n = c.n;
         p.nlines = c.nlines;
         p.inner = c.inner;
-        const TilePlan plan = plan_tile(p, s.lu.p, s.lu.cyclic, 8, kLdsBytes);
+        const TilePlan plan = plan_tile(p, s.lu.p, s.lu.cyclic, c.f32 ? 4 : 8, kLdsBytes);
         const int got = plan.in_place ? kInPlace : plan.lines == 0 ? -1 : plan.segs > 1 ? kCut : kWhole;
         check(got == c.want, "choice", c.order, c.periodic, 8, c.n, c.inner, got);
     }
